@@ -1,0 +1,75 @@
+"""Whole paths in one launch (k_paths) against the wavefront.
+
+A job with counting on always runs in the wavefront; without, small batches
+run in k_paths and large ones are finished by it.  Each path's arithmetic is
+the same, so images and ray counts must be equal bit for bit.
+"""
+import numpy as np
+import pytest
+
+import yune_amd as Y
+
+pytestmark = pytest.mark.gpu
+
+
+def render(ctx, sid, cam, w, h, frames, params, counting):
+    j = ctx.job(sid, cam, w, h, params, base_seed=9)
+    j.set_counting(counting)
+    j.render(frames)
+    img, st = j.read(), j.stats()
+    j.release()
+    return img.view(np.int32), (st.rays_ext, st.rays_shadow, st.samples)
+
+
+PARAMS = {"mis": dict(mis=1, max_bounces=8, rr_threshold=2), "shipped": dict(), "direct": dict(gi=0),
+          "fix": dict(mis=1, fix_mis=1, oren_nayar=1)}
+
+
+@pytest.mark.parametrize("kind", sorted(PARAMS))
+@pytest.mark.parametrize("scene", ["cornell", "room", "brute"])
+def test_paths_equal_wavefront(scene, kind):
+    """Sizes around a wave, a block and one path per wave, and more paths
+    than lanes (taken from the queue as others end)."""
+    s = Y.gen_icosphere_room(7, 6, 3) if scene == "room" else Y.gen_cornell()
+    params = Y.params_reference(0, **PARAMS[kind])
+    with Y.Context(max_paths=1 << 20) as ctx:
+        sid = ctx.scene(s, brute=scene == "brute")
+        for w, h, f in ((1, 1, 1), (9, 7, 1), (64, 1, 1), (13, 5, 3), (64, 65, 1), (97, 61, 2), (640, 500, 3)):
+            a = render(ctx, sid, s.cam, w, h, f, params, False)
+            b = render(ctx, sid, s.cam, w, h, f, params, True)
+            assert np.array_equal(a[0], b[0]), (w, h, f)
+            assert a[1] == b[1], (w, h, f)
+
+
+def test_wavefront_finished_by_paths():
+    """More paths than k_paths takes from the start: the wavefront hands its
+    last rays over, and the image is that of the frames rendered one by one."""
+    s = Y.gen_cornell()
+    params = Y.params_reference(0, mis=1)
+    with Y.Context() as ctx:
+        sid = ctx.scene(s)
+        a = render(ctx, sid, s.cam, 1000, 1000, 9, params, False)
+        j = ctx.job(sid, s.cam, 1000, 1000, params, base_seed=9)
+        for _ in range(9):
+            j.render(1)
+        b = j.read().view(np.int32), (j.stats().rays_ext, j.stats().rays_shadow, j.stats().samples)
+        c = render(ctx, sid, s.cam, 1000, 1000, 9, params, True)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[0], c[0])
+    assert a[1] == b[1] == c[1]
+
+
+def test_paths_over_several_scenes():
+    """A scheduler round with jobs of several scenes against each job alone."""
+    scenes = [Y.gen_cornell(), Y.gen_icosphere_room(3, 4, 3), Y.gen_icosphere_room(5, 2, 2)]
+    params = Y.params_reference(0, mis=1, max_bounces=8, rr_threshold=2)
+    with Y.Context(max_paths=1 << 20, serve_mode=1) as ctx:
+        sids = [ctx.scene(s) for s in scenes]
+        jobs = [ctx.submit(sid, s.cam, 65 + 7 * k, 33, params, 3, 4 + k)
+                for k, (sid, s) in enumerate(zip(sids, scenes))]
+        while ctx.serve(4):
+            pass
+        for k, (j, sid, s) in enumerate(zip(jobs, sids, scenes)):
+            alone = ctx.job(sid, s.cam, 65 + 7 * k, 33, params, base_seed=4 + k)
+            alone.set_counting(True)
+            alone.render(3)
+            assert np.array_equal(j.read().view(np.int32), alone.read().view(np.int32)), k

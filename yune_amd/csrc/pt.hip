@@ -28,397 +28,10 @@
 //    (udpt.cl:599), so it is an any-hit query up to the quad, skipped when
 //    the quad is missed.
 #include "yn_internal_dev.h"
+#include "yn_path.h"
 #include "yn_shade.h"
 
 namespace yune {
-
-namespace {
-
-enum : int {
-    ST_DONE = 0,
-    ST_PRIMARY = 1,
-    ST_BOUNCE = 2,
-    ST_NEE_SH = 3,
-    ST_NEE_MIS = 4,
-    ST_MASK = 0xff,
-    F_DIRECT = 1 << 8,      // NEE result is the first vertex's direct light
-    F_LCAND = 1 << 9,       // pending extension ray ends on the quad
-    F_NGLOSSY = 1 << 10,    // NEE lobe: glossy
-    F_BGLOSSY = 1 << 11,    // bounce lobe: glossy
-    F_CAPSH = 1 << 12,      // first shadow ray already captured
-    SCENE_SHIFT = 16,       // bits 16..23: the path's scene (its job's), read without the job
-};
-
-constexpr float kPinkR = 0.988f, kPinkG = 0.0588f, kPinkB = 0.7529f;   // udpt.cl:110
-
-struct Out {
-    int kind = 0;           // 0 none, 1 extension, 2 shadow
-    bool done = false;      // the path ended and wrote its sample
-    int job = -1;           // the path's job-table entry
-    float4 o_t;
-    float4 d_p;
-};
-
-// A path's state between two shade steps (the fields of PathRecs).
-struct Rec {
-    int4 m0, m1;
-    f4 hp, hn, rd, tp, direct, indirect, nd, bnc, wi, ls, mis;
-};
-
-__device__ __forceinline__ void write_sample(const DevJob& J, int slot, int pix, f4 c)
-{
-    if (any_nan(c)) c = mk(kPinkR, kPinkG, kPinkB, 1.0f);     // udpt.cl:193-194
-    J.samples[(size_t)slot * (size_t)(J.W * J.H) + (size_t)pix] = st4(c);
-}
-
-// The ray's w carries the path's job-table entry: the trace kernels look
-// the scene up through it.
-__device__ __forceinline__ Out make_ray(int kind, f4 o, f4 d, float tmax, int job)
-{
-    Out r;
-    r.kind = kind;
-    r.o_t = make_float4(o.x, o.y, o.z, tmax);
-    r.d_p = make_float4(d.x, d.y, d.z, __int_as_float(job));
-    return r;
-}
-
-// The record a step reads.  The fields most states use are loaded without
-// waiting for the state (a new path's record holds only m0, m1 and the
-// camera ray's direction; the rest is not used then); only the MIS ray's
-// fields, used by one state, wait for it.  The shade pass is bound by the
-// latency of such chains of loads.  Which queue the result came from is
-// known before the state: a bounce result (extension queue) reads the
-// pending bounce and never the NEE light direction, a shadow result the
-// light direction and never the pending bounce (each is rewritten before
-// the step stores it), so each loads only its own.
-__device__ __forceinline__ void load_rec(const PathRecs& I, uint32_t ri, Rec& R, bool ext, bool primary)
-{
-    using F = PathRecs;
-    R.m0 = *reinterpret_cast<const int4*>(I.f(F::M0, ri));
-    R.m1 = *reinterpret_cast<const int4*>(I.f(F::M1, ri));
-    R.rd = ld(*I.f(F::RD, ri));
-    if (primary) {          // a camera ray's record: the rest is set by its step
-        R.hp = R.hn = R.tp = R.direct = R.indirect = R.nd = R.bnc = R.wi = mk(0, 0, 0, 0);
-        return;
-    }
-    R.hp = ld(*I.f(F::HP, ri));
-    R.hn = ld(*I.f(F::HN, ri));
-    R.tp = ld(*I.f(F::TP, ri));
-    R.direct = ld(*I.f(F::DIRECT, ri));
-    R.indirect = ld(*I.f(F::INDIRECT, ri));
-    R.nd = R.bnc = R.wi = mk(0, 0, 0, 0);
-    if (ext) {
-        R.nd = ld(*I.f(F::ND, ri));
-        R.bnc = ld(*I.f(F::BNC, ri));
-    } else {
-        R.wi = ld(*I.f(F::WI, ri));
-    }
-    if ((R.m0.y & ST_MASK) == ST_NEE_MIS) {
-        R.ls = ld(*I.f(F::LS, ri));
-        R.mis = ld(*I.f(F::MIS, ri));
-    }
-}
-
-// The record beside a ray just made: what the next step's state uses.
-__device__ __forceinline__ void store_rec(const PathRecs& O, uint32_t ri, const Rec& R)
-{
-    using F = PathRecs;
-    *reinterpret_cast<int4*>(O.f(F::M0, ri)) = R.m0;
-    *reinterpret_cast<int4*>(O.f(F::M1, ri)) = R.m1;
-    *O.f(F::HP, ri) = st4(R.hp);
-    *O.f(F::HN, ri) = st4(R.hn);
-    *O.f(F::RD, ri) = st4(R.rd);
-    *O.f(F::TP, ri) = st4(R.tp);
-    *O.f(F::DIRECT, ri) = st4(R.direct);
-    *O.f(F::INDIRECT, ri) = st4(R.indirect);
-    const int code = R.m0.y & ST_MASK;
-    if (code == ST_BOUNCE) {
-        *O.f(F::ND, ri) = st4(R.nd);
-        *O.f(F::BNC, ri) = st4(R.bnc);
-    } else {
-        *O.f(F::WI, ri) = st4(R.wi);
-        if (code == ST_NEE_MIS) {
-            *O.f(F::LS, ri) = st4(R.ls);
-            *O.f(F::MIS, ri) = st4(R.mis);
-        }
-    }
-}
-
-// One shade step of the path whose ray sits at entry qi of the extension
-// queue (ext) or of the shadow queue; R holds its record, updated in place
-// for the ray the step makes.  The ray whose result arrived is rebuilt from
-// the path state, bit for bit as it was made: a camera ray starts at the
-// camera's eye (createRay, udpt.cl:236) along the stored direction rd; a
-// bounce ray at hp + nd * EPSILON along the pending bounce direction nd
-// (udpt.cl:766, 906, 945).
-template <bool CAP, int LM>
-__device__ Out advance(const ShadeArgs& a, const DevCapture& cap, bool ext, uint32_t qi, Rec& R, const LdsScene& lds)
-{
-    load_rec(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), R, ext, ext && a.ext_primary);
-    const int4 m0 = R.m0, m1 = R.m1;
-    const int jid = m1.y;
-    const DevJob& J = a.jobs[jid];
-    const yn_render_params& RP = J.p;
-    const int sid = (m0.y >> SCENE_SHIFT) & 0xff;
-    const DevScene& S = a.scenes[sid];                                 // loaded beside J, not after it
-    // LM: materials and light in LDS, the launch's one scene's (1) or every scene's (2)
-    auto mat_of = [&](int id) {
-        return LM == 1 ? load_mat(lds.mats, id) : LM == 2 ? load_mat(lds.mats, S.mat_base + id) : load_mat(S.mats, id);
-    };
-    auto& L = light_of<LM>(S.light, lds, sid);
-    const bool on = RP.oren_nayar != 0;
-    const bool fix = RP.fix_mis != 0;
-
-    int st = m0.y;
-    int code = st & ST_MASK;
-    uint32_t seed = (uint32_t)m0.x;
-    const int pix = m1.x;
-    const int slot = m1.z;
-    const bool cap_on = CAP && cap.prim_tri != nullptr && slot == 0;
-
-    int vmat = m0.w;                    // material of the path's current vertex
-    f4& hp = R.hp;
-    f4& hn = R.hn;
-    f4& rd = R.rd;
-    f4& tp = R.tp;
-    f4& direct = R.direct;
-    f4& indirect = R.indirect;
-    float nee_prob = __int_as_float(m1.w);
-    bool v_dirty = false;
-    int bounce = m0.z;
-
-    // NEE scratch
-    f4 wi = mk(0, 0, 0, 0);
-    float lpdf = 0.0f, nprob = 0.0f;
-    f4 ls = mk(0, 0, 0, 0);
-    f4 em = mk(0, 0, 0, 0);
-    f4 nee_res = mk(0, 0, 0, 0);
-    int occ = 0;
-
-    enum Step { S_NEE_START, S_NEE_SHADOW, S_NEE_MIS, S_NEE_DONE, S_BOUNCE_SAMPLE, S_FINISH, S_FINISH_CONST };
-    Step step;
-    f4 const_color = mk(0, 0, 0, 0);
-
-    if (code == ST_PRIMARY) {
-        float4 h = a.hit[qi];
-        int htri = __float_as_int(h.y);
-        if (cap_on) {
-            cap.prim_tri[pix] = htri;
-            cap.prim_light[pix] = (htri < 0 && (st & F_LCAND)) ? 0 : -1;
-            cap.prim_t[pix] = h.x;
-        }
-        f4 d = rd;
-        if (htri < 0) {
-            if (st & F_LCAND) {     // udpt.cl:440-446
-                const_color = dot(d, ld(L.normal)) < 0 ? mk(1, 1, 1, 1) : mk(0.1f, .1f, .1f, 1);
-            } else {
-                const_color = mk(RP.background[0], RP.background[1], RP.background[2], RP.background[3]);
-            }
-            step = S_FINISH_CONST;
-        } else {
-            f4 o = mk(J.cam.r1.w, J.cam.r2.w, J.cam.r3.w, 1.0f);
-            vmat = tri_material(S.tri_shade, htri);
-            hp = o + d * h.x;
-            hn = shade_normal(S.tri_shade, htri, h.z, h.w);
-            rd = d;
-            tp = mk(1, 1, 1, 1);
-            direct = mk(0, 0, 0, 0);
-            indirect = mk(0, 0, 0, 0);
-            v_dirty = true;
-            bounce = 0;
-            Mat m = mat_of(vmat);
-            if (!m.spec) { st |= F_DIRECT; step = S_NEE_START; }
-            else { step = S_BOUNCE_SAMPLE; }
-        }
-    } else {
-        if (code == ST_NEE_SH) {
-            occ = a.occ[qi];
-            step = S_NEE_SHADOW;
-        } else if (code == ST_NEE_MIS) {
-            occ = a.occ[qi];
-            step = S_NEE_MIS;
-        } else {   // ST_BOUNCE: extension result (udpt.cl:488-529)
-            float4 h = a.hit[qi];
-            int htri = __float_as_int(h.y);
-            Mat m = mat_of(vmat);
-            f4 nd = R.nd;
-            float4 bnc = st4(R.bnc);
-            if (htri < 0) {
-                if ((st & F_LCAND) && m.spec) indirect = indirect + tp * ld(L.ke);
-                step = S_FINISH;
-            } else {
-                f4 o = hp + nd * kEps;
-                f4 nhp = o + nd * h.x;
-                f4 nhn = shade_normal(S.tri_shade, htri, h.z, h.w);
-                const int nmat = tri_material(S.tri_shade, htri);
-                Mat nm = mat_of(nmat);
-                indirect = indirect + tp * nm.ke;
-                if (m.spec) tp = tp * bnc.z;
-                else
-                    tp = ((tp * eval_brdf(m, nd, -rd, hp, hn, (st & F_BGLOSSY) != 0, bnc.y, on, false)) *
-                          fmaxf(dot(nd, hn), 0.0f)) / bnc.x;
-                step = S_NEE_START;
-                if (bounce > RP.rr_threshold) {    // udpt.cl:514-523
-                    float pr = fminf(luminance(tp), 0.95f);
-                    float r = next_rand(seed);
-                    if (r >= pr) step = S_FINISH;
-                    else tp = tp * (1 / pr);
-                }
-                if (step != S_FINISH) {
-                    v_dirty = true;
-                    vmat = nmat;
-                    hp = nhp;
-                    hn = nhn;
-                    rd = nd;
-                    bounce++;
-                    st &= ~F_DIRECT;
-                    if (nm.spec) step = S_BOUNCE_SAMPLE;
-                }
-            }
-        }
-    }
-
-    Out out;
-    bool ended = false;
-    // The steps only ever move forward (NEE start, shadow, MIS, done, bounce
-    // sample, finish), so they run as one forward sequence: a step that
-    // hands over sets `step` to a later one and leaves its block, a step that
-    // makes a ray jumps past the rest.  Without a loop back-edge, values of
-    // one step are not kept live through the others.
-    if (step == S_NEE_START) do {   // evaluateDirectLighting (udpt.cl:535-555)
-        Mat m = mat_of(vmat);
-        em = m.ke;
-        f4 wraw;
-        if (!sample_lights(L, hp, hn, seed, lpdf, wraw) || lpdf <= 0.0f) { nee_res = em; step = S_NEE_DONE; break; }
-        float len = length(wraw);
-        len -= kEps * 1.5f;
-        wi = normalize(wraw);
-        bool glossy = false;
-        nprob = 0.0f;
-        if (fix) {
-            glossy = sample_glossy_pdf(m, seed, nprob, false);
-            if (nprob == 0.0f) { nee_res = em; step = S_NEE_DONE; break; }
-            st = glossy ? (st | F_NGLOSSY) : (st & ~F_NGLOSSY);
-        }
-        f4 so = hp + wi * kEps;
-        float tq;
-        if (cap_on && (st & F_DIRECT) && !(st & F_CAPSH)) {
-            cap.shadow_o[pix] = make_float4(so.x, so.y, so.z, len);
-            cap.shadow_d[pix] = make_float4(wi.x, wi.y, wi.z, 1.0f);
-        }
-        if (quad_hit(L, so, wi, len, tq)) { occ = 1; step = S_NEE_SHADOW; break; }
-        R.wi = mk(wi.x, wi.y, wi.z, lpdf);
-        nee_prob = nprob;
-        st = (st & ~ST_MASK) | ST_NEE_SH;
-        out = make_ray(2, so, wi, len, jid);
-        goto steps_done;
-    } while (0);
-    if (step == S_NEE_SHADOW) do {  // udpt.cl:557-565 and the MIS light weight
-        if (code == ST_NEE_SH) {
-            wi = mk(R.wi.x, R.wi.y, R.wi.z, 0.0f);
-            lpdf = R.wi.w;
-            nprob = nee_prob;
-            code = ST_DONE;     // consumed
-        }
-        if (cap_on && (st & F_DIRECT) && !(st & F_CAPSH)) { cap.shadow_occ[pix] = occ; st |= F_CAPSH; }
-        Mat m = mat_of(vmat);
-        em = m.ke;
-        f4 w_o = -rd;
-        bool glossy = fix ? ((st & F_NGLOSSY) != 0) : false;
-        ls = mk(0, 0, 0, 0);
-        if (!occ) {
-            if (!fix) {
-                glossy = sample_glossy_pdf(m, seed, nprob, false);
-                if (nprob == 0.0f) { nee_res = em; step = S_NEE_DONE; break; }
-            }
-            ls = (eval_brdf(m, wi, w_o, hp, hn, glossy, nprob, on, false) * ld(L.ke)) * fmaxf(dot(wi, hn), 0.0f);
-            ls = ls * (1 / lpdf);
-        }
-        if (!RP.mis) { nee_res = ls + em; step = S_NEE_DONE; break; }
-        float bpdf = glossy ? phong_pdf(m, wi, w_o, hn) : cos_pdf(wi, hn);
-        float mw = power_heuristic(lpdf, lpdf, bpdf);
-        ls = ls * mw;
-        f4 bd = glossy ? phong_sample(m, bpdf, w_o, hp, hn, seed, false) : cosine_sample(bpdf, hp, hn, seed);
-        if (bpdf <= 0.0f) { nee_res = ls + em; step = S_NEE_DONE; break; }
-        f4 bo = hp + bd * kEps;
-        float tq;
-        if (!quad_hit(L, bo, bd, INFINITY, tq)) { nee_res = ls + em; step = S_NEE_DONE; break; }
-        st = glossy ? (st | F_NGLOSSY) : (st & ~F_NGLOSSY);
-        R.ls = ls;
-        R.mis = mk(bd.x, bd.y, bd.z, bpdf);
-        R.wi = mk(wi.x, wi.y, wi.z, lpdf);
-        nee_prob = nprob;
-        st = (st & ~ST_MASK) | ST_NEE_MIS;
-        out = make_ray(2, bo, bd, tq, jid);
-        goto steps_done;
-    } while (0);
-    if (step == S_NEE_MIS) do {     // udpt.cl:599-607
-        Mat m = mat_of(vmat);
-        em = m.ke;
-        ls = R.ls;
-        if (occ) { nee_res = ls + em; step = S_NEE_DONE; break; }
-        f4 bd = mk(R.mis.x, R.mis.y, R.mis.z, 0.0f);
-        float bpdf = R.mis.w;
-        lpdf = R.wi.w;
-        nprob = nee_prob;
-        bool glossy = (st & F_NGLOSSY) != 0;
-        float mw = power_heuristic(bpdf, lpdf, bpdf);
-        f4 bs = (eval_brdf(m, bd, -rd, hp, hn, glossy, nprob, on, false) * ld(L.ke)) * fmaxf(dot(bd, hn), 0.0f);
-        bs = bs * (mw / bpdf);
-        nee_res = (ls + bs) + em;
-        step = S_NEE_DONE;
-        break;
-    } while (0);
-    if (step == S_NEE_DONE) do {
-        if (st & F_DIRECT) direct = nee_res;
-        else indirect = indirect + tp * nee_res;
-        step = S_BOUNCE_SAMPLE;
-        break;
-    } while (0);
-    if (step == S_BOUNCE_SAMPLE) do {   // udpt.cl:458-487
-        if (!RP.gi || bounce >= RP.max_bounces) { step = S_FINISH; break; }
-        Mat m = mat_of(vmat);
-        float pdf = 1.0f, bprob = 0.0f, ior = 1.0f;
-        bool glossy = false;
-        f4 nd;
-        if (m.spec) nd = fresnel_sample(m, hn, -rd, ior, seed);
-        else {
-            glossy = sample_glossy_pdf(m, seed, bprob, false);
-            if (bprob == 0.0f) { step = S_FINISH; break; }
-            nd = glossy ? phong_sample(m, pdf, -rd, hp, hn, seed, false) : cosine_sample(pdf, hp, hn, seed);
-        }
-        if (pdf <= 0.0f) { step = S_FINISH; break; }
-        f4 no = hp + nd * kEps;
-        float tq, tmax = INFINITY;
-        st &= ~F_LCAND;
-        if (quad_hit(L, no, nd, INFINITY, tq)) { tmax = tq; st |= F_LCAND; }
-        st = glossy ? (st | F_BGLOSSY) : (st & ~F_BGLOSSY);
-        R.nd = nd;
-        R.bnc = mk(pdf, bprob, ior, 0.0f);
-        st = (st & ~ST_MASK) | ST_BOUNCE;
-        out = make_ray(1, no, nd, tmax, jid);
-        goto steps_done;
-    } while (0);
-    if (step == S_FINISH) do {
-        write_sample(J, slot, pix, direct + indirect);
-        st = ST_DONE;
-        ended = true;
-        goto steps_done;
-    } while (0);
-    if (step == S_FINISH_CONST) { write_sample(J, slot, pix, const_color); st = ST_DONE; ended = true; }
-steps_done:
-    if (out.kind == 0 && !ended) {   // unreachable by construction; never leave a path hanging
-        write_sample(J, slot, pix, mk(NAN, NAN, NAN, NAN));
-        st = ST_DONE;
-    }
-    out.done = out.kind == 0;
-    out.job = jid;
-    R.m0 = make_int4((int)seed, st, v_dirty ? bounce : m0.z, v_dirty ? vmat : m0.w);
-    R.m1 = make_int4(m1.x, m1.y, m1.z, __float_as_int(nee_prob));
-    return out;
-}
-
-}  // namespace
 
 // WAVES: the occupancy the register allocation is held to, per SIMD.
 // Blocks of shade_block_pt(WAVES) threads walk the queues together, one atomic per
@@ -473,7 +86,9 @@ __global__ __launch_bounds__(shade_block_pt(WAVES), WAVES) void k_shade_pt(Shade
         Rec R;
         if (i < total) {
             const bool ext = i < n_ext;
-            o = advance<CAP, LM>(a, cap, ext, ext ? i : i - n_ext, R, lds);
+            const uint32_t qi = ext ? i : i - n_ext;
+            load_rec(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), R, ext, ext && a.ext_primary);
+            o = advance<CAP, LM>(a, cap, QueueResult{a.hit, a.occ, qi}, R, lds);
         }
         const uint32_t n[2] = {o.kind == 1 ? 1u : 0u, o.kind == 2 ? 1u : 0u};
         uint32_t at[2];

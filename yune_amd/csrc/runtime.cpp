@@ -591,19 +591,80 @@ int ensure_group_graph(yn_ctx* c, const LoopCfg& L, const IterArgs (&iters)[2], 
     return 0;
 }
 
-// Runs one batch of primary-ray regions to completion; samples land in
-// samples[slot][pixel] of each region's job (the sample buffer is shared:
-// job slots are laid out by the caller so regions do not overlap).
-int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, const DevCapture& cap)
+// Batches of at most kPathsDirect paths run in k_paths from their camera rays
+// on (enqueue_paths), larger ones in the wavefront, which k_paths finishes
+// once at most kPathsTail rays are queued.  Time of a batch, wavefront against
+// k_paths (depth 8, NEE + MIS):
+//                  262,144 paths     4.2M paths        16.8M paths
+//   Cornell box    2.06 / 0.51 ms    6.00 / 3.79 ms    14.5 / 14.3 ms
+//   245k triangles 5.24 / 1.27 ms    9.44 / 6.80 ms    22.3 / 24.8 ms
+//   1M triangles   6.02 / 1.38 ms    10.8 / 7.5 ms     24.7 / 27.3 ms
+// Without a bounce limit k_paths leads at 16.8M as well (64 / 39 ms at 1M
+// triangles): the wavefront then runs many iterations over few rays, which
+// the tail rule takes from it (256 frames of the Cornell box, 16.8M paths:
+// 15.4 -> 14.2 ms with the tail at 4M rays; 14.5-14.8 at 0.26-1M).
+constexpr int64_t kPathsDirect = (int64_t)1 << 23;
+constexpr int64_t kPathsTail = (int64_t)1 << 22;
+
+// What enqueue_paths needs to hold: unidirectional paths over width-4 trees,
+// nothing counted or captured.
+bool paths_fit(const LoopCfg& L, bool capture) { return !L.bdpt && !L.count && L.width == 4 && !capture; }
+
+// Enqueues k_paths on the rays of the queues that A's shade reads: their
+// paths run to their ends in one launch.  The counters follow to the host.
+int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
+{
+    PathsArgs pa{};
+    pa.s = A.sa;
+    pa.s.ext_primary = primary ? 1 : 0;
+    pa.next = &c->ctr->work[0][0][0];
+    pa.endless = &c->ctr->q[6][0];
+    // the blocks that fit at once
+    const int grid = c->n_cu * paths_waves(pa.s.lmode);
+    if (int r = ensure_overflow(c, L.max_depth - kPathsLds, (int64_t)grid * kPathsBlock)) return r;
+    if (L.max_depth > kPathsLds + c->ovf_depth) return fail(c, YN_ERR_INVALID, "BVH too deep for the traversal stack");
+    pa.ovf_ref = c->ovf_ref;
+    pa.ovf_t = c->ovf_t;
+    pa.ovf_depth = c->ovf_depth;
+    launch_paths(pa, grid, c->stream);
+    HIPCK(c, hipGetLastError());
+    HIPCK(c, hipMemcpyAsync(c->h_ctr, c->ctr, kCtrHostBytes, hipMemcpyDeviceToHost, c->stream));
+    return 0;
+}
+
+// Waits for the batch's last launches and reads its counters.
+int finish_batch(yn_ctx* c, int64_t total, JobRec& stat_job)
+{
+    HIPCK(c, hipStreamSynchronize(c->stream));
+    if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
+    if (c->h_ctr->q[6][0]) return fail(c, YN_ERR_HIP, "paths did not end");
+    stat_job.st.rays_ext += c->h_ctr->rays_ext;
+    stat_job.st.rays_shadow += c->h_ctr->rays_shadow;
+    stat_job.st.nodes_ext += c->h_ctr->nodes_ext;
+    stat_job.st.tris_ext += c->h_ctr->tris_ext;
+    stat_job.st.nodes_shadow += c->h_ctr->nodes_shadow;
+    stat_job.st.tris_shadow += c->h_ctr->tris_shadow;
+    stat_job.st.samples += (uint64_t)total;
+    return 0;
+}
+
+// Runs one batch of primary-ray regions; samples land in samples[slot][pixel]
+// of each region's job (the sample buffer is shared: job slots are laid out
+// by the caller so regions do not overlap).  The last launches may still run
+// when it returns: the caller enqueues what uses the samples and then calls
+// finish_batch with *paths.
+int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, const DevCapture& cap, int64_t* paths)
 {
     std::vector<GenSeg> segs;
     int64_t total = 0;
+    *paths = 0;
     for (const Region& r : regs) {
         GenSeg g{r.job, r.slot, r.rand, r.x0, r.y0, r.w, r.h, (int32_t)total, 0};
         total += (int64_t)r.w * r.h;
         segs.push_back(g);
     }
     if (total == 0) return 0;
+    *paths = total;
     const bool bdpt = c->jobs[regs[0].job].p.mode == YN_MODE_BDPT;
     // paths in flight: the whole batch when it fits, else the capacity, with
     // ended paths' slots regenerated from the remaining work items
@@ -625,7 +686,7 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     const DevScene* scenes = c->d_scenes;
     auto q = [&](int k) { return &c->ctr->q[k][0]; };
     // counters (q(k) = q[k][0]): q[0],q[1] extension queue counts, q[2],q[3] shadow queue
-    // counts, q[7] stack overflow flag, q[8],q[9] path-list counts
+    // counts, q[6] endless-path flag (k_paths), q[7] stack overflow flag, q[8],q[9] path-list counts
     // (bidirectional mode), q[10] free slots (regeneration), q[11] where a
     // regeneration's rays start in their queue; work[0], work[1]
     // the chunk counters of the extend / shadow traces, per queue slice.
@@ -669,6 +730,8 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     if (use_graph)
         if (int r = ensure_group_graph(c, L, iters, group)) return r;
 
+    const bool paths_ok = paths_fit(L, any_cap);
+    if (paths_ok && total <= kPathsDirect && !regen) return enqueue_paths(c, L, iters[0], true);
     int it = 0;
     for (;;) {
         if (use_graph) {
@@ -693,8 +756,13 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
         HIPCK(c, hipStreamSynchronize(s));
         int nxt = it & 1;
         if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
-        if (it > 200000) return fail(c, YN_ERR_HIP, "wavefront loop did not drain");
+        if (it > kMaxIterations) return fail(c, YN_ERR_HIP, "wavefront loop did not drain");
         bool empty = bdpt ? c->h_ctr->q[8 + nxt][0] == 0 : (c->h_ctr->q[nxt][0] == 0 && c->h_ctr->q[2 + nxt][0] == 0);
+        if (paths_ok && !empty && issued == total &&
+            (int64_t)c->h_ctr->q[nxt][0] + c->h_ctr->q[2 + nxt][0] <= kPathsTail) {
+            if (int r = enqueue_paths(c, L, iters[nxt], false)) return r;
+            break;
+        }
         if (regen && issued < total) {
             // new paths behind the rays of the queue the next iteration
             // traces, once there is room for enough of them (or the
@@ -720,13 +788,6 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     stat_job.st.iterations += (uint64_t)it;
     stat_job.st.trace_launches_ext += (uint64_t)it;
     stat_job.st.trace_launches_shadow += (uint64_t)it;
-    stat_job.st.rays_ext += c->h_ctr->rays_ext;
-    stat_job.st.rays_shadow += c->h_ctr->rays_shadow;
-    stat_job.st.nodes_ext += c->h_ctr->nodes_ext;
-    stat_job.st.tris_ext += c->h_ctr->tris_ext;
-    stat_job.st.nodes_shadow += c->h_ctr->nodes_shadow;
-    stat_job.st.tris_shadow += c->h_ctr->tris_shadow;
-    stat_job.st.samples += (uint64_t)total;
     return 0;
 }
 
@@ -773,10 +834,12 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
             int r = upload_job_table(c, jid, c->samples);
             if (r) return r;
             DevCapture cp = f == 0 ? cap : DevCapture{};
-            r = run_batch(c, regs, J, cp);
+            int64_t paths = 0;
+            r = run_batch(c, regs, J, cp, &paths);
             if (r) return r;
             ResolveArgs ra{c->d_jobs, jid, x0, y0, w, h, nslots, (reset_first && f == 0) ? 1 : 0, accum};
             launch_resolve(ra, c->stream);
+            if (int e = finish_batch(c, paths, J)) return e;
         } else {
             // image larger than the path capacity: row bands, one frame at a time
             if ((int64_t)J.W > pcap) return fail(c, YN_ERR_INVALID, "image row wider than the path capacity");
@@ -792,10 +855,12 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
                 int r = upload_job_table(c, jid, base);
                 if (r) return r;
                 DevCapture cp = f == 0 ? cap : DevCapture{};
-                r = run_batch(c, regs, J, cp);
+                int64_t paths = 0;
+                r = run_batch(c, regs, J, cp, &paths);
                 if (r) return r;
                 ResolveArgs ra{c->d_jobs, jid, x0, yb, w, hh, 1, (reset_first && f == 0) ? 1 : 0, accum};
                 launch_resolve(ra, c->stream);
+                if (int e = finish_batch(c, paths, J)) return e;
             }
         }
         f += (size_t)nslots;
@@ -915,14 +980,15 @@ int serve_round(yn_ctx* c, int* frames_out)
     if (regs.empty()) return 0;
     for (const Plan& pl : plan)
         if (int r = upload_job_table(c, pl.jid, c->samples + pl.off)) return r;
-    if (int r = run_batch(c, regs, c->serve_rec, DevCapture{})) return r;
+    int64_t paths = 0;
+    if (int r = run_batch(c, regs, c->serve_rec, DevCapture{}, &paths)) return r;
     for (const Plan& pl : plan) {
         JobRec& J = c->jobs[pl.jid];
         ResolveArgs ra{c->d_jobs, pl.jid, 0, 0, J.W, J.H, pl.k, pl.reset ? 1 : 0, J.accum};
         launch_resolve(ra, c->stream);
     }
     HIPCK(c, hipGetLastError());
-    HIPCK(c, hipStreamSynchronize(c->stream));
+    if (int r = finish_batch(c, paths, c->serve_rec)) return r;
     double now = ms_since(c);
     for (const Plan& pl : plan) {
         JobRec& J = c->jobs[pl.jid];

@@ -89,6 +89,29 @@ struct ShadeArgs {
                                 //    first iteration), whose record holds only m0, m1, rd
 };
 
+// Whole paths in one launch (paths.hip): the paths of the shade arguments'
+// input queues, each from its queued ray to its end.
+struct PathsArgs {
+    ShadeArgs s;
+    uint32_t* next;             // paths taken beyond the static ones, zero at launch
+    uint32_t* endless;          // set to 1 by a path of kMaxPathBounces bounces (it is given up), zero at launch
+    uint32_t* ovf_ref;          // traversal stack overflow area, as in TraceArgs
+    uint16_t* ovf_t;
+    int32_t ovf_depth;
+};
+
+constexpr int kPathsBlock = 256;    // threads per block of k_paths
+// A batch fails after kMaxIterations bounce iterations, or with a path of as
+// many bounces in k_paths: without roulette and a bounce limit a path in a
+// closed scene need not end.
+constexpr int kMaxIterations = 200000;
+constexpr int kMaxPathBounces = kMaxIterations;
+constexpr int kPathsLds = 12;       // traversal stack entries per lane it keeps in LDS
+// Blocks of it per CU, one wave per SIMD each: what its registers (128 at 4)
+// and LDS (stack, materials and light quads: 39 KB, 44 KB with every
+// scene's lights) leave.
+constexpr int paths_waves(int lmode) { return lmode == 2 ? 3 : 4; }
+
 // Materials and light quads (scene slots) the shade kernels stage in LDS
 // (80 B each).
 constexpr int kLdsMats = 256;
@@ -265,6 +288,7 @@ int trace_lds_stack(int lds);   // traversal stack entries kept in LDS for a con
 int trace_resident_waves(int lds);   // waves per SIMD of a trace launch (the default grid fills them)
 void launch_generate(const GenArgs& a, const DevCapture& cap, hipStream_t stream);
 void launch_shade_pt(const ShadeArgs& a, const DevCapture& cap, int grid, int waves, hipStream_t stream);
+void launch_paths(const PathsArgs& a, int grid, hipStream_t stream);
 void launch_generate_bdpt(const GenArgs& a, const DevCapture& cap, hipStream_t stream);
 void launch_shade_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int grid, hipStream_t stream);
 void launch_resolve(const ResolveArgs& a, hipStream_t stream);
