@@ -73,3 +73,18 @@ def test_paths_over_several_scenes():
             alone.set_counting(True)
             alone.render(3)
             assert np.array_equal(j.read().view(np.int32), alone.read().view(np.int32)), k
+
+
+@pytest.mark.parametrize("kw", [dict(mis=1, bdpt_bounces=5), dict(mis=0, bdpt_bounces=1), dict(),
+                                dict(mis=1, bdpt_bounces=40, fix_mis=1)], ids=["mis5", "one", "shipped", "40"])
+@pytest.mark.parametrize("scene", ["cornell", "room", "brute"])
+def test_bidirectional_paths_equal_wavefront(scene, kw):
+    s = Y.gen_icosphere_room(7, 6, 2) if scene == "room" else Y.gen_cornell()
+    params = Y.params_reference(1, **kw)
+    with Y.Context(max_paths=1 << 20) as ctx:
+        sid = ctx.scene(s, brute=scene == "brute")
+        for w, h, f in ((1, 1, 1), (9, 7, 1), (64, 65, 1), (97, 61, 2), (640, 500, 1)):
+            a = render(ctx, sid, s.cam, w, h, f, params, False)
+            b = render(ctx, sid, s.cam, w, h, f, params, True)
+            assert np.array_equal(a[0], b[0]), (w, h, f)
+            assert a[1] == b[1], (w, h, f)

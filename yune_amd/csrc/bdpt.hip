@@ -24,6 +24,7 @@
 // its two lobe picks only when unoccluded (bdpt.cl:611-620).
 #include "yn_internal_dev.h"
 #include "yn_shade.h"
+#include "yn_trace.h"
 
 namespace yune {
 
@@ -116,12 +117,52 @@ __device__ __forceinline__ void set_ray(BOut& r, f4 o, f4 d, float tmax, int id)
     r.d_p = make_float4(d.x, d.y, d.z, __int_as_float(id));
 }
 
-template <bool CAP, int LM>
-__device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int p, const LdsScene& lds)
+// A path's scalars and colour between two steps (the record's I0, I1, I2 and
+// DIRECT).
+struct BState {
+    int4 i0, i1, i2;
+    f4 color;
+};
+
+__device__ __forceinline__ BState load_state(const BdptSoA& B, int p)
 {
-    const PathSoA& P = a.P;
+    return BState{ld_i4(B, BF::I0, p), ld_i4(B, BF::I1, p), ld_i4(B, BF::I2, p), ld(*B.R.f(BF::DIRECT, p))};
+}
+
+__device__ __forceinline__ void store_state(const BdptSoA& B, int p, const BState& s)
+{
+    *reinterpret_cast<int4*>(B.R.f(BF::I0, p)) = s.i0;
+    *reinterpret_cast<int4*>(B.R.f(BF::I1, p)) = s.i1;
+    *reinterpret_cast<int4*>(B.R.f(BF::I2, p)) = s.i2;
+    *B.R.f(BF::DIRECT, p) = st4(s.color);
+}
+
+// The results of a path's rays in the results arrays.
+struct BQueueResult {
+    const float4* hit_at;
+    const int32_t* occ_at;
+    size_t slot0;           // the path's first shadow-ray slot
+    int path;
+    __device__ __forceinline__ float4 hit() const { return hit_at[path]; }
+    __device__ __forceinline__ int occ(int j) const { return occ_at[slot0 + (size_t)j]; }
+};
+
+// The results in the lane's registers (k_paths_bdpt).
+struct BRegResult {
+    float4 r;               // the closest hit, or any-hit results as bits in x, y
+    __device__ __forceinline__ float4 hit() const { return r; }
+    __device__ __forceinline__ int occ(int j) const
+    {
+        return (int)((((uint64_t)__float_as_uint(r.x) | ((uint64_t)__float_as_uint(r.y) << 32)) >> j) & 1u);
+    }
+};
+
+template <bool CAP, int LM, typename RES>
+__device__ __forceinline__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int p, int jid,
+                                             const RES& res, BState& bs, const LdsScene& lds)
+{
     const BdptSoA& B = a.B;
-    const DevJob& J = a.jobs[P.job[p]];
+    const DevJob& J = a.jobs[jid];
     const yn_render_params& RP = J.p;
     const DevScene& S = a.scenes[J.scene];
     // LM: materials and light in LDS, the launch's one scene's (1) or every scene's (2)
@@ -132,7 +173,7 @@ __device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int 
     const bool fix = RP.fix_mis != 0;
     const int KB = RP.bdpt_bounces;
 
-    const int4 i0 = ld_i4(B, BF::I0, p), i1 = ld_i4(B, BF::I1, p), i2 = ld_i4(B, BF::I2, p);
+    const int4 i0 = bs.i0, i1 = bs.i1, i2 = bs.i2;
     int st = i0.y;
     const int code = st & B_MASK;
     uint32_t seed = (uint32_t)i0.x;
@@ -142,7 +183,7 @@ __device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int 
     int k = i0.z;
     int lp_len = i1.y, ep_len = i1.z;
     float w_eye = __int_as_float(i1.w);
-    f4 color = ld(*B.R.f(BF::DIRECT, p));
+    f4 color = bs.color;
     uint64_t conn = (uint64_t)(uint32_t)i2.x | ((uint64_t)(uint32_t)i2.y << 32);
     float nee_prob = __int_as_float(i2.z);     // NEE lobe probability, carried between rounds
 
@@ -156,7 +197,7 @@ __device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int 
 
     if (code == B_LIGHT || code == B_EYE) {
         const int side = code == B_LIGHT ? 0 : 1;
-        float4 h = P.hit[p];
+        float4 h = res.hit();
         int htri = __float_as_int(h.y);
         if (side == 1 && k == 0) {          // camera ray (createEyePath :517-528, shading :566-571)
             if (cap_on) {
@@ -321,7 +362,7 @@ __device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int 
             Vtx e = load_v(B, 1, k, p);
             Mat m = mat_of(e.mat);
             if (st & BF_NEE_DONE) { nee_res = ld(*B.R.f(BF::LS, p)); step = T_CONNECT; break; }
-            int occ = (st & BF_NEE_Q) ? 1 : B.occ[((size_t)p << B.shift)];
+            int occ = (st & BF_NEE_Q) ? 1 : res.occ(0);
             if (cap_on && k == 0 && !(st & BF_CAPSH)) { cap.shadow_occ[pix] = occ; st |= BF_CAPSH; }
             float4 w4 = *B.R.f(BF::WI, p);
             f4 wi = mk(w4.x, w4.y, w4.z, 0.0f);
@@ -364,7 +405,7 @@ __device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int 
             Mat m = mat_of(e.mat);
             f4 em = m.ke;
             f4 ls = ld(*B.R.f(BF::LS, p));
-            int occ = B.occ[((size_t)p << B.shift)];
+            int occ = res.occ(0);
             if (occ) { nee_res = ls + em; step = T_CONNECT; break; }
             float4 mb = *B.R.f(BF::MIS, p);
             f4 bd = mk(mb.x, mb.y, mb.z, 0.0f);
@@ -390,7 +431,7 @@ __device__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int 
             f4 sub = mk(0, 0, 0, 1);
             for (int j = lp_len - 1; j > 0; --j) {
                 if (!((conn >> j) & 1ull)) continue;
-                if (B.occ[((size_t)p << B.shift) + (size_t)j]) continue;
+                if (res.occ(j)) continue;
                 Vtx l = load_v(B, 0, j, p);
                 f4 d = normalize(l.p - e.p);
                 float dist = length(l.p - e.p);
@@ -422,11 +463,10 @@ emitted:
         write_sample(J, slot, pix, mk(NAN, NAN, NAN, NAN));
         ended = true;
     }
-    *reinterpret_cast<int4*>(B.R.f(BF::I0, p)) = make_int4((int)seed, ended ? B_DONE : st, k, pix);
-    *reinterpret_cast<int4*>(B.R.f(BF::I1, p)) = make_int4(slot, lp_len, ep_len, __float_as_int(w_eye));
-    *reinterpret_cast<int4*>(B.R.f(BF::I2, p)) =
-        make_int4((int)(uint32_t)conn, (int)(uint32_t)(conn >> 32), __float_as_int(nee_prob), 0);
-    *B.R.f(BF::DIRECT, p) = st4(color);
+    bs.i0 = make_int4((int)seed, ended ? B_DONE : st, k, pix);
+    bs.i1 = make_int4(slot, lp_len, ep_len, __float_as_int(w_eye));
+    bs.i2 = make_int4((int)(uint32_t)conn, (int)(uint32_t)(conn >> 32), __float_as_int(nee_prob), 0);
+    bs.color = color;
     return out;
 }
 
@@ -463,7 +503,10 @@ __global__ __launch_bounds__(256, 3) void k_shade_bdpt(BdptShadeArgs a, DevCaptu
         int p = -1;
         if (i < n) {
             p = (int)a.list_in[i];
-            o = advance_bdpt<CAP, LM>(a, cap, p, lds);
+            const int jid = a.P.job[p];
+            BState bs = load_state(a.B, p);
+            o = advance_bdpt<CAP, LM>(a, cap, p, jid, BQueueResult{a.P.hit, a.B.occ, (size_t)p << shift, p}, bs, lds);
+            store_state(a.B, p, bs);
         }
         const bool more = o.ext || o.emit != 0;
         const uint32_t cnt[3] = {o.ext ? 1u : 0u, (uint32_t)__popcll(o.emit), more ? 1u : 0u};
@@ -500,20 +543,20 @@ __global__ __launch_bounds__(256, 3) void k_shade_bdpt(BdptShadeArgs a, DevCaptu
     }
 }
 
-// Camera ray, light vertex 0 and the first light ray (bdpt.cl:162-189,
-// createLightPath :432-462) for a list of segments.
-__global__ __launch_bounds__(256) void k_generate_bdpt(GenArgs a, DevCapture cap)
+// Work item -> path slot p: camera ray, light vertex 0 and the first light
+// ray (bdpt.cl:162-189, createLightPath :432-462).  Returns the path's
+// job-table entry; ray: the path's first ray.
+__device__ __forceinline__ int start_bdpt(const GenArgs& a, const DevCapture& cap, int item, int p, BState& bs,
+                                          float4& ot, float4& dp)
 {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= a.n_paths) return;
     int lo = 0, hi = a.n_segs - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
-        if (a.segs[mid].path_base <= p) lo = mid; else hi = mid - 1;
+        if (a.segs[mid].path_base <= item) lo = mid; else hi = mid - 1;
     }
     const GenSeg& g = a.segs[lo];
     int x, y;
-    seg_pixel(p - g.path_base + g.first, g.w, g.h, x, y);
+    seg_pixel(item - g.path_base + g.first, g.w, g.h, x, y);
     x += g.x0;
     y += g.y0;
     const DevJob& J = a.jobs[g.job];
@@ -559,20 +602,190 @@ __global__ __launch_bounds__(256) void k_generate_bdpt(GenArgs a, DevCapture cap
     }
     float tq, tmax = INFINITY;
     if (quad_hit(L, o, d, INFINITY, tq)) { tmax = tq; st |= BF_LCAND; }
-    a.P.job[p] = g.job;
     // bounce: 1 when the first light ray leaves vertex 0, else 0 (the camera ray)
-    *reinterpret_cast<int4*>(B.R.f(BF::I0, p)) = make_int4((int)seed, st, pdf > 0.0f ? 1 : 0, y * J.W + x);
-    *reinterpret_cast<int4*>(B.R.f(BF::I1, p)) = make_int4(g.slot, 1, 0, __float_as_int(1.0f));
-    *reinterpret_cast<int4*>(B.R.f(BF::I2, p)) = make_int4(0, 0, 0, 0);
-    *B.R.f(BF::DIRECT, p) = make_float4(0, 0, 0, 1);
-    a.ext_out.o_t[p] = make_float4(o.x, o.y, o.z, tmax);
-    a.ext_out.d_p[p] = make_float4(d.x, d.y, d.z, __int_as_float(p));
-    a.list_out[p] = (uint32_t)p;
-    if (p == 0) { *a.ext_out.count = (uint32_t)a.n_paths; *a.list_count = (uint32_t)a.n_paths; }
+    bs.i0 = make_int4((int)seed, st, pdf > 0.0f ? 1 : 0, y * J.W + x);
+    bs.i1 = make_int4(g.slot, 1, 0, __float_as_int(1.0f));
+    bs.i2 = make_int4(0, 0, 0, 0);
+    bs.color = mk(0, 0, 0, 1);
+    ot = make_float4(o.x, o.y, o.z, tmax);
+    dp = make_float4(d.x, d.y, d.z, __int_as_float(p));
     if (cap.prim_tri && g.slot == 0) {
         cap.shadow_occ[y * J.W + x] = -1;
         cap.shadow_d[y * J.W + x] = make_float4(0, 0, 0, 0);
     }
+    return g.job;
+}
+
+// The paths of a list of segments, each in its own slot and listed.
+__global__ __launch_bounds__(256) void k_generate_bdpt(GenArgs a, DevCapture cap)
+{
+    int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= a.n_paths) return;
+    BState bs;
+    float4 ot, dp;
+    a.P.job[p] = start_bdpt(a, cap, p, p, bs, ot, dp);
+    store_state(a.B, p, bs);
+    a.ext_out.o_t[p] = ot;
+    a.ext_out.d_p[p] = dp;
+    a.list_out[p] = (uint32_t)p;
+    if (p == 0) { *a.ext_out.count = (uint32_t)a.n_paths; *a.list_count = (uint32_t)a.n_paths; }
+}
+
+// Idle lanes of a wave before k_paths_bdpt makes new paths: they start at the
+// first stage and the others wait for them (4.2M paths of the Cornell box, 5
+// vertices: 64, 13.5 ms; 56, 13.4; 48, 13.6; each lane at once, 20).
+constexpr int kBdptRefill = 56;
+
+// Whole bidirectional paths in one launch, as k_paths (paths.hip): each lane
+// makes a path, traces its rays one after the other (a round's shadow rays
+// too, their results bits of a mask) and runs the steps between, until the
+// path ends; then it takes another work item.  The path's vertices and
+// pending-ray fields stay in memory, in the slot of the lane (not of the
+// path), so that they stay in cache; its scalars and colour in registers.
+//
+// Bound by vector issue with few lanes at work (84% busy, 16% of the lanes,
+// before the stages below).  The wavefront is bound by launches and the
+// longest ray of each: 640x360 of the Cornell box, 5 vertices, 2,018 -> 1,105
+// us.  Lanes of a wave go through the stages of a path together and wait for
+// each other there: 4.2M paths of the Cornell box 15.7 -> 13.5 ms, of a
+// 15k-triangle room 45.9 -> 33.8.  128 registers with 88 spilled, at 4 waves
+// per SIMD: 12.0 and 29.2 ms; 3 waves (39 spilled): 13.4 and 33.5; 2 waves
+// (none): 17.4 and 44.1; 5 waves (270): 15.4 and 31.0.
+template <int LM>
+__global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(BdptPathsArgs a)
+{
+    constexpr int BL = kPathsBlock;
+    __shared__ uint32_t stk_all[kPathsLds * BL];
+    __shared__ uint16_t stkt_all[kPathsLds * BL];
+    __shared__ float4 smat4[LM ? kLdsMats * 5 : 1];
+    __shared__ float4 slight4[LM == 2 ? kLdsLights * 5 : LM == 1 ? 5 : 1];
+    const BdptShadeArgs& s = a.s;
+    if (LM) {
+        for (int k = (int)threadIdx.x; k < s.n_lmats * 5; k += BL) smat4[k] = s.lmats[k];
+        for (int k = (int)threadIdx.x; k < s.n_lights * 5; k += BL)
+            slight4[k] = reinterpret_cast<const float4*>(&s.scenes[LM == 1 ? s.lscene : k / 5].light)[k % 5];
+        __syncthreads();
+    }
+    const LdsScene lds{(lds_mat*)(void*)smat4, (lds_light*)(void*)slight4};
+    Stack<kPathsLds, BL> st;
+    st.lref = (lds_u32*)stk_all;
+    st.lt = (lds_u16*)stkt_all;
+    st.col = threadIdx.x;
+    st.gstride = gridDim.x * BL;
+    st.gref = (gbl_u32*)a.ovf_ref;
+    st.gt = (gbl_u16*)a.ovf_t;
+    st.gbase = blockIdx.x * BL;
+    st.gcap = a.ovf_depth;
+    st.full = &a.ctr->q[7][0];
+    const int lane = (int)__lane_id();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const uint32_t total = (uint32_t)a.g.n_paths;
+    // few paths spread over all waves, as in k_paths
+    const uint32_t n_waves = gridDim.x * (BL / 64);
+    const uint32_t per = min(64u, (total + n_waves - 1) / n_waves);
+    const uint32_t wave = blockIdx.x * (BL / 64) + (threadIdx.x >> 6);
+    const int p = (int)(wave * per) + lane;         // the lane's slot (used by lanes below `per` only)
+    bool more = total > n_waves * per;
+    const bool mine = (uint32_t)lane < per && (uint32_t)p < total;
+    BState bs;
+    bs.i0 = make_int4(0, B_DONE, 0, 0);
+    float4 ot = make_float4(0, 0, 0, 0), dp = ot;   // the next ray (a round's first)
+    float4 res = ot;                                // closest hit, or the round's any-hit results as bits in x, y
+    bool ext = false;                               // the next ray is an extension ray
+    uint64_t emit = 0;                              // the round's shadow rays still to trace
+    int jid = 0;
+    const DevCapture cap{};
+    bool live = mine;
+    if (live) {
+        jid = start_bdpt(a.g, cap, p, p, bs, ot, dp);
+        ext = true;
+    }
+    unsigned long long n_rays[2] = {0, 0};          // closest-hit and any-hit, of the wave
+    Counts c{0, 0};
+    for (;;) {
+        if (!__ballot(live)) break;
+        // the lanes at the earliest stage go on, the others wait for them:
+        // a wave's lanes then run the same steps, light subpaths, eye
+        // subpaths and rounds each together
+        const int code = bs.i0.y & B_MASK;
+        const int stage = __ballot(live && code == B_LIGHT) ? 0 : __ballot(live && code == B_EYE) ? 1 : 2;
+        const bool act = live && (code == B_LIGHT ? 0 : code == B_EYE ? 1 : 2) == stage;
+        const unsigned long long shadow = __ballot(act && emit != 0);
+        n_rays[0] += (unsigned)__popcll(__ballot(act && ext));
+        n_rays[1] += (unsigned)__popcll(shadow);
+        if (act && (ext || emit != 0)) {
+            const DevScene& S = s.scenes[LM == 1 ? s.lscene : s.jobs[jid].scene];
+            const int j = ext ? 0 : __ffsll((long long)emit) - 1;
+            if (j > 0) {            // a connection ray, made exactly as when it was counted
+                const Vtx ev = load_v(s.B, 1, bs.i0.z, p), l = load_v(s.B, 0, j, p);
+                f4 ro, rd;
+                float len;
+                conn_ray(ev, l, ro, rd, len);
+                ot = make_float4(ro.x, ro.y, ro.z, len);
+                dp = make_float4(rd.x, rd.y, rd.z, 0.0f);
+            }
+            RayState r;
+            const bool fma_ok = start_ray(r, ot, dp, S);
+            r.any = !ext;
+            st.sp = 0;
+            // a ray with a NaN component hits nothing (see k_trace)
+            const bool nan_ray = !(ot.x == ot.x && ot.y == ot.y && ot.z == ot.z && ot.w == ot.w && dp.x == dp.x &&
+                                   dp.y == dp.y && dp.z == dp.z);
+            bool got = false;
+            uint32_t node = 0;
+            bool go = !nan_ray && trav_start<2, false>(S, r, node, got, c);
+            const float4 *nodes = S.nodes, *tri = S.tri_isect;
+            if (__ballot(!fma_ok)) {
+                while (go) go = trav_step<4, 2, kPathsLds, BL, false, true>(nodes, tri, node, r, st, got, c);
+            } else {
+                while (go) go = trav_step<4, 2, kPathsLds, BL, false, false>(nodes, tri, node, r, st, got, c);
+            }
+            if (ext) {
+                res = make_float4(r.best, __int_as_float(r.tri), r.u, r.v);
+                ext = false;
+            } else {
+                const uint64_t bit = 1ull << j;
+                uint64_t occ = (uint64_t)__float_as_uint(res.x) | ((uint64_t)__float_as_uint(res.y) << 32);
+                occ = got ? occ | bit : occ & ~bit;
+                res.x = __uint_as_float((uint32_t)occ);
+                res.y = __uint_as_float((uint32_t)(occ >> 32));
+                emit &= ~bit;
+            }
+        }
+        // a step once every lane of the stage has all its rays' results
+        if (__ballot(act && emit != 0) == 0 && act) {
+            const BOut o = advance_bdpt<false, LM>(s, cap, p, jid, BRegResult{res}, bs, lds);
+            ot = o.o_t;
+            dp = o.d_p;
+            ext = o.ext;
+            emit = o.emit;
+            live = ext || emit != 0;
+        }
+        if (more) {         // lanes whose paths have ended take the next work items, most of a wave at once
+            const unsigned long long idle = __ballot(!live);
+            if (__popcll(idle) >= kBdptRefill) {
+                uint32_t b = 0;
+                if (lane == 0) b = atomicAdd(a.next, (uint32_t)__popcll(idle));
+                b = n_waves * per + __shfl(b, 0);
+                if (b >= total) more = false;
+                const uint32_t i = b + (uint32_t)__popcll(idle & below);
+                if (!live && i < total) {
+                    jid = start_bdpt(a.g, cap, (int)i, p, bs, ot, dp);
+                    ext = live = true;
+                }
+            }
+        }
+    }
+    if (lane == 0 && n_rays[0]) atomicAdd(&a.ctr->rays_ext, n_rays[0]);
+    if (lane == 0 && n_rays[1]) atomicAdd(&a.ctr->rays_shadow, n_rays[1]);
+}
+
+void launch_paths_bdpt(const BdptPathsArgs& a, int grid, hipStream_t s)
+{
+    const int lm = a.s.lmats != nullptr && a.s.n_lmats <= kLdsMats ? a.s.lmode : 0;
+    if (lm == 1) hipLaunchKernelGGL((k_paths_bdpt<1>), dim3(grid), dim3(kPathsBlock), 0, s, a);
+    else if (lm == 2) hipLaunchKernelGGL((k_paths_bdpt<2>), dim3(grid), dim3(kPathsBlock), 0, s, a);
+    else hipLaunchKernelGGL((k_paths_bdpt<0>), dim3(grid), dim3(kPathsBlock), 0, s, a);
 }
 
 void launch_generate_bdpt(const GenArgs& a, const DevCapture& cap, hipStream_t s)

@@ -605,10 +605,17 @@ int ensure_group_graph(yn_ctx* c, const LoopCfg& L, const IterArgs (&iters)[2], 
 // 15.4 -> 14.2 ms with the tail at 4M rays; 14.5-14.8 at 0.26-1M).
 constexpr int64_t kPathsDirect = (int64_t)1 << 23;
 constexpr int64_t kPathsTail = (int64_t)1 << 22;
+// Bidirectional batches in k_paths_bdpt from the start, else in the wavefront
+// to the end (5 vertices, wavefront against k_paths_bdpt):
+//                  262,144 paths     1M paths          4.2M paths
+//   Cornell box    2.36 / 1.13 ms    5.70 / 3.35 ms    14.6 / 12.1 ms
+//   15k triangles  4.20 / 2.16 ms    9.02 / 7.82 ms    29.5 / 29.3 ms
+// and with 20 vertices at 15k triangles 38.2 / 36.4 ms at 1M paths, 124 /
+// 134 ms at 4.2M.
+constexpr int64_t kPathsDirectBdpt = (int64_t)1 << 21;
 
-// What enqueue_paths needs to hold: unidirectional paths over width-4 trees,
-// nothing counted or captured.
-bool paths_fit(const LoopCfg& L, bool capture) { return !L.bdpt && !L.count && L.width == 4 && !capture; }
+// What whole-path launches need: width-4 trees, nothing counted or captured.
+bool paths_fit(const LoopCfg& L, bool capture) { return !L.count && L.width == 4 && !capture; }
 
 // Enqueues k_paths on the rays of the queues that A's shade reads: their
 // paths run to their ends in one launch.  The counters follow to the host.
@@ -627,6 +634,26 @@ int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
     pa.ovf_t = c->ovf_t;
     pa.ovf_depth = c->ovf_depth;
     launch_paths(pa, grid, c->stream);
+    HIPCK(c, hipGetLastError());
+    HIPCK(c, hipMemcpyAsync(c->h_ctr, c->ctr, kCtrHostBytes, hipMemcpyDeviceToHost, c->stream));
+    return 0;
+}
+
+// The same for bidirectional paths, from the work items of g on.
+int enqueue_paths_bdpt(yn_ctx* c, const LoopCfg& L, const IterArgs& A, const GenArgs& g)
+{
+    BdptPathsArgs pa{};
+    pa.s = A.ba;
+    pa.g = g;
+    pa.next = &c->ctr->work[0][0][0];
+    pa.ctr = c->ctr;
+    const int grid = c->n_cu * paths_waves(pa.s.lmode);
+    if (int r = ensure_overflow(c, L.max_depth - kPathsLds, (int64_t)grid * kPathsBlock)) return r;
+    if (L.max_depth > kPathsLds + c->ovf_depth) return fail(c, YN_ERR_INVALID, "BVH too deep for the traversal stack");
+    pa.ovf_ref = c->ovf_ref;
+    pa.ovf_t = c->ovf_t;
+    pa.ovf_depth = c->ovf_depth;
+    launch_paths_bdpt(pa, grid, c->stream);
     HIPCK(c, hipGetLastError());
     HIPCK(c, hipMemcpyAsync(c->h_ctr, c->ctr, kCtrHostBytes, hipMemcpyDeviceToHost, c->stream));
     return 0;
@@ -706,15 +733,6 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     ga.segs = c->d_segs;
     ga.n_segs = (int32_t)segs.size();
     ga.n_paths = (int32_t)issued;
-    if (bdpt) {
-        ga.B = c->B;
-        ga.list_out = c->lst[0];
-        ga.list_count = q(8);
-        launch_generate_bdpt(ga, cap, s);
-    } else {
-        launch_generate(ga, cap, s);
-    }
-
     std::vector<int> scene_ids;
     for (const Region& r : regs) scene_ids.push_back(c->jobs[r.job].scene);
     LoopCfg L;
@@ -723,15 +741,24 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     IterArgs iters[2];
     make_iter(c, L, 0, iters[0]);
     make_iter(c, L, 1, iters[1]);
+    const bool any_cap = cap.prim_tri || cap.prim_light || cap.prim_t || cap.shadow_o || cap.shadow_d || cap.shadow_occ;
+    const bool paths_ok = paths_fit(L, any_cap);
+    if (bdpt) {
+        ga.B = c->B;
+        ga.list_out = c->lst[0];
+        ga.list_count = q(8);
+        if (paths_ok && total <= kPathsDirectBdpt) return enqueue_paths_bdpt(c, L, iters[0], ga);
+        launch_generate_bdpt(ga, cap, s);
+    } else {
+        launch_generate(ga, cap, s);
+        if (paths_ok && total <= kPathsDirect && !regen) return enqueue_paths(c, L, iters[0], true);
+    }
     const int group = 4;                 // iterations between host checks (even)
     // Graph replay of a group (not with ray capture for tests)
-    const bool any_cap = cap.prim_tri || cap.prim_light || cap.prim_t || cap.shadow_o || cap.shadow_d || cap.shadow_occ;
     const bool use_graph = c->cfg.graph != 0 && !any_cap;
     if (use_graph)
         if (int r = ensure_group_graph(c, L, iters, group)) return r;
 
-    const bool paths_ok = paths_fit(L, any_cap);
-    if (paths_ok && total <= kPathsDirect && !regen) return enqueue_paths(c, L, iters[0], true);
     int it = 0;
     for (;;) {
         if (use_graph) {
@@ -758,7 +785,7 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
         if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
         if (it > kMaxIterations) return fail(c, YN_ERR_HIP, "wavefront loop did not drain");
         bool empty = bdpt ? c->h_ctr->q[8 + nxt][0] == 0 : (c->h_ctr->q[nxt][0] == 0 && c->h_ctr->q[2 + nxt][0] == 0);
-        if (paths_ok && !empty && issued == total &&
+        if (paths_ok && !bdpt && !empty && issued == total &&
             (int64_t)c->h_ctr->q[nxt][0] + c->h_ctr->q[2 + nxt][0] <= kPathsTail) {
             if (int r = enqueue_paths(c, L, iters[nxt], false)) return r;
             break;

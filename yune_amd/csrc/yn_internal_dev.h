@@ -107,7 +107,8 @@ constexpr int kPathsBlock = 256;    // threads per block of k_paths
 constexpr int kMaxIterations = 200000;
 constexpr int kMaxPathBounces = kMaxIterations;
 constexpr int kPathsLds = 12;       // traversal stack entries per lane it keeps in LDS
-// Blocks of it per CU, one wave per SIMD each: what its registers (128 at 4)
+// Blocks of it (and of k_paths_bdpt) per CU, one wave per SIMD each: what
+// its registers (128 at 4)
 // and LDS (stack, materials and light quads: 39 KB, 44 KB with every
 // scene's lights) leave.
 constexpr int paths_waves(int lmode) { return lmode == 2 ? 3 : 4; }
@@ -157,6 +158,18 @@ struct GenArgs {
     // the launch sets the queue's count
     int32_t item0;
     uint32_t* queue_base;
+};
+
+// Whole bidirectional paths in one launch (k_paths_bdpt): the work items of
+// g, in slots of s.B.
+struct BdptPathsArgs {
+    BdptShadeArgs s;
+    GenArgs g;
+    uint32_t* next;             // as in PathsArgs
+    uint32_t* ovf_ref;
+    uint16_t* ovf_t;
+    int32_t ovf_depth;
+    DevCounters* ctr;
 };
 
 struct ResolveArgs {
@@ -289,6 +302,7 @@ int trace_resident_waves(int lds);   // waves per SIMD of a trace launch (the de
 void launch_generate(const GenArgs& a, const DevCapture& cap, hipStream_t stream);
 void launch_shade_pt(const ShadeArgs& a, const DevCapture& cap, int grid, int waves, hipStream_t stream);
 void launch_paths(const PathsArgs& a, int grid, hipStream_t stream);
+void launch_paths_bdpt(const BdptPathsArgs& a, int grid, hipStream_t stream);
 void launch_generate_bdpt(const GenArgs& a, const DevCapture& cap, hipStream_t stream);
 void launch_shade_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int grid, hipStream_t stream);
 void launch_resolve(const ResolveArgs& a, hipStream_t stream);
