@@ -1,0 +1,79 @@
+"""Caller's rays in one launch (k_rays): calls of every size give each ray
+the result it has in a call of its own block.
+
+Small calls read and write pinned host memory, larger ones the samples
+buffer; up to one ray per lane a wave takes an equal share of the rays,
+beyond that the lanes are refilled.  The blocks of 1,000 rays that the
+results are compared with are themselves compared with the oracle by
+test_trace_matches_oracle.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import yune_amd as Y
+from yune_amd._lib import lib
+
+pytestmark = pytest.mark.gpu
+
+LANES12, LANES16 = 256 * 7 * 256, 256 * 6 * 256        # rays a grid holds at 12 and 16 stack entries
+
+
+def mixed_rays(n, seed):
+    rng = np.random.default_rng(seed)
+    r = np.zeros((n, 8), np.float32)
+    r[:, :3] = rng.uniform(-4.9, 4.9, (n, 3))
+    r[:, 4:7] = rng.normal(size=(n, 3))
+    r[:, 7] = rng.uniform(size=n) < 0.3
+    r[:, 3] = np.where(r[:, 7] != 0, rng.uniform(0.05, 6.0, n), np.inf)
+    r[::97, 4] = 0.0                    # axis-parallel, NaN, infinite and empty rays among them
+    r[::101, 5] = np.nan
+    r[::103, 3] = 0.0
+    r[::107, 0] = np.inf
+    return r
+
+
+def same(a, b):
+    return all(np.array_equal(x.view(np.int32), y.view(np.int32)) for x, y in zip(a, b))
+
+
+@pytest.fixture(scope="module")
+def room():
+    return Y.gen_icosphere_room(11, 12, 4)
+
+
+@pytest.mark.parametrize("opts", [dict(), dict(bvh_width=2), dict(lds_stack=12, trace_xcd=3), dict(trace_refill=-1)],
+                         ids=["default", "width2", "lds12-xcd3", "norefill"])
+def test_call_sizes_give_the_same_results(room, opts):
+    rays = mixed_rays(LANES12 + 70_001, 5)
+    with Y.Context(max_paths=1 << 20, **opts) as c:
+        sid = c.scene(room)
+        # any-hit occluders depend on nothing but the tree, so all three arrays compare
+        want = [np.concatenate(x) for x in zip(*(c.trace(sid, rays[i:i + 1000]) for i in range(0, 12_000, 1000)))]
+        full = c.trace(sid, rays)
+        assert same([x[:12_000] for x in full], want)
+        for n in (1, 2, 63, 64, 65, 1000, 8191, 8192, 8193, LANES16 - 1, LANES16, LANES16 + 1, LANES12, LANES12 + 1):
+            assert same(c.trace(sid, rays[:n]), [x[:n] for x in full]), n
+
+
+@pytest.mark.parametrize("brute", [False, True])
+def test_device_rays_at_any_alignment(brute):
+    torch = pytest.importorskip("torch")
+    s = Y.gen_cornell()
+    n = 5003
+    rays = mixed_rays(n, 8)
+    rays[:, :3] = rays[:, :3] * 0.2 + np.float32([0, 0, -3])
+    with Y.Context(max_paths=1 << 16) as c:
+        sid = c.scene(s, brute=brute)
+        want = c.trace(sid, rays)
+        for off in (0, 1, 2, 3, 4):     # floats
+            d = torch.zeros(n * 8 + 8, device="cuda")
+            d[off:off + n * 8] = torch.from_numpy(rays.reshape(-1)).cuda()
+            out = [torch.full((n + 3,), -7, dtype=t, device="cuda") for t in (torch.int32, torch.int32, torch.float32)]
+            torch.cuda.synchronize()
+            p = [C.c_void_p(o.data_ptr() + 4) for o in out]
+            assert lib().yn_trace_noalloc(c._p, sid, C.c_void_p(d.data_ptr() + 4 * off), n, *p) == 0
+            got = [o.cpu().numpy() for o in out]
+            assert same([g[1:n + 1] for g in got], want), off
+            assert all((g[0] == -7) and (g[n + 1:] == -7).all() for g in got)

@@ -741,7 +741,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
                 while (go) go = trav_step<4, 2, kPathsLds, BL, false, false>(nodes, tri, node, r, st, got, c);
             }
             if (ext) {
-                res = make_float4(r.best, __int_as_float(r.tri), r.u, r.v);
+                res = hit_record(r);
                 ext = false;
             } else {
                 const uint64_t bit = 1ull << j;

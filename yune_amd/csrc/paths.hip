@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
             }
             unpack(q, r, R);
             const Out o = advance<false, LM>(
-                s, cap, RegResult{make_float4(r.best, __int_as_float(r.tri), r.u, r.v), got ? 1 : 0}, R, lds);
+                s, cap, RegResult{hit_record(r), got ? 1 : 0}, R, lds);
             q = pack(R);
             ot = o.o_t;
             dp = o.d_p;

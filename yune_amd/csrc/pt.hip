@@ -224,25 +224,6 @@ __global__ __launch_bounds__(256) void k_tonemap(const float4* in, float4* out, 
     out[i] = make_float4(ynf_powf(ldr.x, g), ynf_powf(ldr.y, g), ynf_powf(ldr.z, g), ynf_powf(ldr.w, g));
 }
 
-// Rays given by a caller (n x 8 floats: o, len, d, is_shadow): quad test
-// (traceRay, udpt.cl:244-276) and queue fill.  hit/occ slots are indexed by
-// ray number.
-__global__ __launch_bounds__(256) void k_prepare_rays(const DevScene* scene, const float* rays, int n, RayQueue q,
-                                                      int32_t* light_out)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float* r = rays + 8 * (size_t)i;
-    f4 o = mk(r[0], r[1], r[2], 1.0f), d = mk(r[4], r[5], r[6], 0.0f);
-    float len = r[3], t;
-    int light = -1;
-    if (quad_hit(scene->light, o, d, len, t)) { len = t; light = 0; }
-    light_out[i] = light;
-    q.o_t[i] = make_float4(o.x, o.y, o.z, len);
-    q.d_p[i] = make_float4(d.x, d.y, d.z, __int_as_float(i));
-    if (i == 0) *q.count = (uint32_t)n;
-}
-
 // The kernels' sin / cos / pow evaluated on the device (diagnostics).
 __global__ __launch_bounds__(256) void k_fmath(int op, const float* x, const float* y, int n, float* out)
 {
@@ -300,10 +281,6 @@ void launch_resolve(const ResolveArgs& a, hipStream_t s)
 void launch_tonemap(const float4* in, float4* out, int n, int op, hipStream_t s)
 {
     if (n > 0) hipLaunchKernelGGL(k_tonemap, dim3((n + 255) / 256), dim3(256), 0, s, in, out, n, op);
-}
-void launch_prepare(const DevScene* scene, const float* rays, int n, RayQueue q, int32_t* light_out, hipStream_t s)
-{
-    if (n > 0) hipLaunchKernelGGL(k_prepare_rays, dim3((n + 255) / 256), dim3(256), 0, s, scene, rays, n, q, light_out);
 }
 
 }  // namespace yune

@@ -172,6 +172,8 @@ struct yn_ctx {
     StreamState strm;                 // continuous serving
     uint32_t* done_ctr = nullptr;     // per piece: paths ended (device)
     uint32_t* h_done = nullptr;       // pinned mirror
+    float* h_rays = nullptr;          // pinned: rays and results of small yn_trace calls
+    uint32_t* h_full = nullptr;       // pinned: stack overflow flag of caller rays
 };
 
 namespace {
@@ -1450,6 +1452,24 @@ int build_scene(yn_ctx* c, int sid, int width)
     return 0;
 }
 
+// Caller's rays (k_rays): launches of the blocks that fit at once, so that a
+// call of few rays spreads them over every wave of the chip.
+constexpr int kRaysHost = 8192;
+
+int rays_grid(const yn_ctx* c, int lds) { return c->n_cu * trace_resident_waves(rays_lds_stack(lds)); }
+
+RaysArgs rays_args(yn_ctx* c, int sid, int n)
+{
+    RaysArgs a{};
+    a.scene = c->d_scenes + sid;
+    a.n = n;
+    a.work = &c->ctr->work[0][0][0];
+    a.n_slices = c->cfg.trace_xcd;
+    a.refill = c->cfg.trace_refill > 0 ? c->cfg.trace_refill : 64;
+    a.full = c->h_full;         // pinned: no copy back for a flag that is hardly ever set
+    return a;
+}
+
 int check_ctx(yn_ctx* c) { return c ? 0 : fail(nullptr, YN_ERR_INVALID, "null context"); }
 int check_job(yn_ctx* c, int jid)
 {
@@ -1558,7 +1578,9 @@ int yn_create(const yn_config* cfg, yn_ctx** out)
     c->allocs.push_back(c->ctr);
     c->allocs.push_back(c->done_ctr);
     if (hipHostMalloc((void**)&c->h_ctr, sizeof(DevCounters), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_done, sizeof(uint32_t) * kMaxPieces, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&c->h_done, sizeof(uint32_t) * kMaxPieces, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_rays, (size_t)kRaysHost * 44, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_full, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         g_err = "hipHostMalloc failed"; return bail(YN_ERR_HIP);
     }
     c->strm.pieces.resize(kMaxPieces);
@@ -1579,6 +1601,8 @@ void yn_destroy(yn_ctx* c)
     if (c->ovf_t) hipFree(c->ovf_t);
     if (c->h_ctr) hipHostFree(c->h_ctr);
     if (c->h_done) hipHostFree(c->h_done);
+    if (c->h_rays) hipHostFree(c->h_rays);
+    if (c->h_full) hipHostFree(c->h_full);
     for (int i = 0; i < kEvPool; ++i) if (c->ev[i]) hipEventDestroy(c->ev[i]);
     if (c->stream) hipStreamDestroy(c->stream);
     if (c->stream2) hipStreamDestroy(c->stream2);
@@ -2157,69 +2181,45 @@ int yn_trace(yn_ctx* c, int32_t sid, const float* rays, int32_t n, int32_t* tri,
     if (c->strm.active)
         if (int r = stream_drain(c)) return r;
     hipStream_t s = c->stream;
-    std::vector<int> idx[2];
-    for (int i = 0; i < n; ++i) idx[rays[8 * (size_t)i + 7] != 0.0f ? 1 : 0].push_back(i);
-    float* d_rays = nullptr;
-    int32_t* d_light = nullptr;
-    int r = dalloc(c, &d_rays, (size_t)n * 8);
-    if (r) return r;
-    r = dalloc(c, &d_light, (size_t)n);
-    if (r) { hipFree(d_rays); return r; }
-    std::vector<float> sub;
-    std::vector<float4> hits(n);
-    std::vector<int32_t> lights(n), occ(n);
     const SceneRec& S = c->scenes[sid];
-    for (int any = 0; any < 2; ++any) {
-        int m = (int)idx[any].size();
-        if (m == 0) continue;
-        sub.resize((size_t)m * 8);
-        for (int k = 0; k < m; ++k) std::memcpy(&sub[8 * (size_t)k], rays + 8 * (size_t)idx[any][k], 32);
-        HIPCK(c, hipMemcpyAsync(d_rays, sub.data(), sub.size() * 4, hipMemcpyHostToDevice, s));
-        HIPCK(c, hipMemsetAsync(c->ctr, 0, sizeof(DevCounters), s));
-        RayQueue q = c->E[0];
-        q.count = &c->ctr->q[0][0];
-        launch_prepare(c->d_scenes + sid, d_rays, m, q, d_light, s);
-        TraceArgs ta{};
-        ta.scenes = c->d_scenes;
-        ta.jobs = c->d_jobs;
-        ta.path_job = c->P.job;
-        ta.single_scene = sid;
-        ta.chunk = c->cfg.trace_chunk;
-        ta.ctr = c->ctr;
-        ta.q = q;
-        ta.hit_out = c->P.hit;
-        ta.occ_out = any ? c->P.occ : nullptr;
-        ta.work = &c->ctr->work[0][0][0];
-        ta.n_slices = c->cfg.trace_xcd;
-        ta.refill = c->cfg.trace_refill > 0 ? c->cfg.trace_refill : 0;
-        const int lds = lds_for(c, S.info.node_bytes);
-        int grid = c->cfg.trace_grid > 0 ? c->cfg.trace_grid
-                                         : c->n_cu * std::max(1, trace_resident_waves(lds) * 256 / c->cfg.trace_block);
-        if (int rr = ensure_overflow(c, S.info.max_depth - trace_lds_stack(lds), (int64_t)grid * c->cfg.trace_block))
-            return rr;
-        ta.ovf_ref = c->ovf_ref;
-        ta.ovf_t = c->ovf_t;
-        ta.ovf_depth = c->ovf_depth;
-        if (launch_trace(ta, any != 0, S.info.width, S.info.max_depth, c->cfg.trace_block, grid, false, lds, s) != 0)
-            return fail(c, YN_ERR_INVALID, "BVH too deep");
-        HIPCK(c, hipGetLastError());
-        HIPCK(c, hipMemcpyAsync(hits.data(), c->P.hit, (size_t)m * 16, hipMemcpyDeviceToHost, s));
-        HIPCK(c, hipMemcpyAsync(lights.data(), d_light, (size_t)m * 4, hipMemcpyDeviceToHost, s));
-        HIPCK(c, hipMemcpyAsync(c->h_ctr, c->ctr, kCtrHostBytes, hipMemcpyDeviceToHost, s));
-        HIPCK(c, hipStreamSynchronize(s));
-        if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
-        for (int k = 0; k < m; ++k) {
-            int i = idx[any][k];
-            int tr;
-            std::memcpy(&tr, &hits[k].y, 4);
-            tri[i] = tr;
-            t[i] = hits[k].x;
-            // a triangle nearer than the quad replaces the light hit (udpt.cl:386)
-            light[i] = tr >= 0 ? -1 : lights[k];
-        }
+    const int lds = lds_for(c, S.info.node_bytes);
+    const int grid = rays_grid(c, lds);
+    RaysArgs a = rays_args(c, sid, n);
+    // Up to kRaysHost rays the kernel reads and writes pinned host memory: a
+    // copy command each way costs more than the few hundred kB over the bus.
+    // Larger calls go through the samples buffer (64 B per path of capacity;
+    // a ray needs 44), which no frame in flight uses here.
+    const bool host = n <= kRaysHost;
+    float* io = host ? c->h_rays : reinterpret_cast<float*>(c->samples);
+    a.rays = io;
+    a.aligned = 1;
+    a.tri = reinterpret_cast<int32_t*>(io + 8 * (size_t)n);
+    a.light = a.tri + n;
+    a.t = reinterpret_cast<float*>(a.light + n);
+    if (int r = ensure_overflow(c, S.info.max_depth - rays_lds_stack(lds), (int64_t)grid * kRaysBlock)) return r;
+    a.ovf_ref = c->ovf_ref;
+    a.ovf_t = c->ovf_t;
+    a.ovf_depth = c->ovf_depth;
+    if (S.info.max_depth > rays_lds_stack(lds) + a.ovf_depth) return fail(c, YN_ERR_INVALID, "BVH too deep");
+    if (host) std::memcpy(io, rays, (size_t)n * 32);
+    else HIPCK(c, hipMemcpyAsync(io, rays, (size_t)n * 32, hipMemcpyHostToDevice, s));
+    if ((int64_t)n > (int64_t)(grid / a.n_slices) * a.n_slices * kRaysBlock)     // more rays than lanes
+        HIPCK(c, hipMemsetAsync(a.work, 0, sizeof(uint32_t) * kMaxXcd * kWorkStride, s));
+    *a.full = 0;
+    launch_rays(a, S.info.width, lds, grid, s);
+    HIPCK(c, hipGetLastError());
+    if (!host) {
+        HIPCK(c, hipMemcpyAsync(tri, a.tri, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+        HIPCK(c, hipMemcpyAsync(light, a.light, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+        HIPCK(c, hipMemcpyAsync(t, a.t, (size_t)n * 4, hipMemcpyDeviceToHost, s));
     }
-    hipFree(d_rays);
-    hipFree(d_light);
+    HIPCK(c, hipStreamSynchronize(s));
+    if (*a.full) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
+    if (host) {
+        std::memcpy(tri, a.tri, (size_t)n * 4);
+        std::memcpy(light, a.light, (size_t)n * 4);
+        std::memcpy(t, a.t, (size_t)n * 4);
+    }
     return 0;
 }
 
@@ -2234,26 +2234,22 @@ int yn_trace_noalloc(yn_ctx* c, int32_t sid, const float* rays, int32_t n, int32
     if (n == 0) return 0;
     const SceneRec& S = c->scenes[sid];
     hipStream_t s = c->stream;
-    TraceArgs ta{};
-    ta.scenes = c->d_scenes;
-    ta.jobs = c->d_jobs;
-    ta.path_job = c->P.job;
-    ta.single_scene = sid;
-    ta.chunk = c->cfg.trace_chunk;
-    ta.n_slices = c->cfg.trace_xcd;
-    ta.refill = c->cfg.trace_refill > 0 ? c->cfg.trace_refill : 0;
+    RaysArgs a = rays_args(c, sid, n);
+    a.rays = rays;
+    a.aligned = ((uintptr_t)rays & 15) == 0;
+    a.tri = tri;
+    a.light = light;
+    a.t = t;
     // the no-allocation entry keeps 16 LDS entries unless configured
-    const int na_lds = c->cfg.lds_stack > 0 ? c->cfg.lds_stack : 16;
-    if (trace_noalloc_enqueue(c->na_scratch, ta, c->d_scenes + sid, S.info.width, na_lds, c->cfg.trace_block,
-                              rays, n, tri, light, t, s) != 0)
+    const int lds = c->cfg.lds_stack > 0 ? c->cfg.lds_stack : 16;
+    *a.full = 0;
+    if (trace_noalloc_enqueue(c->na_scratch, a, S.info.width, lds, S.info.max_depth, rays_grid(c, lds), s) != 0)
         return fail(c, YN_ERR_INVALID, "trace launch refused");
     HIPCK(c, hipGetLastError());
-    HIPCK(c, hipMemcpyAsync(&c->h_ctr->q[7][0], &trace_noalloc_counters(c->na_scratch)->q[7][0], sizeof(uint32_t),
-                            hipMemcpyDeviceToHost, s));
     HIPCK(c, hipStreamSynchronize(s));
-    if (c->h_ctr->q[7][0])
+    if (*a.full)
         return fail(c, YN_ERR_INVALID, "traversal deeper than the no-allocation stack (" +
-                                           std::to_string(trace_lds_stack(na_lds) + kTraceNoAllocOvfDepth) +
+                                           std::to_string(rays_lds_stack(lds) + kTraceNoAllocOvfDepth) +
                                            " entries)");
     return 0;
 }

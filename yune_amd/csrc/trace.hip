@@ -29,6 +29,7 @@
 // lies beyond the best hit is dropped on pop without fetching it.  Waves pull
 // chunks of rays from the queue with one atomic per chunk.
 #include "yn_internal_dev.h"
+#include "yn_shade.h"
 #include "yn_trace.h"
 
 namespace yune {
@@ -41,6 +42,14 @@ namespace yune {
 // node-fetch latency; past 7 the register spills cost more than they hide.
 template <int LST>
 constexpr int trace_waves() { return LST <= 12 ? 7 : (LST == 16 ? 6 : 3); }
+
+// Result of one ray into the path's slot.
+template <bool ANY>
+__device__ __forceinline__ void store_hit(const TraceArgs& a, int pidx, const RayState& r, bool got)
+{
+    if (ANY) a.occ_out[pidx] = got ? 1 : 0;
+    else a.hit_out[pidx] = hit_record(r);
+}
 
 template <int W, bool ANY, int LST, int BLOCK, bool COUNT>
 __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace(TraceArgs a)
@@ -130,12 +139,7 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace(TraceArgs a
                 got = __ballot(!fma_ok) ? traverse<W, ANY, LST, BLOCK, COUNT, true>(S, r, st, c)
                                         : traverse<W, ANY, LST, BLOCK, COUNT, false>(S, r, st, c);
             ++nrays;
-            if (ANY) {
-                a.occ_out[pidx] = got ? 1 : 0;
-                if (a.hit_out) a.hit_out[pidx] = hit_record<ANY>(S.tri_isect, r);
-            } else {
-                a.hit_out[pidx] = hit_record<ANY>(S.tri_isect, r);
-            }
+            store_hit<ANY>(a, pidx, r, got);
         }
     }
     // one atomic per wave for the statistics
@@ -150,17 +154,12 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace(TraceArgs a
     }
 }
 
-// Result of one ray into the path's slot.
-template <bool ANY>
-__device__ __forceinline__ void store_hit(const TraceArgs& a, int pidx, const float4* __restrict__ tri,
-                                          const RayState& r, bool got)
+// Result of a caller's ray.
+__device__ __forceinline__ void store_ray(const RaysArgs& a, uint32_t i, const RayState& r, bool quad)
 {
-    if (ANY) {
-        a.occ_out[pidx] = got ? 1 : 0;
-        if (a.hit_out) a.hit_out[pidx] = hit_record<ANY>(tri, r);
-    } else {
-        a.hit_out[pidx] = hit_record<ANY>(tri, r);
-    }
+    a.tri[i] = r.tri;
+    a.light[i] = r.tri < 0 && quad ? 0 : -1;
+    a.t[i] = r.best;
 }
 
 // Traversal with lanes refilled.  k_trace runs each lane's ray to its end
@@ -264,39 +263,8 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
                     nodes = S.nodes;
                     tri = S.tri_isect;
                 }
-                // the tests ahead of the tree, as in traverse(): every slot
-                // without a BVH; the hoisted slots; a root that is one leaf
-                if (live && S.brute) {
-                    for (int s = 0; s < S.n_slots; ++s) {
-                        if (COUNT) c.tris++;
-                        got |= tri_test<ANY>(tri, s, r);
-                        if (ANY && got) break;
-                    }
-                    live = false;
-                }
-                if (live) {
-                    for (int s = 0; s < S.n_hoist; ++s) {
-                        float4 lo = gload(S.hoist_box + 2 * s), hi = gload(S.hoist_box + 2 * s + 1);
-                        float e;
-                        if (!box_hit(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, e) ||
-                            e > r.cull)
-                            continue;
-                        if (COUNT) c.tris++;
-                        got |= tri_test<ANY>(tri, s, r);
-                        if (ANY && got) break;
-                    }
-                    node = S.root_ref;
-                    if ((ANY && got) || node == kEmptyRef) {
-                        live = false;
-                    } else if (node & kLeafBit) {
-                        float e;
-                        if (box_hit(S.root_box[0], S.root_box[1], S.root_box[2], S.root_box[3], S.root_box[4],
-                                    S.root_box[5], r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, e))
-                            got |= leaf_test<ANY, COUNT>(tri, node, r, c);
-                        live = false;
-                    }
-                }
-                if (!live) store_hit<ANY>(a, pidx, tri, r, got);
+                if (live) live = trav_start<ANY, COUNT>(S, r, node, got, c);
+                if (!live) store_hit<ANY>(a, pidx, r, got);
             }
         }
         if (__ballot(live) == 0) {
@@ -307,7 +275,7 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
         if (live) {
             live = wexact ? trav_step<W, ANY, LST, BLOCK, COUNT, true>(nodes, tri, node, r, st, got, c)
                           : trav_step<W, ANY, LST, BLOCK, COUNT, false>(nodes, tri, node, r, st, got, c);
-            if (!live) store_hit<ANY>(a, pidx, tri, r, got);
+            if (!live) store_hit<ANY>(a, pidx, r, got);
         }
     }
     unsigned long long tot = wave_sum_u64(nrays);
@@ -317,6 +285,122 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
         if (lane == 0) {
             atomicAdd(ANY ? &a.ctr->nodes_shadow : &a.ctr->nodes_ext, tn);
             atomicAdd(ANY ? &a.ctr->tris_shadow : &a.ctr->tris_ext, tt);
+        }
+    }
+}
+
+// Rays of a caller, in yn_trace's layout: the quad test of traceRay
+// (udpt.cl:244-276) as the ray is taken, closest hit or any hit by the ray's
+// own flag, and the results written as yn_trace reports them (a triangle
+// nearer than the quad replaces the light hit, udpt.cl:386).  One launch for
+// all of it, where a queue fill, a launch for each kind of ray and a result
+// pass had their records in memory between them.  The loop is k_trace_rf's;
+// with no more rays than the grid has lanes each wave takes an equal share
+// of them and no counter is touched.
+// What bounds it: at a million rays the vector memory pipe, as k_trace_rf
+// (285 us for 1,000,003 rays over 123k triangles); at a few hundred the chain
+// of one ray's dependent fetches (48 us).  yn_trace of 1,000,003 host rays
+// 13.7 -> 2.24 ms (the rest is the bus: 32 MB in, 12 MB out), of 150,001
+// shadow rays 1.29 -> 0.43 ms, of 200 rays 104 -> 70 us; yn_trace_noalloc of
+// 200,003 rays 191 -> 111 us.
+template <int W, int LST>
+__global__ __launch_bounds__(kRaysBlock, trace_waves<LST>()) void k_rays(RaysArgs a)
+{
+    constexpr int BLOCK = kRaysBlock;
+    __shared__ uint32_t stk_all[LST * BLOCK];
+    __shared__ uint16_t stkt_all[LST * BLOCK];
+    Stack<LST, BLOCK> st;
+    st.lref = (lds_u32*)stk_all;
+    st.lt = (lds_u16*)stkt_all;
+    st.col = threadIdx.x;
+    st.gstride = gridDim.x * BLOCK;
+    st.gref = (gbl_u32*)a.ovf_ref;
+    st.gt = (gbl_u16*)a.ovf_t;
+    st.gbase = blockIdx.x * BLOCK;
+    st.gcap = a.ovf_depth;
+    st.full = a.full;
+    st.sp = 0;
+    const int lane = (int)__lane_id();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const uint32_t n = (uint32_t)a.n;
+    const DevScene& S = *a.scene;
+    const float4* nodes = S.nodes;
+    const float4* tri = S.tri_isect;
+    // slices of the rays, one per XCD, as in k_trace
+    const uint32_t ns = (uint32_t)a.n_slices, G = gridDim.x, wpb = BLOCK >> 6;
+    const uint32_t wx = (blockIdx.x / ns) * wpb + (threadIdx.x >> 6);
+    auto waves_of = [&](uint32_t y) { return ((G - y + ns - 1) / ns) * wpb; };
+    auto slice_lo = [&](uint32_t y) { return (uint32_t)(((uint64_t)y * n) / ns); };
+    auto sreg = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };   // wave-uniform
+    const uint32_t min_waves = (G / ns) * wpb;
+    const bool all_static = (uint64_t)n <= (uint64_t)ns * min_waves * 64u;
+    // rays of a wave's first fetch: its share of a slice (at most n / ns + 1 rays) when they all fit
+    const uint32_t per = all_static ? min(64u, (n / ns + min_waves) / min_waves) : 64u;
+    uint32_t y = blockIdx.x % ns, moved = 0;
+    uint32_t y_lo = sreg(slice_lo(y)), y_hi = sreg(slice_lo(y + 1)), y_waves = sreg(waves_of(y));
+    Counts c{0, 0};
+    RayState r{};
+    uint32_t node = 0, ray = 0;
+    bool live = false, got = false, exact = false, quad = false;
+    bool more = true, first = true;
+    for (;;) {
+        const unsigned long long idle = __ballot(!live);
+        const int n_idle = __popcll(idle);
+        if (more && (first || n_idle >= a.refill)) {
+            uint32_t base = 0, lim = 0;
+            for (;;) {
+                if (first) {
+                    base = y_lo + wx * per;          // every lane is idle on the first fetch
+                    first = false;
+                    if (base < y_hi) { lim = min(y_hi, base + per); break; }
+                } else {
+                    uint32_t b = 0;
+                    if (lane == 0) b = atomicAdd(a.work + y * kWorkStride, (uint32_t)n_idle);
+                    base = y_lo + y_waves * 64u + __shfl(b, 0);
+                    if (base < y_hi) { lim = y_hi; break; }
+                }
+                if (all_static || ++moved >= ns) { more = false; break; }
+                y = (y + 1) % ns;
+                y_lo = sreg(slice_lo(y));
+                y_hi = sreg(slice_lo(y + 1));
+                y_waves = sreg(waves_of(y));
+            }
+            if (all_static) more = false;
+            const uint32_t i = base + (uint32_t)__popcll(idle & below);
+            if (!live && i < lim) {
+                ray = i;
+                float4 ot, dp;
+                const float* q = a.rays + 8 * (size_t)i;
+                if (a.aligned) {
+                    ot = gload(reinterpret_cast<const float4*>(q));
+                    dp = gload(reinterpret_cast<const float4*>(q) + 1);
+                } else {
+                    ot = make_float4(q[0], q[1], q[2], q[3]);
+                    dp = make_float4(q[4], q[5], q[6], q[7]);
+                }
+                float t;
+                quad = quad_hit(S.light, mk(ot.x, ot.y, ot.z, 1.0f), mk(dp.x, dp.y, dp.z, 0.0f), ot.w, t);
+                if (quad) ot.w = t;
+                exact = !start_ray(r, ot, dp, S);
+                r.any = dp.w != 0.0f;
+                st.sp = 0;
+                got = false;
+                // a ray with a NaN component hits nothing (see k_trace)
+                live = ot.x == ot.x && ot.y == ot.y && ot.z == ot.z && ot.w == ot.w && dp.x == dp.x &&
+                       dp.y == dp.y && dp.z == dp.z;
+                if (live) live = trav_start<2, false>(S, r, node, got, c);
+                if (!live) store_ray(a, ray, r, quad);
+            }
+        }
+        if (__ballot(live) == 0) {
+            if (!more) break;
+            continue;
+        }
+        const bool wexact = __ballot(live && exact) != 0;
+        if (live) {
+            live = wexact ? trav_step<W, 2, LST, BLOCK, false, true>(nodes, tri, node, r, st, got, c)
+                          : trav_step<W, 2, LST, BLOCK, false, false>(nodes, tri, node, r, st, got, c);
+            if (!live) store_ray(a, ray, r, quad);
         }
     }
 }
@@ -376,6 +460,21 @@ int trace_resident_waves(int lds)
 {
     lds = trace_lds_stack(lds);
     return lds == 8 ? trace_waves<8>() : lds == 12 ? trace_waves<12>() : (lds == 32 ? trace_waves<32>() : trace_waves<16>());
+}
+
+// LDS part of a caller's rays' stack: 12 or 16 entries.
+int rays_lds_stack(int lds) { return lds > 0 && lds <= 12 ? 12 : 16; }
+
+void launch_rays(const RaysArgs& a, int width, int lds, int grid, hipStream_t s)
+{
+    const bool l12 = rays_lds_stack(lds) == 12;
+    if (width == 2) {
+        if (l12) hipLaunchKernelGGL((k_rays<2, 12>), dim3(grid), dim3(kRaysBlock), 0, s, a);
+        else hipLaunchKernelGGL((k_rays<2, 16>), dim3(grid), dim3(kRaysBlock), 0, s, a);
+    } else {
+        if (l12) hipLaunchKernelGGL((k_rays<4, 12>), dim3(grid), dim3(kRaysBlock), 0, s, a);
+        else hipLaunchKernelGGL((k_rays<4, 16>), dim3(grid), dim3(kRaysBlock), 0, s, a);
+    }
 }
 
 // `stack`: traversal stack entries the scene can need; the launch is refused

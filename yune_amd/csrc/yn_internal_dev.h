@@ -32,6 +32,26 @@ struct TraceArgs {
                                 //    to its queue position (unidirectional paths)
 };
 
+// A caller's rays in yn_trace's layout (k_rays): n x 8 floats in, three
+// arrays out, all addresses the device can reach.
+constexpr int kRaysBlock = 256;
+struct RaysArgs {
+    const DevScene* scene;
+    const float* rays;
+    int32_t n;
+    int32_t aligned;            // rays is 16-byte aligned
+    int32_t* tri;
+    int32_t* light;
+    float* t;
+    uint32_t* work;             // as in TraceArgs; used by launches of more rays than lanes
+    int32_t n_slices;
+    int32_t refill;             // idle lanes of a wave before it takes new rays (64: a whole wave)
+    uint32_t* ovf_ref;          // traversal stack overflow area, as in TraceArgs
+    uint16_t* ovf_t;
+    int32_t ovf_depth;
+    uint32_t* full;             // set to 1 by a traversal that would overflow the stack
+};
+
 // Segment of primary rays: a rectangle of one job's image at one frame.
 // Its work items are the rectangle's pixels in tile order (seg_pixel) from
 // item `first` on (0 unless a frame's pixels are issued in several parts).
@@ -284,19 +304,18 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred)
 }
 #endif
 
-// yn_trace_noalloc (trace_noalloc.hip): rays per call at most, threads of
-// its trace launches, and traversal stack entries its overflow area holds
-// beyond the LDS part.
+// yn_trace_noalloc (trace_noalloc.hip): rays per call at most, and traversal
+// stack entries per ray beyond the LDS part at most.
 constexpr int kTraceNoAllocMaxRays = YN_TRACE_NOALLOC_MAX_RAYS;
-constexpr int kTraceNoAllocGridThreads = 1 << 16;
 constexpr int kTraceNoAllocOvfDepth = 32;
 int trace_noalloc_init(int device, void** ptr);
-int trace_noalloc_enqueue(void* base, const TraceArgs& proto, const DevScene* scene, int width, int lds, int block,
-                          const float* rays, int n, int32_t* tri, int32_t* light, float* t, hipStream_t s);
-DevCounters* trace_noalloc_counters(void* base);
+int trace_noalloc_enqueue(void* base, const RaysArgs& rays, int width, int lds, int max_depth, int max_grid,
+                          hipStream_t s);
 
 int launch_trace(const TraceArgs& a, bool any_hit, int width, int stack, int block, int grid, bool count, int lds,
                  hipStream_t stream);
+void launch_rays(const RaysArgs& a, int width, int lds, int grid, hipStream_t stream);
+int rays_lds_stack(int lds);    // traversal stack entries k_rays keeps in LDS for a configured depth
 int trace_lds_stack(int lds);   // traversal stack entries kept in LDS for a configured depth
 int trace_resident_waves(int lds);   // waves per SIMD of a trace launch (the default grid fills them)
 void launch_generate(const GenArgs& a, const DevCapture& cap, hipStream_t stream);
@@ -308,7 +327,5 @@ void launch_shade_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int grid, 
 void launch_resolve(const ResolveArgs& a, hipStream_t stream);
 void launch_fmath(int op, const float* x, const float* y, int n, float* out, hipStream_t stream);
 void launch_tonemap(const float4* in, float4* out, int n, int op, hipStream_t stream);
-void launch_prepare(const DevScene* scene, const float* rays, int n, RayQueue q, int32_t* light_out,
-                    hipStream_t stream);
 
 }  // namespace yune

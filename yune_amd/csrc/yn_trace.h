@@ -17,8 +17,8 @@ struct RayState {
     float hx, hy, hz;       //   one way for the box's lo planes, the other for its hi planes
     float best;             // current tmax
     float cull;             // nodes entered beyond it are skipped: best * (1 + 1e-4) * kWiden
-    int tri;                // best hit: triangle id (-1: none), u, v; for any-hit rays
-    float u, v;             //   the slot, with id, u and v recomputed at the end if wanted
+    int tri;                // best hit: triangle id (-1: none), u, v
+    float u, v;
     bool any;               // ANY 2: this ray is done at its first hit
 };
 
@@ -110,11 +110,9 @@ __device__ __forceinline__ bool tri_test(const float4* __restrict__ tri, int s, 
     float t, u, v;
     int id;
     if (tri_uvt(tri, s, r, t, u, v, id) && t > 0.0f && t < r.best) {
-        r.best = t;
-        r.cull = cull_of(t);
-        if (ANY == 1) {
-            r.tri = s;
-        } else {
+        if (ANY != 1) {         // an any-hit ray ends here, and only whether it hit counts
+            r.best = t;
+            r.cull = cull_of(t);
             r.tri = id;
             r.u = u;
             r.v = v;
@@ -124,17 +122,11 @@ __device__ __forceinline__ bool tri_test(const float4* __restrict__ tri, int s, 
     return false;
 }
 
-// The result record {t, triangle id bits, u, v} of a finished traversal.
-// Any-hit rays kept the slot: its id, u and v come from the same test on
-// the same inputs as when it was found.
-template <int ANY>
-__device__ __forceinline__ float4 hit_record(const float4* __restrict__ tri, const RayState& r)
+// The result record {t, triangle id bits, u, v} of a finished closest-hit
+// traversal.
+__device__ __forceinline__ float4 hit_record(const RayState& r)
 {
-    if (ANY != 1 || r.tri < 0) return make_float4(r.best, __int_as_float(r.tri), r.u, r.v);
-    float t, u, v;
-    int id;
-    tri_uvt(tri, r.tri, r, t, u, v, id);
-    return make_float4(r.best, __int_as_float(id), u, v);
+    return make_float4(r.best, __int_as_float(r.tri), r.u, r.v);
 }
 
 struct Counts { unsigned nodes, tris; };
@@ -272,7 +264,7 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
                     uint32_t nearc = (uint32_t)C.x, farc = (uint32_t)C.y;
                     float fe = e1;
                     if (e1 < e0) { nearc = (uint32_t)C.y; farc = (uint32_t)C.x; fe = e0; }
-                    if (!st.push(farc, fe)) { atomicOr(st.full, 1u); return got; }   // cannot happen: depth bound
+                    if (!st.push(farc, fe)) { *st.full = 1u; return got; }   // cannot happen: depth bound
                     node = nearc;
                     continue;
                 } else if (h0) { node = (uint32_t)C.x; continue; }
@@ -310,7 +302,7 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
                     if (k3 != INFINITY) ok &= st.push(c3, k3);
                     if (k2 != INFINITY) ok &= st.push(c2, k2);
                     if (k1 != INFINITY) ok &= st.push(c1, k1);
-                    if (!ok) { atomicOr(st.full, 1u); return got; }   // cannot happen: depth bound
+                    if (!ok) { *st.full = 1u; return got; }   // cannot happen: depth bound
                     node = c0;
                     continue;
                 }
@@ -395,7 +387,7 @@ __device__ __forceinline__ bool trav_step(const float4* __restrict__ nodes, cons
                 uint32_t nearc = (uint32_t)C.x, farc = (uint32_t)C.y;
                 float fe = e1;
                 if (e1 < e0) { nearc = (uint32_t)C.y; farc = (uint32_t)C.x; fe = e0; }
-                if (!st.push(farc, fe)) { atomicOr(st.full, 1u); return false; }   // cannot happen: depth bound
+                if (!st.push(farc, fe)) { *st.full = 1u; return false; }   // cannot happen: depth bound
                 node = nearc;
                 if (!(node & kLeafBit)) return true;
             } else if (h0) { node = (uint32_t)C.x; if (!(node & kLeafBit)) return true; }
@@ -434,7 +426,7 @@ __device__ __forceinline__ bool trav_step(const float4* __restrict__ nodes, cons
                 if (k3 != INFINITY) ok &= st.push(c3, k3);
                 if (k2 != INFINITY) ok &= st.push(c2, k2);
                 if (k1 != INFINITY) ok &= st.push(c1, k1);
-                if (!ok) { atomicOr(st.full, 1u); return false; }   // cannot happen: depth bound
+                if (!ok) { *st.full = 1u; return false; }   // cannot happen: depth bound
                 node = c0;
                 if (!(node & kLeafBit)) return true;
             } else goto pop;
