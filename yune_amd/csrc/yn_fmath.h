@@ -43,8 +43,10 @@
  * it is used, by two scalar moves the compiler may not hoist: otherwise it
  * lifts every coefficient to the kernel's entry, and in the shade kernels,
  * which hold many live values, parks them in spill lanes and reads them
- * back around each use.  The bits are those of the literal either way. */
-#if defined(__HIP_DEVICE_COMPILE__)
+ * back around each use.  The bits are those of the literal either way.  A
+ * kernel that is little more than these functions defines
+ * YNF_PLAIN_CONSTANTS. */
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(YNF_PLAIN_CONSTANTS)
 template <unsigned long long B>
 __device__ static inline double ynf_kk()
 {
@@ -138,7 +140,7 @@ YN_FM float ynf_cosf(float xf)
 }
 
 /* natural log of a positive, finite, normal double */
-YN_FM double ynf_log(double x)
+YN_FM double ynf_log_split(double x, int* ex)     /* x = m 2^ex; returns m */
 {
     uint64_t b = ynf_bits(x);
     int e = (int)((b >> 52) & 0x7ff) - 1023;
@@ -147,7 +149,12 @@ YN_FM double ynf_log(double x)
         m = m * 0.5;
         e += 1;
     }
-    double s = (m - 1.0) / (m + 1.0);
+    *ex = e;
+    return m;
+}
+
+YN_FM double ynf_log_series(double s, int e)      /* s = (m - 1) / (m + 1) */
+{
     double z = s * s;
     double p = YNF_K(0.047619047619047616);              /* 1/21 */
     p = p * z + YNF_K(0.05263157894736842);              /* 1/19 */
@@ -163,6 +170,13 @@ YN_FM double ynf_log(double x)
     double lm = 2.0 * (s * p);
     double de = (double)e;
     return de * YNF_K(YNF_LN2_HI) + (lm + de * YNF_K(YNF_LN2_LO));
+}
+
+YN_FM double ynf_log(double x)
+{
+    int e;
+    const double m = ynf_log_split(x, &e);
+    return ynf_log_series((m - 1.0) / (m + 1.0), e);
 }
 
 /* e^z for |z| <= 110 */
@@ -186,7 +200,7 @@ YN_FM double ynf_exp(double z)
     p = p * r + 1.0;
     /* scale by 2^k: p in [0.7, 1.5] and |k| <= 160, so the result stays a
      * normal double and the exponent add is exact */
-    return ynf_from_bits(ynf_bits(p) + ((uint64_t)(int64_t)(long long)k << 52));
+    return ynf_from_bits(ynf_bits(p) + ((uint64_t)(uint32_t)(int32_t)k << 52));
 }
 
 /* powf with the C99 special cases (Annex F.9.4.4) */
