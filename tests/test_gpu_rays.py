@@ -77,3 +77,27 @@ def test_device_rays_at_any_alignment(brute):
             got = [o.cpu().numpy() for o in out]
             assert same([g[1:n + 1] for g in got], want), off
             assert all((g[0] == -7) and (g[n + 1:] == -7).all() for g in got)
+
+
+def test_traversal_beyond_the_fixed_stack_is_refused():
+    """yn_trace_noalloc's stack ends at 32 entries beyond the LDS part: a
+    deeper traversal is an error, and the next call works."""
+    torch = pytest.importorskip("torch")
+    from test_gpu_pt import comb_scene
+    deep, flat = comb_scene(60), Y.gen_cornell()
+    rays = np.zeros((64, 8), np.float32)
+    rays[:, 0] = np.linspace(-0.01, 0.01, 64)
+    rays[:, 3] = np.inf
+    rays[:, 6] = -1.0
+    d = torch.from_numpy(rays).cuda()
+    out = [torch.zeros(64, dtype=t, device="cuda") for t in (torch.int32, torch.int32, torch.float32)]
+    torch.cuda.synchronize()
+    with Y.Context(bvh_width=2, max_paths=1 << 12, hoist_frac=-1, leaf_max=10, bvh_build=2) as c:
+        a, b = c.scene(deep, deep.nodes), c.scene(flat)
+        assert c.scene_info(a).max_depth > 48
+        p = [C.c_void_p(o.data_ptr()) for o in out]
+        call = lambda sid: lib().yn_trace_noalloc(c._p, sid, C.c_void_p(d.data_ptr()), 64, *p)  # noqa: E731
+        assert (c.trace(a, rays)[0] == 0).all()         # its stack follows the scene
+        assert call(a) == -2
+        assert call(b) == 0
+        assert same([o.cpu().numpy() for o in out], c.trace(b, rays))

@@ -157,14 +157,13 @@ struct BRegResult {
     }
 };
 
-template <bool CAP, int LM, typename RES>
-__device__ __forceinline__ BOut advance_bdpt(const BdptShadeArgs& a, const DevCapture& cap, int p, int jid,
+template <bool CAP, int LM, typename TAB, typename RES>
+__device__ __forceinline__ BOut advance_bdpt(const BdptSoA& B, const TAB& tab, const DevCapture& cap, int p, int jid,
                                              const RES& res, BState& bs, const LdsScene& lds)
 {
-    const BdptSoA& B = a.B;
-    const DevJob& J = a.jobs[jid];
+    const DevJob& J = tab.job(jid);
     const yn_render_params& RP = J.p;
-    const DevScene& S = a.scenes[J.scene];
+    const DevScene& S = tab.scene(J.scene);
     // LM: materials and light in LDS, the launch's one scene's (1) or every scene's (2)
     auto mat_of = [&](int id) {
         return LM == 1 ? load_mat(lds.mats, id) : LM == 2 ? load_mat(lds.mats, S.mat_base + id) : load_mat(S.mats, id);
@@ -505,7 +504,7 @@ __global__ __launch_bounds__(256, 3) void k_shade_bdpt(BdptShadeArgs a, DevCaptu
             p = (int)a.list_in[i];
             const int jid = a.P.job[p];
             BState bs = load_state(a.B, p);
-            o = advance_bdpt<CAP, LM>(a, cap, p, jid, BQueueResult{a.P.hit, a.B.occ, (size_t)p << shift, p}, bs, lds);
+            o = advance_bdpt<CAP, LM>(a.B, JobTables{a.jobs, a.scenes}, cap, p, jid, BQueueResult{a.P.hit, a.B.occ, (size_t)p << shift, p}, bs, lds);
             store_state(a.B, p, bs);
         }
         const bool more = o.ext || o.emit != 0;
@@ -631,6 +630,18 @@ __global__ __launch_bounds__(256) void k_generate_bdpt(GenArgs a, DevCapture cap
     if (p == 0) { *a.ext_out.count = (uint32_t)a.n_paths; *a.list_count = (uint32_t)a.n_paths; }
 }
 
+template <bool ONE>
+__device__ __forceinline__ auto tables_of(const BdptPathsArgs& a)
+{
+    if constexpr (ONE) {        // an address opaque at each call, as in k_paths
+        auto* k = (const __attribute__((address_space(4))) BdptPathsArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+        __asm__ volatile("" : "+s"(k));
+        return OneJob{*(const DevJob*)&k->job, *(const DevScene*)&k->scene};
+    } else {
+        return JobTables{a.s.jobs, a.s.scenes};
+    }
+}
+
 // Idle lanes of a wave before k_paths_bdpt makes new paths: they start at the
 // first stage and the others wait for them (4.2M paths of the Cornell box, 5
 // vertices: 64, 13.5 ms; 56, 13.4; 48, 13.6; each lane at once, 20).
@@ -651,7 +662,8 @@ constexpr int kBdptRefill = 56;
 // 15k-triangle room 45.9 -> 33.8.  128 registers with 88 spilled, at 4 waves
 // per SIMD: 12.0 and 29.2 ms; 3 waves (39 spilled): 13.4 and 33.5; 2 waves
 // (none): 17.4 and 44.1; 5 waves (270): 15.4 and 31.0.
-template <int LM>
+// ONE: all paths of one job (LM 1).
+template <int LM, bool ONE>
 __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(BdptPathsArgs a)
 {
     constexpr int BL = kPathsBlock;
@@ -714,7 +726,8 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
         n_rays[0] += (unsigned)__popcll(__ballot(act && ext));
         n_rays[1] += (unsigned)__popcll(shadow);
         if (act && (ext || emit != 0)) {
-            const DevScene& S = s.scenes[LM == 1 ? s.lscene : s.jobs[jid].scene];
+            const auto tab = tables_of<ONE>(a);
+            const DevScene& S = tab.scene(LM == 1 ? s.lscene : tab.job(jid).scene);
             const int j = ext ? 0 : __ffsll((long long)emit) - 1;
             if (j > 0) {            // a connection ray, made exactly as when it was counted
                 const Vtx ev = load_v(s.B, 1, bs.i0.z, p), l = load_v(s.B, 0, j, p);
@@ -754,7 +767,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
         }
         // a step once every lane of the stage has all its rays' results
         if (__ballot(act && emit != 0) == 0 && act) {
-            const BOut o = advance_bdpt<false, LM>(s, cap, p, jid, BRegResult{res}, bs, lds);
+            const BOut o = advance_bdpt<false, LM>(s.B, tables_of<ONE>(a), cap, p, jid, BRegResult{res}, bs, lds);
             ot = o.o_t;
             dp = o.d_p;
             ext = o.ext;
@@ -783,9 +796,10 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
 void launch_paths_bdpt(const BdptPathsArgs& a, int grid, hipStream_t s)
 {
     const int lm = a.s.lmats != nullptr && a.s.n_lmats <= kLdsMats ? a.s.lmode : 0;
-    if (lm == 1) hipLaunchKernelGGL((k_paths_bdpt<1>), dim3(grid), dim3(kPathsBlock), 0, s, a);
-    else if (lm == 2) hipLaunchKernelGGL((k_paths_bdpt<2>), dim3(grid), dim3(kPathsBlock), 0, s, a);
-    else hipLaunchKernelGGL((k_paths_bdpt<0>), dim3(grid), dim3(kPathsBlock), 0, s, a);
+    if (lm == 1 && a.one) hipLaunchKernelGGL((k_paths_bdpt<1, true>), dim3(grid), dim3(kPathsBlock), 0, s, a);
+    else if (lm == 1) hipLaunchKernelGGL((k_paths_bdpt<1, false>), dim3(grid), dim3(kPathsBlock), 0, s, a);
+    else if (lm == 2) hipLaunchKernelGGL((k_paths_bdpt<2, false>), dim3(grid), dim3(kPathsBlock), 0, s, a);
+    else hipLaunchKernelGGL((k_paths_bdpt<0, false>), dim3(grid), dim3(kPathsBlock), 0, s, a);
 }
 
 void launch_generate_bdpt(const GenArgs& a, const DevCapture& cap, hipStream_t s)

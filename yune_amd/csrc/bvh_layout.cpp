@@ -741,6 +741,9 @@ int make_layout(const yn_triangle* tris, int n_tri, int n_mat, const yn_bvh_node
         if (n < 0) { err = "BVH is not a tree"; return -2; }
         if (f.depth * (width - 1) > L.max_depth) L.max_depth = f.depth * (width - 1);
         uint32_t refs[4] = {kEmptyRef, kEmptyRef, kEmptyRef, kEmptyRef};
+        if (width == 4)         // absent children: a box that the FMA slab form misses (yn_slab.h)
+            for (int k = n; k < 4; ++k)
+                for (int a = 0; a < 6; ++a) L.nodes[(size_t)f.gnode * fpn + 4 * a + k] = NAN;
         kids.clear();
         for (int k = 0; k < n; ++k) {
             int c = ch[k];

@@ -61,9 +61,25 @@ __device__ __forceinline__ void unpack(const Pend& q, const RayState& r, Rec& R)
     R.mis = mk(r.dx, r.dy, r.dz, q.e);
 }
 
+// (The arguments' address is opaque at each call: otherwise the compiler
+// loads every field before the loop and spills what the registers cannot
+// hold, instead of loading it again where it is used.)
+template <bool ONE>
+__device__ __forceinline__ auto tables_of(const PathsArgs& a)
+{
+    if constexpr (ONE) {
+        auto* k = (const __attribute__((address_space(4))) PathsArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+        __asm__ volatile("" : "+s"(k));
+        return OneJob{*(const DevJob*)&k->job, *(const DevScene*)&k->scene};
+    } else {
+        return JobTables{a.s.jobs, a.s.scenes};
+    }
+}
+
 }  // namespace
 
-template <int LM>
+// ONE: all paths of one job (LM 1).
+template <int LM, bool ONE>
 __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArgs a)
 {
     constexpr int BL = kPathsBlock;
@@ -126,7 +142,8 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
         n_rays[0] += (unsigned)__popcll(lm) - k;
         n_rays[1] += k;
         if (live) {
-            const DevScene& S = s.scenes[LM == 1 ? s.lscene : (R.m0.y >> SCENE_SHIFT) & 0xff];
+            const auto tab = tables_of<ONE>(a);
+            const DevScene& S = tab.scene(LM == 1 ? s.lscene : (R.m0.y >> SCENE_SHIFT) & 0xff);
             RayState r;
             const bool fma_ok = start_ray(r, ot, dp, S);
             r.any = any;
@@ -145,7 +162,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
             }
             unpack(q, r, R);
             const Out o = advance<false, LM>(
-                s, cap, RegResult{hit_record(r), got ? 1 : 0}, R, lds);
+                tab, cap, RegResult{hit_record(r), got ? 1 : 0}, R, lds);
             q = pack(R);
             ot = o.o_t;
             dp = o.d_p;
@@ -179,9 +196,10 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
 void launch_paths(const PathsArgs& a, int grid, hipStream_t stream)
 {
     const int lm = a.s.lmats != nullptr && a.s.n_lmats <= kLdsMats ? a.s.lmode : 0;
-    if (lm == 1) hipLaunchKernelGGL((k_paths<1>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
-    else if (lm == 2) hipLaunchKernelGGL((k_paths<2>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
-    else hipLaunchKernelGGL((k_paths<0>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
+    if (lm == 1 && a.one) hipLaunchKernelGGL((k_paths<1, true>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
+    else if (lm == 1) hipLaunchKernelGGL((k_paths<1, false>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
+    else if (lm == 2) hipLaunchKernelGGL((k_paths<2, false>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
+    else hipLaunchKernelGGL((k_paths<0, false>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
 }
 
 }  // namespace yune

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(shade_block_pt(WAVES), WAVES) void k_shade_pt(Shade
             const bool ext = i < n_ext;
             const uint32_t qi = ext ? i : i - n_ext;
             load_rec(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), R, ext, ext && a.ext_primary);
-            o = advance<CAP, LM>(a, cap, QueueResult{a.hit, a.occ, qi}, R, lds);
+            o = advance<CAP, LM>(JobTables{a.jobs, a.scenes}, cap, QueueResult{a.hit, a.occ, qi}, R, lds);
         }
         const uint32_t n[2] = {o.kind == 1 ? 1u : 0u, o.kind == 2 ? 1u : 0u};
         uint32_t at[2];

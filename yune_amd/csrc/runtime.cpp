@@ -55,6 +55,7 @@ struct JobRec {
     yn_cam cam{};
     int32_t W = 0, H = 0;
     yn_render_params p{};
+    DevJob dev{};                 // its entry in the device's job table, as last uploaded
     std::mt19937 engine;
     uint64_t frame = 0;
     float4* accum = nullptr;
@@ -372,6 +373,7 @@ void add_spans(const std::vector<Span>& spans, yn_stats& st)
 struct LoopCfg {
     bool bdpt = false;
     int single = -1;                  // >= 0: every path renders this scene
+    int job = -1;                     // >= 0: every path belongs to this job
     int lds = 16;                     // LDS stack entries of the trace launches (lds_for)
     int width = 2, max_depth = 0;
     int block = 256, grid = 1, shade_grid = 1;
@@ -619,6 +621,17 @@ constexpr int64_t kPathsDirectBdpt = (int64_t)1 << 21;
 // What whole-path launches need: width-4 trees, nothing counted or captured.
 bool paths_fit(const LoopCfg& L, bool capture) { return !L.count && L.width == 4 && !capture; }
 
+// The launch's one job and scene as kernel arguments, when it has one and the
+// scene's materials fit LDS.
+template <typename A>
+void one_job(const yn_ctx* c, const LoopCfg& L, A& a)
+{
+    if (L.job < 0 || L.single < 0 || a.s.lmode != 1) return;
+    a.one = 1;
+    a.job = c->jobs[L.job].dev;
+    a.scene = c->scenes[L.single].dev;
+}
+
 // Enqueues k_paths on the rays of the queues that A's shade reads: their
 // paths run to their ends in one launch.  The counters follow to the host.
 int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
@@ -628,6 +641,7 @@ int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
     pa.s.ext_primary = primary ? 1 : 0;
     pa.next = &c->ctr->work[0][0][0];
     pa.endless = &c->ctr->q[6][0];
+    one_job(c, L, pa);
     // the blocks that fit at once
     const int grid = c->n_cu * paths_waves(pa.s.lmode);
     if (int r = ensure_overflow(c, L.max_depth - kPathsLds, (int64_t)grid * kPathsBlock)) return r;
@@ -649,6 +663,7 @@ int enqueue_paths_bdpt(yn_ctx* c, const LoopCfg& L, const IterArgs& A, const Gen
     pa.g = g;
     pa.next = &c->ctr->work[0][0][0];
     pa.ctr = c->ctr;
+    one_job(c, L, pa);
     const int grid = c->n_cu * paths_waves(pa.s.lmode);
     if (int r = ensure_overflow(c, L.max_depth - kPathsLds, (int64_t)grid * kPathsBlock)) return r;
     if (L.max_depth > kPathsLds + c->ovf_depth) return fail(c, YN_ERR_INVALID, "BVH too deep for the traversal stack");
@@ -739,6 +754,9 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     for (const Region& r : regs) scene_ids.push_back(c->jobs[r.job].scene);
     LoopCfg L;
     if (int r = loop_cfg(c, bdpt, scene_ids, stat_job.counting != 0, L)) return r;
+    L.job = regs[0].job;
+    for (const Region& r : regs)
+        if (r.job != L.job) L.job = -1;
     std::vector<Span> spans;
     IterArgs iters[2];
     make_iter(c, L, 0, iters[0]);
@@ -822,7 +840,8 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
 
 int upload_job_table(yn_ctx* c, int jid, float4* samples)
 {
-    DevJob d = make_devjob(c->jobs[jid]);
+    DevJob& d = c->jobs[jid].dev;
+    d = make_devjob(c->jobs[jid]);
     d.samples = samples;
     HIPCK(c, hipMemcpyAsync(c->d_jobs + jid, &d, sizeof(DevJob), hipMemcpyHostToDevice, c->stream));
     return 0;

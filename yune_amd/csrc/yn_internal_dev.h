@@ -109,11 +109,31 @@ struct ShadeArgs {
                                 //    first iteration), whose record holds only m0, m1, rd
 };
 
+// Where a shade step finds a path's job and scene: the device tables, or, in
+// a launch whose paths all belong to one job, its kernel arguments (scalar
+// loads that do not wait for the path's record, instead of per-lane loads
+// that do).
+struct JobTables {
+    const DevJob* jobs;
+    const DevScene* scenes;
+    __device__ __forceinline__ const DevJob& job(int j) const { return jobs[j]; }
+    __device__ __forceinline__ const DevScene& scene(int i) const { return scenes[i]; }
+};
+struct OneJob {
+    const DevJob& j;
+    const DevScene& s;
+    __device__ __forceinline__ const DevJob& job(int) const { return j; }
+    __device__ __forceinline__ const DevScene& scene(int) const { return s; }
+};
+
 // Whole paths in one launch (paths.hip): the paths of the shade arguments'
 // input queues, each from its queued ray to its end.
 struct PathsArgs {
     ShadeArgs s;
     uint32_t* next;             // paths taken beyond the static ones, zero at launch
+    int32_t one;                // 1: every path belongs to `job`, in `scene` (then s.lmode is 1)
+    DevJob job;
+    DevScene scene;
     uint32_t* endless;          // set to 1 by a path of kMaxPathBounces bounces (it is given up), zero at launch
     uint32_t* ovf_ref;          // traversal stack overflow area, as in TraceArgs
     uint16_t* ovf_t;
@@ -186,6 +206,9 @@ struct BdptPathsArgs {
     BdptShadeArgs s;
     GenArgs g;
     uint32_t* next;             // as in PathsArgs
+    int32_t one;
+    DevJob job;
+    DevScene scene;
     uint32_t* ovf_ref;
     uint16_t* ovf_t;
     int32_t ovf_depth;

@@ -134,16 +134,17 @@ struct QueueResult {
 // a camera ray starts at the camera's eye (createRay, udpt.cl:236) along the
 // stored direction rd; a bounce ray at hp + nd * EPSILON along the pending
 // bounce direction nd (udpt.cl:766, 906, 945).
-template <bool CAP, int LM, typename RES>
-__device__ __forceinline__ Out advance(const ShadeArgs& a, const DevCapture& cap, const RES& res, Rec& R,
+// `tab`: where the path's job and scene are found (JobTables or OneJob).
+template <bool CAP, int LM, typename TAB, typename RES>
+__device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, const RES& res, Rec& R,
                                        const LdsScene& lds)
 {
     const int4 m0 = R.m0, m1 = R.m1;
     const int jid = m1.y;
-    const DevJob& J = a.jobs[jid];
+    const DevJob& J = tab.job(jid);
     const yn_render_params& RP = J.p;
     const int sid = (m0.y >> SCENE_SHIFT) & 0xff;
-    const DevScene& S = a.scenes[sid];                                 // loaded beside J, not after it
+    const DevScene& S = tab.scene(sid);                                // loaded beside J, not after it
     // LM: materials and light in LDS, the launch's one scene's (1) or every scene's (2)
     auto mat_of = [&](int id) {
         return LM == 1 ? load_mat(lds.mats, id) : LM == 2 ? load_mat(lds.mats, S.mat_base + id) : load_mat(S.mats, id);

@@ -6,6 +6,7 @@
 #pragma once
 
 #include "yn_device.h"
+#include "yn_exact.h"
 #include "yn_internal.h"
 #include "yn_slab.h"
 
@@ -46,7 +47,7 @@ __device__ __forceinline__ bool start_ray(RayState& r, const float4& ot, const f
 {
     r.ox = ot.x; r.oy = ot.y; r.oz = ot.z;
     r.dx = dp.x; r.dy = dp.y; r.dz = dp.z;
-    r.ix = 1 / r.dx; r.iy = 1 / r.dy; r.iz = 1 / r.dz;   // dir_inv (udpt.cl:395)
+    r.ix = x_rcp(r.dx); r.iy = x_rcp(r.dy); r.iz = x_rcp(r.dz);   // dir_inv (udpt.cl:395)
     fma_offsets(r.ox, r.ix, r.lx, r.hx);
     fma_offsets(r.oy, r.iy, r.ly, r.hy);
     fma_offsets(r.oz, r.iz, r.lz, r.hz);
@@ -90,7 +91,7 @@ __device__ __forceinline__ bool tri_uvt(const float4* __restrict__ tri, int s, c
     float py = r.dz * C.x - r.dx * C.z;
     float pz = r.dx * C.y - r.dy * C.x;
     float det = B.x * px + B.y * py + B.z * pz;
-    float inv_det = 1.0f / det;
+    float inv_det = x_rcp(det);
     float sx = r.ox - A.x, sy = r.oy - A.y, sz = r.oz - A.z;
     u = (px * sx + py * sy + pz * sz) * inv_det;
     if (u < 0.0f || u > 1.0f) return false;
@@ -134,14 +135,15 @@ struct Counts { unsigned nodes, tris; };
 template <int ANY, bool COUNT>
 __device__ __forceinline__ bool leaf_test(const float4* __restrict__ tri, uint32_t ref, RayState& r, Counts& c)
 {
-    int first = (int)((ref >> 4) & 0x7FFFFFFu);
-    int cnt = (int)(ref & 15u);
+    int s = (int)((ref >> 4) & 0x7FFFFFFu);
+    int left = (int)(ref & 15u);
     bool got = false;
-    for (int k = 0; k < cnt; ++k) {
+    do {                    // a leaf holds at least one triangle (kEmptyRef is never entered)
         if (COUNT) c.tris++;
-        got |= tri_test<ANY>(tri, first + k, r);
+        got |= tri_test<ANY>(tri, s, r);
         if (ends<ANY>(r, got)) return true;
-    }
+        ++s;
+    } while (--left > 0);
     return got;
 }
 
@@ -178,29 +180,55 @@ struct Stack {
         return c;
     }
 
-    __device__ __forceinline__ bool push(uint32_t ref, float t)
+    __device__ __forceinline__ void put(uint32_t ref, float t)
     {
-        uint16_t tb = (uint16_t)(__float_as_uint(t) >> 16);   // truncation: a lower bound of t >= 0
+        const uint32_t i = sp * BLOCK + column();
+        lref[i] = ref;
+        lt[i] = (uint16_t)(__float_as_uint(t) >> 16);   // truncation: a lower bound of t >= 0
+    }
+
+    // An entry anywhere.  One that the overflow area has no room for is left
+    // out and raises the flag: the caller's results are then refused.
+    __device__ __forceinline__ void push(uint32_t ref, float t)
+    {
         if (sp < LST) {
-            const uint32_t i = sp * BLOCK + column();
-            lref[i] = ref;
-            lt[i] = tb;
+            put(ref, t);
         } else {
             int k = sp - LST;
-            if (k >= gcap) return false;
+            if (k >= gcap) { *full = 1u; return; }      // cannot happen: depth bound
             const size_t i = (size_t)k * gstride + gbase + column();
             gref[i] = ref;
-            gt[i] = tb;
+            gt[i] = (uint16_t)(__float_as_uint(t) >> 16);
         }
         ++sp;
-        return true;
     }
+
+    // The farther children of a node, k1 <= k2 <= k3 with +inf where there is
+    // none, the nearest on top.  While every lane of the wave has room for
+    // three in LDS, each is written whether there or not and the next goes
+    // over it, without a branch for each.
+    __device__ __forceinline__ void push3(float k1, uint32_t c1, float k2, uint32_t c2, float k3, uint32_t c3)
+    {
+        if (__builtin_expect(__ballot(sp > LST - 3) == 0, 1)) {
+            put(c3, k3);
+            sp += k3 != INFINITY ? 1 : 0;
+            put(c2, k2);
+            sp += k2 != INFINITY ? 1 : 0;
+            put(c1, k1);
+            sp += k1 != INFINITY ? 1 : 0;
+        } else {
+            if (k3 != INFINITY) push(c3, k3);
+            if (k2 != INFINITY) push(c2, k2);
+            if (k1 != INFINITY) push(c1, k1);
+        }
+    }
+
     __device__ __forceinline__ uint32_t pop(float& t)
     {
         --sp;
         uint32_t ref;
         uint16_t tb;
-        if (sp < LST) {
+        if (__builtin_expect(__ballot(sp >= LST) == 0, 1) || sp < LST) {
             const uint32_t i = sp * BLOCK + column();
             ref = lref[i];
             tb = lt[i];
@@ -264,7 +292,7 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
                     uint32_t nearc = (uint32_t)C.x, farc = (uint32_t)C.y;
                     float fe = e1;
                     if (e1 < e0) { nearc = (uint32_t)C.y; farc = (uint32_t)C.x; fe = e0; }
-                    if (!st.push(farc, fe)) { *st.full = 1u; return got; }   // cannot happen: depth bound
+                    st.push(farc, fe);
                     node = nearc;
                     continue;
                 } else if (h0) { node = (uint32_t)C.x; continue; }
@@ -279,11 +307,12 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
                 bool h2 = child_hit<EXACT>(LX.z, LY.z, LZ.z, HX.z, HY.z, HZ.z, r, k2);
                 bool h3 = child_hit<EXACT>(LX.w, LY.w, LZ.w, HX.w, HY.w, HZ.w, r, k3);
                 uint32_t c0 = (uint32_t)C.x, c1 = (uint32_t)C.y, c2 = (uint32_t)C.z, c3 = (uint32_t)C.w;
-                // missed, culled or absent children sort last (key +inf)
-                k0 = (h0 && k0 <= r.cull && c0 != kEmptyRef) ? k0 : INFINITY;
-                k1 = (h1 && k1 <= r.cull && c1 != kEmptyRef) ? k1 : INFINITY;
-                k2 = (h2 && k2 <= r.cull && c2 != kEmptyRef) ? k2 : INFINITY;
-                k3 = (h3 && k3 <= r.cull && c3 != kEmptyRef) ? k3 : INFINITY;
+                // missed, culled or absent children sort last (key +inf); the
+                // FMA form misses the NaN box of an absent child
+                k0 = (h0 && k0 <= r.cull && (!EXACT || c0 != kEmptyRef)) ? k0 : INFINITY;
+                k1 = (h1 && k1 <= r.cull && (!EXACT || c1 != kEmptyRef)) ? k1 : INFINITY;
+                k2 = (h2 && k2 <= r.cull && (!EXACT || c2 != kEmptyRef)) ? k2 : INFINITY;
+                k3 = (h3 && k3 <= r.cull && (!EXACT || c3 != kEmptyRef)) ? k3 : INFINITY;
                 // 4-input sorting network, ascending entry distance
 #define YN_CS(ka, ca, kb, cb)                                              \
     {                                                                      \
@@ -298,11 +327,7 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
                 YN_CS(k1, c1, k2, c2);
 #undef YN_CS
                 if (k0 != INFINITY) {
-                    bool ok = true;
-                    if (k3 != INFINITY) ok &= st.push(c3, k3);
-                    if (k2 != INFINITY) ok &= st.push(c2, k2);
-                    if (k1 != INFINITY) ok &= st.push(c1, k1);
-                    if (!ok) { *st.full = 1u; return got; }   // cannot happen: depth bound
+                    st.push3(k1, c1, k2, c2, k3, c3);
                     node = c0;
                     continue;
                 }
@@ -387,7 +412,7 @@ __device__ __forceinline__ bool trav_step(const float4* __restrict__ nodes, cons
                 uint32_t nearc = (uint32_t)C.x, farc = (uint32_t)C.y;
                 float fe = e1;
                 if (e1 < e0) { nearc = (uint32_t)C.y; farc = (uint32_t)C.x; fe = e0; }
-                if (!st.push(farc, fe)) { *st.full = 1u; return false; }   // cannot happen: depth bound
+                st.push(farc, fe);
                 node = nearc;
                 if (!(node & kLeafBit)) return true;
             } else if (h0) { node = (uint32_t)C.x; if (!(node & kLeafBit)) return true; }
@@ -402,12 +427,16 @@ __device__ __forceinline__ bool trav_step(const float4* __restrict__ nodes, cons
             bool h1 = child_hit<EXACT>(LX.y, LY.y, LZ.y, HX.y, HY.y, HZ.y, r, k1);
             bool h2 = child_hit<EXACT>(LX.z, LY.z, LZ.z, HX.z, HY.z, HZ.z, r, k2);
             bool h3 = child_hit<EXACT>(LX.w, LY.w, LZ.w, HX.w, HY.w, HZ.w, r, k3);
+            // loaded with the boxes: sunk below the tests (where it is used) it
+            // would be one more trip to memory in every step's chain
+            __asm__ volatile("" : "+v"(C.x), "+v"(C.y), "+v"(C.z), "+v"(C.w));
             uint32_t c0 = (uint32_t)C.x, c1 = (uint32_t)C.y, c2 = (uint32_t)C.z, c3 = (uint32_t)C.w;
-            // missed, culled or absent children sort last (key +inf)
-            k0 = (h0 && k0 <= r.cull && c0 != kEmptyRef) ? k0 : INFINITY;
-            k1 = (h1 && k1 <= r.cull && c1 != kEmptyRef) ? k1 : INFINITY;
-            k2 = (h2 && k2 <= r.cull && c2 != kEmptyRef) ? k2 : INFINITY;
-            k3 = (h3 && k3 <= r.cull && c3 != kEmptyRef) ? k3 : INFINITY;
+            // missed, culled or absent children sort last (key +inf); the
+                // FMA form misses the NaN box of an absent child
+            k0 = (h0 && k0 <= r.cull && (!EXACT || c0 != kEmptyRef)) ? k0 : INFINITY;
+            k1 = (h1 && k1 <= r.cull && (!EXACT || c1 != kEmptyRef)) ? k1 : INFINITY;
+            k2 = (h2 && k2 <= r.cull && (!EXACT || c2 != kEmptyRef)) ? k2 : INFINITY;
+            k3 = (h3 && k3 <= r.cull && (!EXACT || c3 != kEmptyRef)) ? k3 : INFINITY;
             // 4-input sorting network, ascending entry distance
 #define YN_CS(ka, ca, kb, cb)                                              \
 {                                                                      \
@@ -422,11 +451,7 @@ __device__ __forceinline__ bool trav_step(const float4* __restrict__ nodes, cons
             YN_CS(k1, c1, k2, c2);
 #undef YN_CS
             if (k0 != INFINITY) {
-                bool ok = true;
-                if (k3 != INFINITY) ok &= st.push(c3, k3);
-                if (k2 != INFINITY) ok &= st.push(c2, k2);
-                if (k1 != INFINITY) ok &= st.push(c1, k1);
-                if (!ok) { *st.full = 1u; return false; }   // cannot happen: depth bound
+                st.push3(k1, c1, k2, c2, k3, c3);
                 node = c0;
                 if (!(node & kLeafBit)) return true;
             } else goto pop;
