@@ -376,6 +376,7 @@ struct LoopCfg {
     int job = -1;                     // >= 0: every path belongs to this job
     int lds = 16;                     // LDS stack entries of the trace launches (lds_for)
     int width = 2, max_depth = 0;
+    size_t node_bytes = 0;            // of the largest scene's tree
     int block = 256, grid = 1, shade_grid = 1;
     bool overlap = false, count = false;
     uint32_t* done_ctr = nullptr;     // continuous serving: ended paths per piece (entry - kMaxJobs)
@@ -408,14 +409,13 @@ int loop_cfg(yn_ctx* c, bool bdpt, const std::vector<int>& scene_ids, bool count
     bool same = !scene_ids.empty();
     for (int sc : scene_ids) same &= sc == scene_ids[0];
     if (same) L.single = scene_ids[0];
-    size_t node_bytes = 0;
     for (int sc : scene_ids) {
         const SceneRec& sr = c->scenes[sc];
         L.max_depth = std::max(L.max_depth, sr.info.max_depth);
         L.width = sr.info.width;      // all scenes of a context share the width
-        node_bytes = std::max(node_bytes, sr.info.node_bytes);
+        L.node_bytes = std::max(L.node_bytes, sr.info.node_bytes);
     }
-    L.lds = lds_for(c, node_bytes);
+    L.lds = lds_for(c, L.node_bytes);
     L.block = c->cfg.trace_block;
     // default: the trace blocks that fit at once (4 SIMDs per CU)
     L.grid = c->cfg.trace_grid > 0 ? c->cfg.trace_grid
@@ -597,26 +597,32 @@ int ensure_group_graph(yn_ctx* c, const LoopCfg& L, const IterArgs (&iters)[2], 
 
 // Batches of at most kPathsDirect paths run in k_paths from their camera rays
 // on (enqueue_paths), larger ones in the wavefront, which k_paths finishes
-// once at most kPathsTail rays are queued.  Time of a batch, wavefront against
-// k_paths (depth 8, NEE + MIS):
-//                  262,144 paths     4.2M paths        16.8M paths
-//   Cornell box    2.06 / 0.51 ms    6.00 / 3.79 ms    14.5 / 14.3 ms
-//   245k triangles 5.24 / 1.27 ms    9.44 / 6.80 ms    22.3 / 24.8 ms
-//   1M triangles   6.02 / 1.38 ms    10.8 / 7.5 ms     24.7 / 27.3 ms
-// Without a bounce limit k_paths leads at 16.8M as well (64 / 39 ms at 1M
-// triangles): the wavefront then runs many iterations over few rays, which
-// the tail rule takes from it (256 frames of the Cornell box, 16.8M paths:
-// 15.4 -> 14.2 ms with the tail at 4M rays; 14.5-14.8 at 0.26-1M).
-constexpr int64_t kPathsDirect = (int64_t)1 << 23;
-constexpr int64_t kPathsTail = (int64_t)1 << 22;
-// Bidirectional batches in k_paths_bdpt from the start, else in the wavefront
-// to the end (5 vertices, wavefront against k_paths_bdpt):
-//                  262,144 paths     1M paths          4.2M paths
-//   Cornell box    2.36 / 1.13 ms    5.70 / 3.35 ms    14.6 / 12.1 ms
-//   15k triangles  4.20 / 2.16 ms    9.02 / 7.82 ms    29.5 / 29.3 ms
-// and with 20 vertices at 15k triangles 38.2 / 36.4 ms at 1M paths, 124 /
-// 134 ms at 4.2M.
-constexpr int64_t kPathsDirectBdpt = (int64_t)1 << 21;
+// once at most kPathsTail rays are queued.  Time of a batch, such a wavefront
+// against k_paths alone (depth 8, NEE + MIS):
+//                  2.1M paths        4.2M paths        8.4M paths
+//   Cornell box    2.60 / 2.08 ms    4.17 / 3.95 ms    7.14 / 7.68 ms
+//   245k triangles 3.80 / 3.56 ms    6.16 / 6.39 ms    10.7 / 12.0 ms
+//   1M triangles   4.21 / 3.89 ms    6.74 / 6.93 ms    11.7 / 13.1 ms
+// and below 1M paths the wavefront's launches cost two to six times k_paths.
+// The tail at 8M rays instead of 4M: 256 frames of the Cornell box (16.8M
+// paths) 13.98 -> 13.66 ms, a 1M-triangle room within 1%.
+constexpr int64_t kPathsDirect = (int64_t)1 << 22;
+constexpr int64_t kPathsTail = (int64_t)1 << 23;
+
+// Bidirectional batches run in k_paths_bdpt from the start or in the
+// wavefront to the end.  Wavefront against k_paths_bdpt:
+//                                1M paths          4.2M paths        8.4M paths
+//   Cornell box, 5 vertices      5.55 / 3.10 ms    14.0 / 11.0 ms    25.7 / 21.6 ms
+//   Cornell box, 20 vertices     12.7 / 6.66 ms    35.7 / 24.9 ms    64.8 / 48.5 ms
+//   15k triangles, 5 vertices    8.77 / 7.25 ms    28.7 / 27.4 ms    55.1 / 53.7 ms
+//   15k triangles, 20 vertices   37.6 / 34.1 ms    122 / 126 ms      231 / 246 ms
+// Long subpaths over trees larger than an L1 cache go to the wavefront above
+// 1M paths: their lanes wait for each other's walks.
+constexpr int64_t kPathsDirectBdptLong = (int64_t)1 << 20;
+bool bdpt_paths_win(int64_t paths, int vertices, size_t node_bytes)
+{
+    return paths <= kPathsDirectBdptLong || vertices <= 8 || node_bytes <= ((size_t)32 << 10);
+}
 
 // What whole-path launches need: width-4 trees, nothing counted or captured.
 bool paths_fit(const LoopCfg& L, bool capture) { return !L.count && L.width == 4 && !capture; }
@@ -767,7 +773,9 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
         ga.B = c->B;
         ga.list_out = c->lst[0];
         ga.list_count = q(8);
-        if (paths_ok && total <= kPathsDirectBdpt) return enqueue_paths_bdpt(c, L, iters[0], ga);
+        int vertices = 0;
+        for (const Region& r : regs) vertices = std::max(vertices, (int)c->jobs[r.job].p.bdpt_bounces);
+        if (paths_ok && bdpt_paths_win(total, vertices, L.node_bytes)) return enqueue_paths_bdpt(c, L, iters[0], ga);
         launch_generate_bdpt(ga, cap, s);
     } else {
         launch_generate(ga, cap, s);
