@@ -1,15 +1,14 @@
-// yn_exact.h — correctly rounded reciprocal and square root on the device,
-// in fewer instructions than the compiler's.
+// yn_exact.h — the correctly rounded reciprocal on the device, in fewer
+// instructions than the compiler's division.
 //
-// 1 / x and sqrt(x) must round as IEEE says, since the CPU oracle's do.  The
-// compiler's sequences (division: 11 instructions and the waits its flag
-// register asks for; square root: 16) also cover denormals, infinities and
-// zeros.  Here an argument whose exponent keeps every intermediate normal
-// takes the hardware's approximation and Newton's steps in FMAs (Markstein,
-// IBM J. R&D 34, 1990), any other the compiler's sequence; a wave without
-// such a lane skips it.  Compared with the compiler's results for all 2^32
-// arguments on gfx950: equal for exponent fields 1..252 (x_rcp, either sign)
-// and 25..254 (x_sqrt, positive), the ranges tested below.
+// 1 / x must round as IEEE says, since the oracle's does.  The compiler's
+// division (11 instructions and the waits its flag register asks for) also
+// covers denormals, infinities and zeros.  Here an argument whose exponent
+// keeps every intermediate normal takes the hardware's approximation and one
+// of Newton's steps in FMAs (Markstein, IBM J. R&D 34, 1990), any other the
+// division; a wave without such a lane skips it.  Compared with the division
+// for all 2^32 arguments on gfx950: equal for exponent fields 1..252 of
+// either sign, the range tested below.
 #pragma once
 
 #include <math.h>
@@ -27,35 +26,6 @@ __device__ __forceinline__ float x_rcp(float x)
         r = fmaf(fmaf(-x, r, 1.0f), r, r);
     } else {
         r = 1.0f / x;
-    }
-    return r;
-}
-
-__device__ __forceinline__ float x_sqrt(float x)
-{
-    float s;
-    if (__builtin_expect(__float_as_uint(x) - (25u << 23) < (230u << 23), 1)) {
-        const float y = __builtin_amdgcn_rsqf(x);
-        s = x * y;
-        s = fmaf(fmaf(-s, s, x), 0.5f * y, s);
-    } else {
-        s = sqrtf(x);
-    }
-    return s;
-}
-
-// 1 / sqrt(x), both rounded.
-__device__ __forceinline__ float x_rcp_sqrt(float x)
-{
-    float r;
-    if (__builtin_expect(__float_as_uint(x) - (25u << 23) < (230u << 23), 1)) {
-        const float y = __builtin_amdgcn_rsqf(x);
-        float s = x * y;
-        s = fmaf(fmaf(-s, s, x), 0.5f * y, s);      // exponent field 76..190
-        r = __builtin_amdgcn_rcpf(s);
-        r = fmaf(fmaf(-s, r, 1.0f), r, r);
-    } else {
-        r = 1.0f / sqrtf(x);
     }
     return r;
 }
