@@ -88,3 +88,25 @@ def test_bidirectional_paths_equal_wavefront(scene, kw):
             b = render(ctx, sid, s.cam, w, h, f, params, True)
             assert np.array_equal(a[0], b[0]), (w, h, f)
             assert a[1] == b[1], (w, h, f)
+
+
+@pytest.mark.parametrize("mode", [0, 1], ids=["pt", "bdpt"])
+def test_frames_in_the_arguments(mode):
+    """Launches of up to 16 frames take their seeds as arguments, longer ones
+    from memory; ray queries between them use the same counters."""
+    s = Y.gen_cornell()
+    params = Y.params_reference(mode, mis=1, bdpt_bounces=3)
+    rays = np.zeros((400000, 8), np.float32) + np.float32((0, 0, 9, 1e9, 0, 0, -1, 0))     # more than lanes
+    with Y.Context(max_paths=1 << 19) as ctx:
+        sid = ctx.scene(s)
+        j = ctx.job(sid, s.cam, 33, 21, params, base_seed=9)
+        ref = ctx.job(sid, s.cam, 33, 21, params, base_seed=9)
+        ref.set_counting(True)
+        for f in (1, 2, 15, 16, 17, 33, 1):
+            j.render(f)
+            if f & 1:
+                ctx.trace(sid, rays)
+            ref.render(f)
+            assert np.array_equal(j.read().view(np.int32), ref.read().view(np.int32)), f
+            a, b = j.stats(), ref.stats()
+            assert (a.rays_ext, a.rays_shadow, a.samples) == (b.rays_ext, b.rays_shadow, b.samples), f

@@ -545,21 +545,17 @@ __global__ __launch_bounds__(256, 3) void k_shade_bdpt(BdptShadeArgs a, DevCaptu
 // Work item -> path slot p: camera ray, light vertex 0 and the first light
 // ray (bdpt.cl:162-189, createLightPath :432-462).  Returns the path's
 // job-table entry; ray: the path's first ray.
-__device__ __forceinline__ int start_bdpt(const GenArgs& a, const DevCapture& cap, int item, int p, BState& bs,
-                                          float4& ot, float4& dp)
+template <typename TAB>
+__device__ __forceinline__ int start_bdpt(const GenArgs& a, const TAB& tab, const DevCapture& cap, int item, int p,
+                                          BState& bs, float4& ot, float4& dp)
 {
-    int lo = 0, hi = a.n_segs - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (a.segs[mid].path_base <= item) lo = mid; else hi = mid - 1;
-    }
-    const GenSeg& g = a.segs[lo];
+    const GenSeg g = seg_of<kOwnFramesBdpt>(a, item);
     int x, y;
     seg_pixel(item - g.path_base + g.first, g.w, g.h, x, y);
     x += g.x0;
     y += g.y0;
-    const DevJob& J = a.jobs[g.job];
-    const DevScene& S = a.scenes[J.scene];
+    const DevJob& J = tab.job(g.job);
+    const DevScene& S = tab.scene(J.scene);
     const yn_light_quad& L = S.light;
     const BdptSoA& B = a.B;
     uint32_t seed = pixel_seed(g.rand, x, y, J.W);
@@ -622,7 +618,7 @@ __global__ __launch_bounds__(256) void k_generate_bdpt(GenArgs a, DevCapture cap
     if (p >= a.n_paths) return;
     BState bs;
     float4 ot, dp;
-    a.P.job[p] = start_bdpt(a, cap, p, p, bs, ot, dp);
+    a.P.job[p] = start_bdpt(a, JobTables{a.jobs, a.scenes}, cap, p, p, bs, ot, dp);
     store_state(a.B, p, bs);
     a.ext_out.o_t[p] = ot;
     a.ext_out.d_p[p] = dp;
@@ -709,7 +705,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
     const DevCapture cap{};
     bool live = mine;
     if (live) {
-        jid = start_bdpt(a.g, cap, p, p, bs, ot, dp);
+        jid = start_bdpt(a.g, tables_of<ONE>(a), cap, p, p, bs, ot, dp);
         ext = true;
     }
     unsigned long long n_rays[2] = {0, 0};          // closest-hit and any-hit, of the wave
@@ -783,7 +779,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
                 if (b >= total) more = false;
                 const uint32_t i = b + (uint32_t)__popcll(idle & below);
                 if (!live && i < total) {
-                    jid = start_bdpt(a.g, cap, (int)i, p, bs, ot, dp);
+                    jid = start_bdpt(a.g, tables_of<ONE>(a), cap, (int)i, p, bs, ot, dp);
                     ext = live = true;
                 }
             }

@@ -127,6 +127,8 @@ __global__ __launch_bounds__(shade_block_pt(WAVES), WAVES) void k_shade_pt(Shade
 // Primary rays (pathtracer entry, udpt.cl:162-189) for a list of segments:
 // work item -> (segment, pixel), a ray at the item's queue position and the
 // new path's record beside it.
+// ONE: every path belongs to the arguments' job.
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_generate(GenArgs a, DevCapture cap)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -135,18 +137,13 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a, DevCapture cap)
     // behind the rays already queued: k_queue_reserve took the count before
     // this launch and added n_paths to it
     const uint32_t qpos = a.queue_base ? *a.queue_base + (uint32_t)i : (uint32_t)i;
-    int lo = 0, hi = a.n_segs - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (a.segs[mid].path_base <= item) lo = mid; else hi = mid - 1;
-    }
-    const GenSeg& g = a.segs[lo];
+    const GenSeg g = seg_of<kOwnFrames>(a, item);
     int x, y;
     seg_pixel(item - g.path_base + g.first, g.w, g.h, x, y);
     x += g.x0;
     y += g.y0;
-    const DevJob& J = a.jobs[g.job];
-    const DevScene& S = a.scenes[J.scene];
+    const DevJob& J = ONE ? a.job : a.jobs[g.job];
+    const yn_light_quad& light = ONE ? a.light : a.scenes[J.scene].light;
     uint32_t seed = pixel_seed(g.rand, x, y, J.W);
     float r1 = next_rand(seed);
     float r2 = next_rand(seed);
@@ -154,7 +151,7 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a, DevCapture cap)
     create_ray((float)x + r1, (float)y + r2, J.W, J.H, J.cam, o, d);
     float tq, tmax = INFINITY;
     int st = ST_PRIMARY | (J.scene << SCENE_SHIFT);
-    if (quad_hit(S.light, o, d, INFINITY, tq)) { tmax = tq; st |= F_LCAND; }
+    if (quad_hit(light, o, d, INFINITY, tq)) { tmax = tq; st |= F_LCAND; }
     *reinterpret_cast<int4*>(a.rec.f(PathRecs::M0, qpos)) = make_int4((int)seed, st, 0, -1);
     *reinterpret_cast<int4*>(a.rec.f(PathRecs::M1, qpos)) = make_int4(y * J.W + x, g.job, g.slot, 0);
     *a.rec.f(PathRecs::RD, qpos) = st4(d);
@@ -171,14 +168,20 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a, DevCapture cap)
 __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a)
 {
     int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a.ctr && blockIdx.x == 0 && threadIdx.x < 64) {     // the batch's last launch: its counters
+        const int i = (int)threadIdx.x;
+        unsigned long long *from = &a.ctr->rays_ext, *to = &a.host->rays_ext;
+        if (i < 6) to[i] = from[i];
+        if (i < 12) a.host->q[i][0] = a.ctr->q[i][0];
+        clear_counters(a.ctr);
+    }
     if (q >= a.w * a.h) return;
-    const DevJob& J = a.jobs[a.job];
     int x = a.x0 + q % a.w, y = a.y0 + q / a.w;
-    size_t pix = (size_t)y * J.W + x;
-    size_t npix = (size_t)J.W * J.H;
-    f4 acc = ld(a.accum[pix]);
+    size_t pix = (size_t)y * a.W + x;
+    size_t npix = (size_t)a.W * a.H;
+    f4 acc = ld(a.prev[pix]);
     for (int k = 0; k < a.n_slots; ++k) {
-        f4 c = ld(J.samples[(size_t)k * npix + pix]);
+        f4 c = ld(a.samples[(size_t)k * npix + pix]);
         if (k == 0 && a.reset_first) {
             c.w = 1;
         } else {
@@ -222,7 +225,8 @@ void launch_generate(const GenArgs& a, const DevCapture& cap, hipStream_t s)
     if (a.queue_base)
         hipLaunchKernelGGL(k_queue_reserve, dim3(1), dim3(64), 0, s, a.ext_out.count, (uint32_t)a.n_paths,
                            a.queue_base);
-    hipLaunchKernelGGL(k_generate, dim3(grid), dim3(256), 0, s, a, cap);
+    if (a.one) hipLaunchKernelGGL((k_generate<true>), dim3(grid), dim3(256), 0, s, a, cap);
+    else hipLaunchKernelGGL((k_generate<false>), dim3(grid), dim3(256), 0, s, a, cap);
 }
 void launch_shade_pt(const ShadeArgs& a, const DevCapture& cap, int grid, int waves, hipStream_t s)
 {

@@ -145,6 +145,7 @@ struct yn_ctx {
     RayQueue E[2]{}, Sh[2]{};
     DevCounters* ctr = nullptr;
     DevCounters* h_ctr = nullptr;     // pinned mirror
+    bool ctr_clear = false;           // every counter is zero (left so by a batch's last launch)
     GenSeg* d_segs = nullptr;
     int seg_cap = 0;
     float4* samples = nullptr;
@@ -629,17 +630,24 @@ bool paths_fit(const LoopCfg& L, bool capture) { return !L.count && L.width == 4
 
 // The launch's one job and scene as kernel arguments, when it has one and the
 // scene's materials fit LDS.
+bool is_one_job(const yn_ctx* c, const LoopCfg& L)
+{
+    if (L.job < 0 || L.single < 0) return false;
+    const SceneRec& S = c->scenes[L.single];
+    return S.bufs[4] && S.h_mats.size() <= (size_t)kLdsMats;
+}
+
 template <typename A>
 void one_job(const yn_ctx* c, const LoopCfg& L, A& a)
 {
-    if (L.job < 0 || L.single < 0 || a.s.lmode != 1) return;
+    if (!is_one_job(c, L)) return;
     a.one = 1;
     a.job = c->jobs[L.job].dev;
     a.scene = c->scenes[L.single].dev;
 }
 
 // Enqueues k_paths on the rays of the queues that A's shade reads: their
-// paths run to their ends in one launch.  The counters follow to the host.
+// paths run to their ends in one launch.
 int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
 {
     PathsArgs pa{};
@@ -657,7 +665,6 @@ int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
     pa.ovf_depth = c->ovf_depth;
     launch_paths(pa, grid, c->stream);
     HIPCK(c, hipGetLastError());
-    HIPCK(c, hipMemcpyAsync(c->h_ctr, c->ctr, kCtrHostBytes, hipMemcpyDeviceToHost, c->stream));
     return 0;
 }
 
@@ -678,14 +685,37 @@ int enqueue_paths_bdpt(yn_ctx* c, const LoopCfg& L, const IterArgs& A, const Gen
     pa.ovf_depth = c->ovf_depth;
     launch_paths_bdpt(pa, grid, c->stream);
     HIPCK(c, hipGetLastError());
-    HIPCK(c, hipMemcpyAsync(c->h_ctr, c->ctr, kCtrHostBytes, hipMemcpyDeviceToHost, c->stream));
     return 0;
+}
+
+// Folds a batch's samples into an image; the batch's last one also hands the
+// counters to the host and clears them.
+void resolve(yn_ctx* c, const DevJob& d, int x0, int y0, int w, int h, int frames, bool reset_first, float4* accum,
+             const float4* prev, bool last)
+{
+    ResolveArgs ra{};
+    ra.W = d.W;
+    ra.H = d.H;
+    ra.samples = d.samples;
+    ra.x0 = x0;
+    ra.y0 = y0;
+    ra.w = w;
+    ra.h = h;
+    ra.n_slots = frames;
+    ra.reset_first = reset_first ? 1 : 0;
+    ra.accum = accum;
+    ra.prev = prev ? prev : accum;
+    ra.ctr = last ? c->ctr : nullptr;
+    ra.host = c->h_ctr;
+    launch_resolve(ra, c->stream);
 }
 
 // Waits for the batch's last launches and reads its counters.
 int finish_batch(yn_ctx* c, int64_t total, JobRec& stat_job)
 {
+    HIPCK(c, hipGetLastError());
     HIPCK(c, hipStreamSynchronize(c->stream));
+    c->ctr_clear = true;
     if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
     if (c->h_ctr->q[6][0]) return fail(c, YN_ERR_HIP, "paths did not end");
     stat_job.st.rays_ext += c->h_ctr->rays_ext;
@@ -698,11 +728,32 @@ int finish_batch(yn_ctx* c, int64_t total, JobRec& stat_job)
     return 0;
 }
 
+// A job's table entry for the next batch (run_batch uploads it if its
+// launches read the table).
+void set_job(yn_ctx* c, int jid, float4* samples)
+{
+    JobRec& J = c->jobs[jid];
+    J.dev = make_devjob(J);
+    J.dev.samples = samples;
+}
+
+int upload_jobs(yn_ctx* c, const std::vector<Region>& regs)
+{
+    int last = -1;
+    for (const Region& r : regs) {      // a job's regions follow each other
+        if (r.job == last) continue;
+        last = r.job;
+        HIPCK(c, hipMemcpyAsync(c->d_jobs + r.job, &c->jobs[r.job].dev, sizeof(DevJob), hipMemcpyHostToDevice,
+                                c->stream));
+    }
+    return 0;
+}
+
 // Runs one batch of primary-ray regions; samples land in samples[slot][pixel]
 // of each region's job (the sample buffer is shared: job slots are laid out
 // by the caller so regions do not overlap).  The last launches may still run
-// when it returns: the caller enqueues what uses the samples and then calls
-// finish_batch with *paths.
+// when it returns: the caller folds the samples (resolve, the last one with
+// `last`) and then calls finish_batch with *paths.
 int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, const DevCapture& cap, int64_t* paths)
 {
     std::vector<GenSeg> segs;
@@ -722,17 +773,9 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     if (bdpt ? total > C : total > c->sample_cap) return fail(c, YN_ERR_INVALID, "batch larger than the path capacity");
     const bool regen = !bdpt && total > C;
     int64_t issued = std::min<int64_t>(total, C);
-    if ((int)segs.size() > c->seg_cap) {
-        if (c->d_segs) hipFree(c->d_segs);
-        c->d_segs = nullptr;
-        c->seg_cap = std::max<int>((int)segs.size(), 256);
-        int r = dalloc(c, &c->d_segs, (size_t)c->seg_cap);
-        if (r) return r;
-    }
     hipStream_t s = c->stream;
-    HIPCK(c, hipMemcpyAsync(c->d_segs, segs.data(), sizeof(GenSeg) * segs.size(), hipMemcpyHostToDevice, s));
-    HIPCK(c, hipMemsetAsync(c->ctr, 0, sizeof(DevCounters), s));
-
+    const bool clear = c->ctr_clear;
+    c->ctr_clear = false;       // until finish_batch
     const DevScene* scenes = c->d_scenes;
     auto q = [&](int k) { return &c->ctr->q[k][0]; };
     // counters (q(k) = q[k][0]): q[0],q[1] extension queue counts, q[2],q[3] shadow queue
@@ -747,15 +790,6 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     }
     c->ev_used = 0;
 
-    GenArgs ga{};
-    ga.scenes = scenes;
-    ga.jobs = c->d_jobs;
-    ga.P = c->P;
-    ga.rec = c->P.R[0];
-    ga.ext_out = c->E[0];
-    ga.segs = c->d_segs;
-    ga.n_segs = (int32_t)segs.size();
-    ga.n_paths = (int32_t)issued;
     std::vector<int> scene_ids;
     for (const Region& r : regs) scene_ids.push_back(c->jobs[r.job].scene);
     LoopCfg L;
@@ -769,17 +803,59 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     make_iter(c, L, 1, iters[1]);
     const bool any_cap = cap.prim_tri || cap.prim_light || cap.prim_t || cap.shadow_o || cap.shadow_d || cap.shadow_occ;
     const bool paths_ok = paths_fit(L, any_cap);
+    bool direct = paths_ok && !regen && total <= kPathsDirect;
+    if (bdpt) {
+        int vertices = 0;
+        for (const Region& r : regs) vertices = std::max(vertices, (int)c->jobs[r.job].p.bdpt_bounces);
+        direct = paths_ok && bdpt_paths_win(total, vertices, L.node_bytes);
+    }
+
+    GenArgs ga{};
+    ga.scenes = scenes;
+    ga.jobs = c->d_jobs;
+    ga.P = c->P;
+    ga.rec = c->P.R[0];
+    ga.ext_out = c->E[0];
+    ga.n_segs = (int32_t)segs.size();
+    ga.n_paths = (int32_t)issued;
+    // a few frames of one rectangle travel in the arguments
+    bool own = segs.size() <= (size_t)(bdpt ? kOwnFramesBdpt : kOwnFrames);
+    for (size_t k = 0; k < segs.size() && own; ++k) {
+        const GenSeg &a = segs[0], &b = segs[k];
+        own = b.job == a.job && b.slot == a.slot + (int32_t)k && b.x0 == a.x0 && b.y0 == a.y0 && b.w == a.w && b.h == a.h;
+        ga.frame_rand[k] = b.rand;
+    }
+    if (own) {
+        ga.seg = segs[0];
+    } else {
+        if ((int)segs.size() > c->seg_cap) {
+            if (c->d_segs) hipFree(c->d_segs);
+            c->d_segs = nullptr;
+            c->seg_cap = std::max<int>((int)segs.size(), 256);
+            if (int r = dalloc(c, &c->d_segs, (size_t)c->seg_cap)) return r;
+        }
+        HIPCK(c, hipMemcpyAsync(c->d_segs, segs.data(), sizeof(GenSeg) * segs.size(), hipMemcpyHostToDevice, s));
+        ga.segs = c->d_segs;
+    }
+    // so does the one job of a launch of whole paths
+    const bool one = direct && is_one_job(c, L);
+    if (one) {
+        ga.one = 1;
+        ga.job = c->jobs[L.job].dev;
+        ga.light = c->scenes[L.single].dev.light;
+    } else if (int r = upload_jobs(c, regs)) {
+        return r;
+    }
+    if (!clear) HIPCK(c, hipMemsetAsync(c->ctr, 0, sizeof(DevCounters), s));
     if (bdpt) {
         ga.B = c->B;
         ga.list_out = c->lst[0];
         ga.list_count = q(8);
-        int vertices = 0;
-        for (const Region& r : regs) vertices = std::max(vertices, (int)c->jobs[r.job].p.bdpt_bounces);
-        if (paths_ok && bdpt_paths_win(total, vertices, L.node_bytes)) return enqueue_paths_bdpt(c, L, iters[0], ga);
+        if (direct) return enqueue_paths_bdpt(c, L, iters[0], ga);
         launch_generate_bdpt(ga, cap, s);
     } else {
         launch_generate(ga, cap, s);
-        if (paths_ok && total <= kPathsDirect && !regen) return enqueue_paths(c, L, iters[0], true);
+        if (direct) return enqueue_paths(c, L, iters[0], true);
     }
     const int group = 4;                 // iterations between host checks (even)
     // Graph replay of a group (not with ray capture for tests)
@@ -846,21 +922,13 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     return 0;
 }
 
-int upload_job_table(yn_ctx* c, int jid, float4* samples)
-{
-    DevJob& d = c->jobs[jid].dev;
-    d = make_devjob(c->jobs[jid]);
-    d.samples = samples;
-    HIPCK(c, hipMemcpyAsync(c->d_jobs + jid, &d, sizeof(DevJob), hipMemcpyHostToDevice, c->stream));
-    return 0;
-}
-
 int stream_drain(yn_ctx* c);
 
 // Render n frames of rectangle [x0,x0+w) x [y0,y0+h) into `accum`, frames
-// taking seeds from `seeds`; first frame resets when reset_first.
+// taking seeds from `seeds`; first frame resets when reset_first, else it is
+// folded into `prev` (null: accum itself).
 int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h, const std::vector<uint32_t>& seeds,
-                bool reset_first, const DevCapture& cap)
+                bool reset_first, const DevCapture& cap, const float4* prev = nullptr)
 {
     JobRec& J = c->jobs[jid];
     int64_t npix = (int64_t)w * h;
@@ -887,14 +955,12 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
         if (kcap >= 1) {
             nslots = (int)std::min<int64_t>(kcap, (int64_t)(seeds.size() - f));
             for (int k = 0; k < nslots; ++k) regs.push_back({jid, k, seeds[f + k], x0, y0, w, h});
-            int r = upload_job_table(c, jid, c->samples);
-            if (r) return r;
+            set_job(c, jid, c->samples);
             DevCapture cp = f == 0 ? cap : DevCapture{};
             int64_t paths = 0;
-            r = run_batch(c, regs, J, cp, &paths);
+            int r = run_batch(c, regs, J, cp, &paths);
             if (r) return r;
-            ResolveArgs ra{c->d_jobs, jid, x0, y0, w, h, nslots, (reset_first && f == 0) ? 1 : 0, accum};
-            launch_resolve(ra, c->stream);
+            resolve(c, J.dev, x0, y0, w, h, nslots, reset_first && f == 0, accum, f == 0 ? prev : nullptr, true);
             if (int e = finish_batch(c, paths, J)) return e;
         } else {
             // image larger than the path capacity: row bands, one frame at a time
@@ -908,14 +974,12 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
                 // sample slot 0 is addressed as [pixel]; offset the buffer so the
                 // band's pixels land inside the path-sized sample buffer
                 float4* base = c->samples - (int64_t)yb * J.W;
-                int r = upload_job_table(c, jid, base);
-                if (r) return r;
+                set_job(c, jid, base);
                 DevCapture cp = f == 0 ? cap : DevCapture{};
                 int64_t paths = 0;
-                r = run_batch(c, regs, J, cp, &paths);
+                int r = run_batch(c, regs, J, cp, &paths);
                 if (r) return r;
-                ResolveArgs ra{c->d_jobs, jid, x0, yb, w, hh, 1, (reset_first && f == 0) ? 1 : 0, accum};
-                launch_resolve(ra, c->stream);
+                resolve(c, J.dev, x0, yb, w, hh, 1, reset_first && f == 0, accum, f == 0 ? prev : nullptr, true);
                 if (int e = finish_batch(c, paths, J)) return e;
             }
         }
@@ -1034,16 +1098,13 @@ int serve_round(yn_ctx* c, int* frames_out)
         if (J.t_start < 0) J.t_start = ms_since(c);
     }
     if (regs.empty()) return 0;
-    for (const Plan& pl : plan)
-        if (int r = upload_job_table(c, pl.jid, c->samples + pl.off)) return r;
+    for (const Plan& pl : plan) set_job(c, pl.jid, c->samples + pl.off);
     int64_t paths = 0;
     if (int r = run_batch(c, regs, c->serve_rec, DevCapture{}, &paths)) return r;
     for (const Plan& pl : plan) {
         JobRec& J = c->jobs[pl.jid];
-        ResolveArgs ra{c->d_jobs, pl.jid, 0, 0, J.W, J.H, pl.k, pl.reset ? 1 : 0, J.accum};
-        launch_resolve(ra, c->stream);
+        resolve(c, J.dev, 0, 0, J.W, J.H, pl.k, pl.reset, J.accum, nullptr, &pl == &plan.back());
     }
-    HIPCK(c, hipGetLastError());
     if (int r = finish_batch(c, paths, c->serve_rec)) return r;
     double now = ms_since(c);
     for (const Plan& pl : plan) {
@@ -1116,6 +1177,7 @@ int stream_start(yn_ctx* c)
     StreamState& S = c->strm;
     hipStream_t s = c->stream;
     S.active = true;
+    c->ctr_clear = false;
     S.it = 0;
     S.cap = stream_cap(c);
     S.issue.clear();
@@ -1261,8 +1323,9 @@ int stream_fold(yn_ctx* c)
             if (!P.orphan) {
                 JobRec& J = c->jobs[P.job];
                 if ((int64_t)J.frame != P.f0) continue;      // an earlier piece of the job is not folded yet
-                ResolveArgs ra{c->d_jobs, kMaxJobs + i, 0, 0, J.W, J.H, P.k, P.f0 == 0 ? 1 : 0, J.accum};
-                launch_resolve(ra, c->stream);
+                DevJob d = make_devjob(J);
+                d.samples = c->samples + P.soff;
+                resolve(c, d, 0, 0, J.W, J.H, P.k, P.f0 == 0, J.accum, nullptr, false);
                 J.frame += (uint64_t)P.k;
                 J.st.frames += (uint64_t)P.k;
                 J.st.samples += (uint64_t)P.items;
@@ -1727,7 +1790,7 @@ int yn_job_create(yn_ctx* c, int32_t sid, const yn_cam* cam, int32_t W, int32_t 
     J.bytes = bytes;
     c->job_bytes += bytes;
     *job_id = jid;
-    return upload_job_table(c, jid, c->samples);
+    return 0;
 }
 
 int yn_job_render(yn_ctx* c, int32_t jid, int32_t n_frames)
@@ -2165,14 +2228,9 @@ int yn_pathtracer(yn_ctx* c, float* out_img, const float* in_img, const yn_cam* 
     JobRec& J = c->jobs[jid];
     J = JobRec();
     J.scene = sid; J.cam = *cam; J.W = W; J.H = H; J.p = *params; J.p.gi = gi_check;
-    // previous frame -> output for the tile, then fold this frame in place
-    if (!reset)
-        HIPCK(c, hipMemcpy2DAsync(out_img + 4 * ((size_t)y0 * W + x0), (size_t)W * 16, in_img + 4 * ((size_t)y0 * W + x0),
-                                  (size_t)W * 16, (size_t)w * 16, (size_t)h, hipMemcpyDeviceToDevice, c->stream));
     std::vector<uint32_t> seeds(1, rand);
-    int r = render_rect(c, jid, (float4*)out_img, x0, y0, w, h, seeds, reset != 0, DevCapture{});
-    if (r == 0) HIPCK(c, hipStreamSynchronize(c->stream));
-    return r;
+    return render_rect(c, jid, (float4*)out_img, x0, y0, w, h, seeds, reset != 0, DevCapture{},
+                       reset ? nullptr : (const float4*)in_img);
 }
 
 int yn_tonemap_op(yn_ctx* c, const float* in_img, float* out_img, int32_t W, int32_t H, int32_t op)
@@ -2231,7 +2289,10 @@ int yn_trace(yn_ctx* c, int32_t sid, const float* rays, int32_t n, int32_t* tri,
     if (host) std::memcpy(io, rays, (size_t)n * 32);
     else HIPCK(c, hipMemcpyAsync(io, rays, (size_t)n * 32, hipMemcpyHostToDevice, s));
     if ((int64_t)n > (int64_t)(grid / a.n_slices) * a.n_slices * kRaysBlock)     // more rays than lanes
+    {
+        c->ctr_clear = false;
         HIPCK(c, hipMemsetAsync(a.work, 0, sizeof(uint32_t) * kMaxXcd * kWorkStride, s));
+    }
     *a.full = 0;
     launch_rays(a, S.info.width, lds, grid, s);
     HIPCK(c, hipGetLastError());

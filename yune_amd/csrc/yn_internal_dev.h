@@ -180,14 +180,21 @@ struct BdptShadeArgs {
     int32_t n_lights;
 };
 
+// Frames whose seeds travel in the arguments.  One in bidirectional mode: the
+// selection below in the refill of k_paths_bdpt cost 0.6% (8 frames of
+// 1280x720: 13.44 -> 13.52 ms) and a loop over the frames 5%.
+constexpr int kOwnFrames = 16;
+constexpr int kOwnFramesBdpt = 1;
 struct GenArgs {
     const DevScene* scenes;
     const DevJob* jobs;
     PathSoA P;                  // bidirectional mode
     PathRecs rec;               // unidirectional mode: the records beside ext_out
     RayQueue ext_out;
-    const GenSeg* segs;
-    int32_t n_segs;
+    const GenSeg* segs;         // or null: a few frames of one rectangle, `seg`
+    int32_t n_segs;             //   the first and frame_rand their seeds, so that a small
+    GenSeg seg;                 //   launch needs no copy to the device
+    uint32_t frame_rand[kOwnFrames];
     int32_t n_paths;
     BdptSoA B;                  // bidirectional mode only
     uint32_t* list_out;         // bidirectional mode: every path starts listed
@@ -198,7 +205,43 @@ struct GenArgs {
     // the launch sets the queue's count
     int32_t item0;
     uint32_t* queue_base;
+    int32_t one;                // 1: every path belongs to `job`, in a scene with `light`
+    DevJob job;
+    yn_light_quad light;
 };
+
+// The segment of a work item (see GenArgs::segs).
+template <int FRAMES>
+__device__ __forceinline__ GenSeg seg_of(const GenArgs& a, int item)
+{
+    if (a.segs) {
+        int lo = 0, hi = a.n_segs - 1;
+        while (lo < hi) {
+            int mid = (lo + hi + 1) >> 1;
+            if (a.segs[mid].path_base <= item) lo = mid; else hi = mid - 1;
+        }
+        return a.segs[lo];
+    }
+    GenSeg g = a.seg;
+    const int px = g.w * g.h;
+    for (int k = 1; k < FRAMES; ++k)
+        if (k < a.n_segs && item >= a.seg.path_base + k * px) {
+            g.slot = a.seg.slot + k;
+            g.path_base = a.seg.path_base + k * px;
+            g.rand = a.frame_rand[k];
+        }
+    return g;
+}
+
+// Clears every counter (one wave calls it).
+__device__ __forceinline__ void clear_counters(DevCounters* c)
+{
+    const int i = (int)__lane_id();
+    unsigned long long* h = &c->rays_ext;
+    if (i < 6) h[i] = 0;
+    if (i < 12) c->q[i][0] = 0;
+    if (i < 2 * kMaxXcd) c->work[i / kMaxXcd][i % kMaxXcd][0] = 0;
+}
 
 // Whole bidirectional paths in one launch (k_paths_bdpt): the work items of
 // g, in slots of s.B.
@@ -216,12 +259,15 @@ struct BdptPathsArgs {
 };
 
 struct ResolveArgs {
-    DevJob* jobs;
-    int32_t job;
+    int32_t W, H;               // the image and the rectangle of it to fold
+    const float4* samples;      // [frame slot][W*H]
     int32_t x0, y0, w, h;
     int32_t n_slots;            // frames in this batch, oldest first
     int32_t reset_first;        // first frame of the batch overwrites (kernel arg 9)
     float4* accum;              // the job's RGBA32F image, .w = count
+    const float4* prev;         // the image before the first frame (kernel arg 1; accum itself for a job)
+    DevCounters* ctr;           // not null: the batch's counters go to `host` (pinned) and are cleared
+    DevCounters* host;
 };
 
 // Capture of the first frame for hit-ID parity (null pointers: off).
