@@ -110,3 +110,26 @@ def test_frames_in_the_arguments(mode):
             assert np.array_equal(j.read().view(np.int32), ref.read().view(np.int32)), f
             a, b = j.stats(), ref.stats()
             assert (a.rays_ext, a.rays_shadow, a.samples) == (b.rays_ext, b.rays_shadow, b.samples), f
+
+
+@pytest.mark.parametrize("size,frames", [(9, 1), (64, 3), (1500, 4)])
+def test_continuous_jobs_end_in_one_launch(size, frames):
+    """Jobs of two scenes, few enough for one launch or (9M paths) a wavefront
+    first, with submissions between the calls, against each job alone."""
+    scenes = [Y.gen_cornell(), Y.gen_icosphere_room(3, 4, 3)]
+    params = Y.params_reference(0, mis=1)
+    with Y.Context(serve_mode=0) as ctx:
+        sids = [ctx.scene(s) for s in scenes]
+        jobs = []
+        for k in range(4):
+            jobs.append((ctx.submit(sids[k % 2], scenes[k % 2].cam, size + k, size, params, frames, 4 + k), k))
+            if k & 1:
+                ctx.serve(1)
+        while ctx.serve(4):
+            pass
+        for j, k in jobs:
+            alone = ctx.job(sids[k % 2], scenes[k % 2].cam, size + k, size, params, base_seed=4 + k)
+            alone.set_counting(True)
+            alone.render(frames)
+            assert np.array_equal(j.read().view(np.int32), alone.read().view(np.int32)), k
+            alone.release()
