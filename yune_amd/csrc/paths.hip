@@ -37,30 +37,6 @@ struct RegResult {
     __device__ __forceinline__ int occ() const { return o; }
 };
 
-// What a path's pending ray needs of its record while it is traced: the
-// fields of Rec that its state uses (BOUNCE: nd, bnc; NEE_SH: wi; NEE_MIS:
-// ls, mis, wi's pdf), without the direction, which the ray holds.  Six
-// registers instead of Rec's twenty.
-struct Pend { float a, b, c, d, e, f; };
-
-__device__ __forceinline__ Pend pack(const Rec& R)
-{
-    const int code = R.m0.y & ST_MASK;
-    if (code == ST_NEE_MIS) return Pend{R.ls.x, R.ls.y, R.ls.z, R.ls.w, R.mis.w, R.wi.w};
-    if (code == ST_NEE_SH) return Pend{R.wi.w, 0, 0, 0, 0, 0};
-    return Pend{R.nd.w, R.bnc.x, R.bnc.y, R.bnc.z, 0, 0};
-}
-
-__device__ __forceinline__ void unpack(const Pend& q, const RayState& r, Rec& R)
-{
-    const bool mis = (R.m0.y & ST_MASK) == ST_NEE_MIS;
-    R.nd = mk(r.dx, r.dy, r.dz, q.a);
-    R.bnc = mk(q.b, q.c, q.d, 0.0f);
-    R.wi = mk(r.dx, r.dy, r.dz, mis ? q.f : q.a);
-    R.ls = mk(q.a, q.b, q.c, q.d);
-    R.mis = mk(r.dx, r.dy, r.dz, q.e);
-}
-
 // (The arguments' address is opaque at each call: otherwise the compiler
 // loads every field before the loop and spills what the registers cannot
 // hold, instead of loading it again where it is used.)
@@ -117,7 +93,6 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
     bool more = total > n_waves * per;              // paths beyond the static ones
     Rec R;
     R.m0 = make_int4(0, 0, 0, 0);
-    Pend q{0, 0, 0, 0, 0, 0};
     float4 ot = make_float4(0, 0, 0, 0), dp = ot;
     bool any = false, live = false;
     // takes path i of the queues: first the extension queue's, then the shadow queue's
@@ -128,8 +103,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
         any = !ext;
         ot = ext ? s.ext_in.o_t[qi] : s.sh_in.o_t[qi];
         dp = ext ? s.ext_in.d_p[qi] : s.sh_in.d_p[qi];
-        load_rec(s.in, ext ? qi : (uint32_t)(s.in.cap - 1 - (int64_t)qi), R, ext, ext && s.ext_primary);
-        q = pack(R);
+        load_rec(s.in, ext ? qi : (uint32_t)(s.in.cap - 1 - (int64_t)qi), dp, R, ext && s.ext_primary);
     };
     if ((uint32_t)lane < per && wave * per + (uint32_t)lane < total) take(wave * per + (uint32_t)lane);
     unsigned long long n_rays[2] = {0, 0};          // closest-hit and any-hit, of the wave
@@ -160,10 +134,10 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
             } else {
                 while (go) go = trav_step<4, 2, kPathsLds, BL, false, false>(nodes, tri, node, r, st, got, c);
             }
-            unpack(q, r, R);
+            R.dir = mk(dp.x, dp.y, dp.z, 0.0f);
+            R.job = __float_as_int(dp.w);
             const Out o = advance<false, LM>(
                 tab, cap, RegResult{hit_record(r), got ? 1 : 0}, R, lds);
-            q = pack(R);
             ot = o.o_t;
             dp = o.d_p;
             any = o.kind == 2;

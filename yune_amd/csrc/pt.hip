@@ -87,7 +87,8 @@ __global__ __launch_bounds__(shade_block_pt(WAVES), WAVES) void k_shade_pt(Shade
         if (i < total) {
             const bool ext = i < n_ext;
             const uint32_t qi = ext ? i : i - n_ext;
-            load_rec(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), R, ext, ext && a.ext_primary);
+            const float4 dp = ext ? a.ext_in.d_p[qi] : a.sh_in.d_p[qi];
+            load_rec(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), dp, R, ext && a.ext_primary);
             o = advance<CAP, LM>(JobTables{a.jobs, a.scenes}, cap, QueueResult{a.hit, a.occ, qi}, R, lds);
         }
         const uint32_t n[2] = {o.kind == 1 ? 1u : 0u, o.kind == 2 ? 1u : 0u};
@@ -152,9 +153,8 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a, DevCapture cap)
     float tq, tmax = INFINITY;
     int st = ST_PRIMARY | (J.scene << SCENE_SHIFT);
     if (quad_hit(light, o, d, INFINITY, tq)) { tmax = tq; st |= F_LCAND; }
-    *reinterpret_cast<int4*>(a.rec.f(PathRecs::M0, qpos)) = make_int4((int)seed, st, 0, -1);
-    *reinterpret_cast<int4*>(a.rec.f(PathRecs::M1, qpos)) = make_int4(y * J.W + x, g.job, g.slot, 0);
-    *a.rec.f(PathRecs::RD, qpos) = st4(d);
+    const uint32_t sample = (uint32_t)g.slot * (uint32_t)(J.W * J.H) + (uint32_t)(y * J.W + x);
+    *reinterpret_cast<int4*>(a.rec.f(PathRecs::M0, qpos)) = make_int4((int)seed, st, (int)sample, 0);
     a.ext_out.o_t[qpos] = make_float4(o.x, o.y, o.z, tmax);
     a.ext_out.d_p[qpos] = make_float4(d.x, d.y, d.z, __int_as_float(g.job));
     if (!a.queue_base && i == 0) *a.ext_out.count = (uint32_t)a.n_paths;

@@ -61,31 +61,29 @@ struct RayQueue {
 // so records move with their rays in queue order and every access is
 // coalesced.
 struct PathRecs {
-    // Thirteen 16-byte fields per record in one allocation, in tiles of
+    // Nine 16-byte fields per record in one allocation, in tiles of
     // kTile records: tile t holds field 0 of its records, then field 1, ...
     // (field f of record r at base[((r / kTile) * FIELDS + f) * kTile +
     // r % kTile]).  A wave's 64 consecutive records still read each field
-    // as two whole 512-byte runs, and all thirteen fields of a record lie
-    // within +-3 KB of its field 6, so one address per record and immediate
+    // as two whole 512-byte runs, and all nine fields of a record lie
+    // within +-2 KB of its field 4, so one address per record and immediate
     // offsets reach them (a field-major layout needs one 64-bit base per
     // field, which the shade kernels could only keep in spill lanes).
     static constexpr int kTile = 32;
     float4* base;
     int64_t cap;                // records (paths in flight at most)
     enum Field {
-        M0,                     // int4 {seed, state | flags, bounce, material of the current vertex}
-        M1,                     // int4 {pixel, job-table entry, frame slot, NEE lobe probability bits}
+        M0,                     // int4 {seed, state | flags, bounce, material of the current vertex};
+                                //   a new path's: {seed, state | flags, sample, 0}, its only field
+        M1,                     // {sample (frame slot * W * H + pixel) bits, a, b, c}: floats of the
+                                //   pending ray (see Rec)
         HP,                     // vertex position
         HN,                     // shading normal
-        RD,                     // incoming direction (the camera ray's for a new path)
-        TP,                     // throughput
-        DIRECT,                 // direct light of the first vertex
-        INDIRECT,               // everything else
-        ND,                     // pending bounce direction
-        BNC,                    // pending bounce: pdf, lobe probability, ior
-        WI,                     // NEE: light direction, w = light pdf
-        LS,                     // NEE: MIS-weighted light sample
-        MIS,                    // NEE: MIS BRDF direction, w = BRDF pdf
+        RD,                     // incoming direction
+        TP,                     // throughput            | not held at the first vertex, where it is
+        DIRECT,                 // direct light of it    | 1, while that vertex's light is sampled,
+        INDIRECT,               // everything else       | where it is 0, and at it, where it is 0
+        LS,                     // MIS ray pending: the weighted light sample
         FIELDS
     };
     __host__ __device__ float4* f(int field, int64_t r) const

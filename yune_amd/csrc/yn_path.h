@@ -33,16 +33,24 @@ struct Out {
     float4 d_p;
 };
 
-// A path's state between two shade steps (the fields of PathRecs).
+// A path's state between two shade steps (the fields of PathRecs, and of the
+// pending ray, which holds the rest).
 struct Rec {
-    int4 m0, m1;
-    f4 hp, hn, rd, tp, direct, indirect, nd, bnc, wi, ls, mis;
+    int4 m0;
+    uint32_t sample;        // frame slot * W * H + pixel (below 4 * 2^30: what fits the card)
+    int job;                // the ray's: job-table entry
+    f4 dir;                 // the ray's: its direction, w = 0
+    // of a bounce ray: pdf and lobe probability, or, off a specular surface,
+    // the index-of-refraction factor and the direction's w; of a shadow ray:
+    // light pdf and lobe probability; of a MIS ray also the BRDF's pdf
+    float a, b, c;
+    f4 hp, hn, rd, tp, direct, indirect, ls;
 };
 
-__device__ __forceinline__ void write_sample(const DevJob& J, int slot, int pix, f4 c)
+__device__ __forceinline__ void write_sample(const DevJob& J, uint32_t sample, f4 c)
 {
     if (any_nan(c)) c = mk(kPinkR, kPinkG, kPinkB, 1.0f);     // udpt.cl:193-194
-    J.samples[(size_t)slot * (size_t)(J.W * J.H) + (size_t)pix] = st4(c);
+    J.samples[sample] = st4(c);
 }
 
 // The ray's w carries the path's job-table entry: the trace kernels look
@@ -56,40 +64,40 @@ __device__ __forceinline__ Out make_ray(int kind, f4 o, f4 d, float tmax, int jo
     return r;
 }
 
-// The record a step reads.  The fields most states use are loaded without
-// waiting for the state (a new path's record holds only m0, m1 and the
-// camera ray's direction; the rest is not used then); only the MIS ray's
-// fields, used by one state, wait for it.  The shade pass is bound by the
-// latency of such chains of loads.  Which queue the result came from is
-// known before the state: a bounce result (extension queue) reads the
-// pending bounce and never the NEE light direction, a shadow result the
-// light direction and never the pending bounce (each is rewritten before
-// the step stores it), so each loads only its own.
-__device__ __forceinline__ void load_rec(const PathRecs& I, uint32_t ri, Rec& R, bool ext, bool primary)
+// The record a step reads; dp: the pending ray's second half.  The shade pass
+// is bound by memory traffic, so a record holds nothing that the ray or the
+// state already says: the ray's direction and job are read from the queue, a
+// new path has no fields but M0, and the first vertex's constants (half of
+// all steps are there) are not stored.  What every later state uses is loaded
+// without waiting for the state, the rest once it is known.
+__device__ __forceinline__ void load_rec(const PathRecs& I, uint32_t ri, float4 dp, Rec& R, bool primary)
 {
     using F = PathRecs;
     R.m0 = *reinterpret_cast<const int4*>(I.f(F::M0, ri));
-    R.m1 = *reinterpret_cast<const int4*>(I.f(F::M1, ri));
-    R.rd = ld(*I.f(F::RD, ri));
-    if (primary) {          // a camera ray's record: the rest is set by its step
-        R.hp = R.hn = R.tp = R.direct = R.indirect = R.nd = R.bnc = R.wi = mk(0, 0, 0, 0);
-        return;
+    R.dir = mk(dp.x, dp.y, dp.z, 0.0f);
+    R.job = __float_as_int(dp.w);
+    R.hp = R.hn = R.rd = R.direct = R.indirect = R.ls = mk(0, 0, 0, 0);
+    R.tp = mk(1, 1, 1, 1);
+    R.a = R.b = R.c = 0;
+    if (!primary) {
+        const float4 m1 = *I.f(F::M1, ri);
+        R.sample = __float_as_uint(m1.x);
+        R.a = m1.y; R.b = m1.z; R.c = m1.w;
+        R.hp = ld(*I.f(F::HP, ri));
+        R.hn = ld(*I.f(F::HN, ri));
+        R.rd = ld(*I.f(F::RD, ri));
     }
-    R.hp = ld(*I.f(F::HP, ri));
-    R.hn = ld(*I.f(F::HN, ri));
-    R.tp = ld(*I.f(F::TP, ri));
-    R.direct = ld(*I.f(F::DIRECT, ri));
-    R.indirect = ld(*I.f(F::INDIRECT, ri));
-    R.nd = R.bnc = R.wi = mk(0, 0, 0, 0);
-    if (ext) {
-        R.nd = ld(*I.f(F::ND, ri));
-        R.bnc = ld(*I.f(F::BNC, ri));
+    const int code = R.m0.y & ST_MASK;
+    if (code == ST_PRIMARY) {
+        R.sample = (uint32_t)R.m0.z;
+        R.m0.z = 0;
     } else {
-        R.wi = ld(*I.f(F::WI, ri));
-    }
-    if ((R.m0.y & ST_MASK) == ST_NEE_MIS) {
-        R.ls = ld(*I.f(F::LS, ri));
-        R.mis = ld(*I.f(F::MIS, ri));
+        if (R.m0.z > 0) {
+            R.tp = ld(*I.f(F::TP, ri));
+            R.indirect = ld(*I.f(F::INDIRECT, ri));
+        }
+        if (R.m0.z > 0 || code == ST_BOUNCE) R.direct = ld(*I.f(F::DIRECT, ri));
+        if (code == ST_NEE_MIS) R.ls = ld(*I.f(F::LS, ri));
     }
 }
 
@@ -98,24 +106,17 @@ __device__ __forceinline__ void store_rec(const PathRecs& O, uint32_t ri, const 
 {
     using F = PathRecs;
     *reinterpret_cast<int4*>(O.f(F::M0, ri)) = R.m0;
-    *reinterpret_cast<int4*>(O.f(F::M1, ri)) = R.m1;
+    *O.f(F::M1, ri) = make_float4(__uint_as_float(R.sample), R.a, R.b, R.c);
     *O.f(F::HP, ri) = st4(R.hp);
     *O.f(F::HN, ri) = st4(R.hn);
     *O.f(F::RD, ri) = st4(R.rd);
-    *O.f(F::TP, ri) = st4(R.tp);
-    *O.f(F::DIRECT, ri) = st4(R.direct);
-    *O.f(F::INDIRECT, ri) = st4(R.indirect);
     const int code = R.m0.y & ST_MASK;
-    if (code == ST_BOUNCE) {
-        *O.f(F::ND, ri) = st4(R.nd);
-        *O.f(F::BNC, ri) = st4(R.bnc);
-    } else {
-        *O.f(F::WI, ri) = st4(R.wi);
-        if (code == ST_NEE_MIS) {
-            *O.f(F::LS, ri) = st4(R.ls);
-            *O.f(F::MIS, ri) = st4(R.mis);
-        }
+    if (R.m0.z > 0) {
+        *O.f(F::TP, ri) = st4(R.tp);
+        *O.f(F::INDIRECT, ri) = st4(R.indirect);
     }
+    if (R.m0.z > 0 || code == ST_BOUNCE) *O.f(F::DIRECT, ri) = st4(R.direct);
+    if (code == ST_NEE_MIS) *O.f(F::LS, ri) = st4(R.ls);
 }
 
 // The result of a path's ray in the results arrays, read when a step needs
@@ -130,17 +131,18 @@ struct QueueResult {
 
 // One shade step of the path whose record is R and whose ray's result is
 // `res`; R is updated in place for the ray the step makes.  The ray whose
-// result arrived is rebuilt from the path state, bit for bit as it was made:
-// a camera ray starts at the camera's eye (createRay, udpt.cl:236) along the
-// stored direction rd; a bounce ray at hp + nd * EPSILON along the pending
-// bounce direction nd (udpt.cl:766, 906, 945).
+// result arrived is rebuilt, bit for bit as it was made, from its direction
+// and the path state: a camera ray starts at the camera's eye (createRay,
+// udpt.cl:236), a bounce ray at hp + nd * EPSILON along the bounce direction
+// nd (udpt.cl:766, 906, 945).  (Sampled directions have w = 0, or are NaN in
+// every component; a specular one's w is kept, see Rec.)
 // `tab`: where the path's job and scene are found (JobTables or OneJob).
 template <bool CAP, int LM, typename TAB, typename RES>
 __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, const RES& res, Rec& R,
                                        const LdsScene& lds)
 {
-    const int4 m0 = R.m0, m1 = R.m1;
-    const int jid = m1.y;
+    const int4 m0 = R.m0;
+    const int jid = R.job;
     const DevJob& J = tab.job(jid);
     const yn_render_params& RP = J.p;
     const int sid = (m0.y >> SCENE_SHIFT) & 0xff;
@@ -156,9 +158,8 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
     int st = m0.y;
     int code = st & ST_MASK;
     uint32_t seed = (uint32_t)m0.x;
-    const int pix = m1.x;
-    const int slot = m1.z;
-    const bool cap_on = CAP && cap.prim_tri != nullptr && slot == 0;
+    const uint32_t pix = R.sample;      // in frame slot 0, the only one captured
+    const bool cap_on = CAP && cap.prim_tri != nullptr && pix < (uint32_t)(J.W * J.H);
 
     int vmat = m0.w;                    // material of the path's current vertex
     f4& hp = R.hp;
@@ -167,7 +168,6 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
     f4& tp = R.tp;
     f4& direct = R.direct;
     f4& indirect = R.indirect;
-    float nee_prob = __int_as_float(m1.w);
     bool v_dirty = false;
     int bounce = m0.z;
 
@@ -191,7 +191,7 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
             cap.prim_light[pix] = (htri < 0 && (st & F_LCAND)) ? 0 : -1;
             cap.prim_t[pix] = h.x;
         }
-        f4 d = rd;
+        f4 d = R.dir;
         if (htri < 0) {
             if (st & F_LCAND) {     // udpt.cl:440-446
                 const_color = dot(d, ld(L.normal)) < 0 ? mk(1, 1, 1, 1) : mk(0.1f, .1f, .1f, 1);
@@ -225,8 +225,8 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
             float4 h = res.hit();
             int htri = __float_as_int(h.y);
             Mat m = mat_of(vmat);
-            f4 nd = R.nd;
-            float4 bnc = st4(R.bnc);
+            f4 nd = R.dir;
+            if (m.spec) nd.w = R.b;
             if (htri < 0) {
                 if ((st & F_LCAND) && m.spec) indirect = indirect + tp * ld(L.ke);
                 step = S_FINISH;
@@ -237,10 +237,10 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
                 const int nmat = tri_material(S.tri_shade, htri);
                 Mat nm = mat_of(nmat);
                 indirect = indirect + tp * nm.ke;
-                if (m.spec) tp = tp * bnc.z;
+                if (m.spec) tp = tp * R.a;
                 else
-                    tp = ((tp * eval_brdf(m, nd, -rd, hp, hn, (st & F_BGLOSSY) != 0, bnc.y, on, false)) *
-                          fmaxf(dot(nd, hn), 0.0f)) / bnc.x;
+                    tp = ((tp * eval_brdf(m, nd, -rd, hp, hn, (st & F_BGLOSSY) != 0, R.b, on, false)) *
+                          fmaxf(dot(nd, hn), 0.0f)) / R.a;
                 step = S_NEE_START;
                 if (bounce > RP.rr_threshold) {    // udpt.cl:514-523
                     float pr = fminf(luminance(tp), 0.95f);
@@ -291,17 +291,17 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
             cap.shadow_d[pix] = make_float4(wi.x, wi.y, wi.z, 1.0f);
         }
         if (quad_hit(L, so, wi, len, tq)) { occ = 1; step = S_NEE_SHADOW; break; }
-        R.wi = mk(wi.x, wi.y, wi.z, lpdf);
-        nee_prob = nprob;
+        R.a = lpdf;
+        R.b = nprob;
         st = (st & ~ST_MASK) | ST_NEE_SH;
         out = make_ray(2, so, wi, len, jid);
         goto steps_done;
     } while (0);
     if (step == S_NEE_SHADOW) do {  // udpt.cl:557-565 and the MIS light weight
         if (code == ST_NEE_SH) {
-            wi = mk(R.wi.x, R.wi.y, R.wi.z, 0.0f);
-            lpdf = R.wi.w;
-            nprob = nee_prob;
+            wi = R.dir;
+            lpdf = R.a;
+            nprob = R.b;
             code = ST_DONE;     // consumed
         }
         if (cap_on && (st & F_DIRECT) && !(st & F_CAPSH)) { cap.shadow_occ[pix] = occ; st |= F_CAPSH; }
@@ -329,9 +329,9 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
         if (!quad_hit(L, bo, bd, INFINITY, tq)) { nee_res = ls + em; step = S_NEE_DONE; break; }
         st = glossy ? (st | F_NGLOSSY) : (st & ~F_NGLOSSY);
         R.ls = ls;
-        R.mis = mk(bd.x, bd.y, bd.z, bpdf);
-        R.wi = mk(wi.x, wi.y, wi.z, lpdf);
-        nee_prob = nprob;
+        R.a = lpdf;
+        R.b = nprob;
+        R.c = bpdf;
         st = (st & ~ST_MASK) | ST_NEE_MIS;
         out = make_ray(2, bo, bd, tq, jid);
         goto steps_done;
@@ -341,10 +341,10 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
         em = m.ke;
         ls = R.ls;
         if (occ) { nee_res = ls + em; step = S_NEE_DONE; break; }
-        f4 bd = mk(R.mis.x, R.mis.y, R.mis.z, 0.0f);
-        float bpdf = R.mis.w;
-        lpdf = R.wi.w;
-        nprob = nee_prob;
+        f4 bd = R.dir;
+        float bpdf = R.c;
+        lpdf = R.a;
+        nprob = R.b;
         bool glossy = (st & F_NGLOSSY) != 0;
         float mw = power_heuristic(bpdf, lpdf, bpdf);
         f4 bs = (eval_brdf(m, bd, -rd, hp, hn, glossy, nprob, on, false) * ld(L.ke)) * fmaxf(dot(bd, hn), 0.0f);
@@ -377,28 +377,27 @@ __device__ __forceinline__ Out advance(const TAB& tab, const DevCapture& cap, co
         st &= ~F_LCAND;
         if (quad_hit(L, no, nd, INFINITY, tq)) { tmax = tq; st |= F_LCAND; }
         st = glossy ? (st | F_BGLOSSY) : (st & ~F_BGLOSSY);
-        R.nd = nd;
-        R.bnc = mk(pdf, bprob, ior, 0.0f);
+        R.a = m.spec ? ior : pdf;
+        R.b = m.spec ? nd.w : bprob;
         st = (st & ~ST_MASK) | ST_BOUNCE;
         out = make_ray(1, no, nd, tmax, jid);
         goto steps_done;
     } while (0);
     if (step == S_FINISH) do {
-        write_sample(J, slot, pix, direct + indirect);
+        write_sample(J, R.sample, direct + indirect);
         st = ST_DONE;
         ended = true;
         goto steps_done;
     } while (0);
-    if (step == S_FINISH_CONST) { write_sample(J, slot, pix, const_color); st = ST_DONE; ended = true; }
+    if (step == S_FINISH_CONST) { write_sample(J, R.sample, const_color); st = ST_DONE; ended = true; }
 steps_done:
     if (out.kind == 0 && !ended) {   // unreachable by construction; never leave a path hanging
-        write_sample(J, slot, pix, mk(NAN, NAN, NAN, NAN));
+        write_sample(J, R.sample, mk(NAN, NAN, NAN, NAN));
         st = ST_DONE;
     }
     out.done = out.kind == 0;
     out.job = jid;
     R.m0 = make_int4((int)seed, st, v_dirty ? bounce : m0.z, v_dirty ? vmat : m0.w);
-    R.m1 = make_int4(m1.x, m1.y, m1.z, __float_as_int(nee_prob));
     return out;
 }
 
