@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
                                    dp.y == dp.y && dp.z == dp.z);
             bool got = false;
             uint32_t node = 0;
-            bool go = !nan_ray && trav_start<2, false>(S, r, node, got, c);
+            bool go = !nan_ray && trav_start<2, false, LM == 1>(S, r, node, got, c);
             const float4 *nodes = S.nodes, *tri = S.tri_isect;
             if (__ballot(!fma_ok)) {
                 while (go) go = trav_step<4, 2, kPathsLds, BL, false, true>(nodes, tri, node, r, st, got, c);

@@ -263,7 +263,7 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
                     nodes = S.nodes;
                     tri = S.tri_isect;
                 }
-                if (live) live = trav_start<ANY, COUNT>(S, r, node, got, c);
+                if (live) live = trav_start<ANY, COUNT, SS>(S, r, node, got, c);
                 if (!live) store_hit<ANY>(a, pidx, r, got);
             }
         }
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(kRaysBlock, trace_waves<LST>()) void k_rays(RaysArg
                 // a ray with a NaN component hits nothing (see k_trace)
                 live = ot.x == ot.x && ot.y == ot.y && ot.z == ot.z && ot.w == ot.w && dp.x == dp.x &&
                        dp.y == dp.y && dp.z == dp.z;
-                if (live) live = trav_start<2, false>(S, r, node, got, c);
+                if (live) live = trav_start<2, false, true>(S, r, node, got, c);
                 if (!live) store_ray(a, ray, r, quad);
             }
         }

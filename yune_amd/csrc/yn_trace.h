@@ -78,14 +78,23 @@ __device__ __forceinline__ int4 gload(const int4* p)
     return make_int4(v.x, v.y, v.z, v.w);
 }
 
-// rayTriangleIntersection (udpt.cl:326-390) on a stored slot; xyz only
-// (the w terms of the reference's dots are exact zeros).  Returns whether
-// (u, v) lies in the triangle, with t; id: the triangle id.
-__device__ __forceinline__ bool tri_uvt(const float4* __restrict__ tri, int s, const RayState& r, float& t, float& u,
-                                        float& v, int& id)
+// The same address in every lane, as one the scalar unit loads from.
+typedef const __attribute__((address_space(4))) yn_v4f yn_cv4f;
+__device__ __forceinline__ yn_cv4f* scalar_ptr(const float4* p)
 {
-    float4 A = gload(tri + 3 * s), B = gload(tri + 3 * s + 1), C = gload(tri + 3 * s + 2);
-    id = __float_as_int(A.w);
+    const uint64_t u = (uint64_t)p;
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return (yn_cv4f*)(hi << 32 | lo);
+}
+
+// rayTriangleIntersection (udpt.cl:326-390) on a stored slot {A, B, C}; xyz
+// only (the w terms of the reference's dots are exact zeros).  Returns whether
+// (u, v) lies in the triangle, with t.
+template <typename V>
+__device__ __forceinline__ bool tri_uvt(const V& A, const V& B, const V& C, const RayState& r, float& t, float& u,
+                                        float& v)
+{
     // pvec = cross(dir, v1v3)
     float px = r.dy * C.z - r.dz * C.y;
     float py = r.dz * C.x - r.dx * C.z;
@@ -105,22 +114,27 @@ __device__ __forceinline__ bool tri_uvt(const float4* __restrict__ tri, int s, c
     return true;
 }
 
-template <int ANY>
-__device__ __forceinline__ bool tri_test(const float4* __restrict__ tri, int s, RayState& r)
+template <int ANY, typename V>
+__device__ __forceinline__ bool tri_test(const V& A, const V& B, const V& C, RayState& r)
 {
     float t, u, v;
-    int id;
-    if (tri_uvt(tri, s, r, t, u, v, id) && t > 0.0f && t < r.best) {
+    if (tri_uvt(A, B, C, r, t, u, v) && t > 0.0f && t < r.best) {
         if (ANY != 1) {         // an any-hit ray ends here, and only whether it hit counts
             r.best = t;
             r.cull = cull_of(t);
-            r.tri = id;
+            r.tri = __float_as_int(A.w);
             r.u = u;
             r.v = v;
         }
         return true;
     }
     return false;
+}
+
+template <int ANY>
+__device__ __forceinline__ bool tri_test(const float4* __restrict__ tri, int s, RayState& r)
+{
+    return tri_test<ANY>(gload(tri + 3 * s), gload(tri + 3 * s + 1), gload(tri + 3 * s + 2), r);
 }
 
 // The result record {t, triangle id bits, u, v} of a finished closest-hit
@@ -349,10 +363,42 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
 }
 
 
+// The hoisted triangles of one scene: boxes and triangles come through the
+// scalar unit, each box while the one before it is tested, instead of as
+// loads of one address by every lane.  Those were a tenth of a walk's loads
+// through the vector memory pipe, which bounds the walks of large trees, and
+// a chain of a dozen trips to memory before each of them: 32 frames of
+// 1920x1080 of a 1M-triangle room 72.9 -> 68.8 ms, 1280x720 of a 245k-triangle
+// room 1,955 -> 1,868 us, 16.8M paths of the Cornell box (4 hoisted) 12.9 ->
+// 12.5 ms, 8 bidirectional frames of 1280x720 of it 13.35 -> 12.49 ms, twelve
+// served jobs of three scenes 35.3 -> 33.5 ms.
+// Returns whether the walk ends here.
+template <int ANY, bool COUNT>
+__device__ __forceinline__ bool hoisted(yn_cv4f* hb, yn_cv4f* ht, int n, RayState& r, bool& got, Counts& c)
+{
+    if (n <= 0) return false;
+    yn_v4f lo = hb[0], hi = hb[1];
+    for (int s = 0; s < n; ++s) {
+        const int k = s + 1 < n ? s + 1 : s;
+        const yn_v4f nlo = hb[2 * k], nhi = hb[2 * k + 1];
+        float e;
+        if (box_hit(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, e) && !(e > r.cull)) {
+            if (COUNT) c.tris++;
+            const yn_v4f A = ht[3 * s], B = ht[3 * s + 1], C = ht[3 * s + 2];
+            got |= tri_test<ANY>(A, B, C, r);
+            if (ends<ANY>(r, got)) return true;
+        }
+        lo = nlo;
+        hi = nhi;
+    }
+    return false;
+}
+
 // The tests ahead of the tree, as in traverse(): every slot of a scene
 // without a BVH; the hoisted slots; a root that is one leaf.  Returns whether
-// the ray goes on to the tree, at `node`.
-template <int ANY, bool COUNT>
+// the ray goes on to the tree, at `node`.  UNI: every lane of the wave is in
+// the same scene.
+template <int ANY, bool COUNT, bool UNI>
 __device__ __forceinline__ bool trav_start(const DevScene& S, RayState& r, uint32_t& node, bool& got, Counts& c)
 {
     const float4* __restrict__ tri = S.tri_isect;
@@ -364,14 +410,19 @@ __device__ __forceinline__ bool trav_start(const DevScene& S, RayState& r, uint3
         }
         return false;
     }
-    for (int s = 0; s < S.n_hoist; ++s) {
-        float4 lo = gload(S.hoist_box + 2 * s), hi = gload(S.hoist_box + 2 * s + 1);
-        float e;
-        if (!box_hit(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, e) || e > r.cull)
-            continue;
-        if (COUNT) c.tris++;
-        got |= tri_test<ANY>(tri, s, r);
-        if (ends<ANY>(r, got)) return false;
+    if (UNI) {
+        if (hoisted<ANY, COUNT>(scalar_ptr(S.hoist_box), scalar_ptr(tri), __builtin_amdgcn_readfirstlane(S.n_hoist), r,
+                                got, c))
+            return false;
+    } else {
+        for (;;) {      // the wave's scenes one after the other
+            yn_cv4f* hb = scalar_ptr(S.hoist_box);
+            yn_cv4f* ht = scalar_ptr(tri);
+            const int n = __builtin_amdgcn_readfirstlane(S.n_hoist);
+            if ((uint64_t)ht != (uint64_t)tri) continue;
+            if (hoisted<ANY, COUNT>(hb, ht, n, r, got, c)) return false;
+            break;
+        }
     }
     node = S.root_ref;
     if (node == kEmptyRef) return false;
