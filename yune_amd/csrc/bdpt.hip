@@ -745,8 +745,10 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths_bdpt(Bdp
             bool go = !nan_ray && trav_start<2, false, LM == 1>(S, r, node, got, c);
             const float4 *nodes = S.nodes, *tri = S.tri_isect;
             if (__ballot(!fma_ok)) {
+                if (LM == 1 && go) go = trav_root<false, true>(nodes, node, r, st, c);
                 while (go) go = trav_step<4, 2, kPathsLds, BL, false, true>(nodes, tri, node, r, st, got, c);
             } else {
+                if (LM == 1 && go) go = trav_root<false, false>(nodes, node, r, st, c);
                 while (go) go = trav_step<4, 2, kPathsLds, BL, false, false>(nodes, tri, node, r, st, got, c);
             }
             if (ext) {

@@ -264,6 +264,10 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
                     tri = S.tri_isect;
                 }
                 if (live) live = trav_start<ANY, COUNT, SS>(S, r, node, got, c);
+                if (SS && W == 4 && live) {
+                    if (__ballot(exact)) live = trav_root<COUNT, true>(nodes, node, r, st, c);
+                    else live = trav_root<COUNT, false>(nodes, node, r, st, c);
+                }
                 if (!live) store_hit<ANY>(a, pidx, r, got);
             }
         }
@@ -389,6 +393,10 @@ __global__ __launch_bounds__(kRaysBlock, trace_waves<LST>()) void k_rays(RaysArg
                 live = ot.x == ot.x && ot.y == ot.y && ot.z == ot.z && ot.w == ot.w && dp.x == dp.x &&
                        dp.y == dp.y && dp.z == dp.z;
                 if (live) live = trav_start<2, false, true>(S, r, node, got, c);
+                if (W == 4 && live) {
+                    if (__ballot(exact)) live = trav_root<false, true>(nodes, node, r, st, c);
+                    else live = trav_root<false, false>(nodes, node, r, st, c);
+                }
                 if (!live) store_ray(a, ray, r, quad);
             }
         }
