@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
         any = !ext;
         ot = ext ? s.ext_in.o_t[qi] : s.sh_in.o_t[qi];
         dp = ext ? s.ext_in.d_p[qi] : s.sh_in.d_p[qi];
-        load_rec(s.in, ext ? qi : (uint32_t)(s.in.cap - 1 - (int64_t)qi), dp, R, ext && s.ext_primary);
+        load_rec<false>(s.in, ext ? qi : (uint32_t)(s.in.cap - 1 - (int64_t)qi), dp, R, ext && s.ext_primary);
     };
     if ((uint32_t)lane < per && wave * per + (uint32_t)lane < total) take(wave * per + (uint32_t)lane);
     unsigned long long n_rays[2] = {0, 0};          // closest-hit and any-hit, of the wave

@@ -87,21 +87,21 @@ __global__ __launch_bounds__(shade_block_pt(WAVES), WAVES) void k_shade_pt(Shade
         if (i < total) {
             const bool ext = i < n_ext;
             const uint32_t qi = ext ? i : i - n_ext;
-            const float4 dp = ext ? a.ext_in.d_p[qi] : a.sh_in.d_p[qi];
-            load_rec(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), dp, R, ext && a.ext_primary);
+            const float4 dp = nt_load(ext ? &a.ext_in.d_p[qi] : &a.sh_in.d_p[qi]);
+            load_rec<true>(a.in, ext ? qi : (uint32_t)(a.in.cap - 1 - (int64_t)qi), dp, R, ext && a.ext_primary);
             o = advance<CAP, LM>(JobTables{a.jobs, a.scenes}, cap, QueueResult{a.hit, a.occ, qi}, R, lds);
         }
         const uint32_t n[2] = {o.kind == 1 ? 1u : 0u, o.kind == 2 ? 1u : 0u};
         uint32_t at[2];
         block_reserve<2, BL>(rsv, par, ctr, n, at);
         if (o.kind == 1) {
-            a.ext_out.o_t[at[0]] = o.o_t;
-            a.ext_out.d_p[at[0]] = o.d_p;
+            nt_store(&a.ext_out.o_t[at[0]], o.o_t);
+            nt_store(&a.ext_out.d_p[at[0]], o.d_p);
             store_rec(a.out, at[0], R);
         }
         if (o.kind == 2) {
-            a.sh_out.o_t[at[1]] = o.o_t;
-            a.sh_out.d_p[at[1]] = o.d_p;
+            nt_store(&a.sh_out.o_t[at[1]], o.o_t);
+            nt_store(&a.sh_out.d_p[at[1]], o.d_p);
             store_rec(a.out, (uint32_t)(a.out.cap - 1 - (int64_t)at[1]), R);
         }
         if (a.done_ctr) {

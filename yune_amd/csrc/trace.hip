@@ -48,7 +48,7 @@ template <bool ANY>
 __device__ __forceinline__ void store_hit(const TraceArgs& a, int pidx, const RayState& r, bool got)
 {
     if (ANY) a.occ_out[pidx] = got ? 1 : 0;
-    else a.hit_out[pidx] = hit_record(r);
+    else nt_store(a.hit_out + pidx, hit_record(r));
 }
 
 template <int W, bool ANY, int LST, int BLOCK, bool COUNT>
@@ -244,8 +244,8 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
             if (all_static) more = false;            // nothing past the static rays
             const uint32_t i = base + (uint32_t)__popcll(idle & below);
             if (!live && i < lim) {
-                float4 ot = a.q.o_t[i];
-                float4 dp = a.q.d_p[i];
+                float4 ot = nt_load(a.q.o_t + i);
+                float4 dp = nt_load(a.q.d_p + i);
                 pidx = __float_as_int(dp.w);
                 int sc = SS ? ss
                             : a.single_scene >= 0 ? a.single_scene

@@ -9,6 +9,26 @@
 
 namespace yune {
 
+// Streamed memory: the wavefront's records, rays and results are written by
+// one launch and read once, by the next, gigabytes later.  Marked so, they
+// leave the caches to the tree and the triangles: 32 frames of 1920x1080 of a
+// 1M-triangle room 163.9 -> 160.5 ms, twelve served jobs 34.8 -> 34.3 ms, 64
+// frames of 512x512 of the Cornell box 12.41 -> 12.28 ms (the records alone:
+// 0.3%, 0.7% and 0.8%).  k_paths reads the few records it is handed plainly
+// (1280x720 of a 245k-triangle room 0.5% slower with them streamed).
+typedef float nt_v4f __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 nt_load(const float4* p)
+{
+    const nt_v4f v = __builtin_nontemporal_load((const __attribute__((address_space(1))) nt_v4f*)(const void*)p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void nt_store(float4* p, float4 v)
+{
+    const nt_v4f x = {v.x, v.y, v.z, v.w};
+    __builtin_nontemporal_store(x, (__attribute__((address_space(1))) nt_v4f*)(void*)p);
+}
+
+
 struct TraceArgs {
     const DevScene* scenes;     // scene table (device)
     const DevJob* jobs;         // job table (device)

@@ -64,28 +64,37 @@ __device__ __forceinline__ Out make_ray(int kind, f4 o, f4 d, float tmax, int jo
     return r;
 }
 
+template <bool NT>
+__device__ __forceinline__ float4 rec_load(const float4* p)
+{
+    if constexpr (NT) return nt_load(p);
+    else return *p;
+}
+
 // The record a step reads; dp: the pending ray's second half.  The shade pass
 // is bound by memory traffic, so a record holds nothing that the ray or the
 // state already says: the ray's direction and job are read from the queue, a
 // new path has no fields but M0, and the first vertex's constants (half of
 // all steps are there) are not stored.  What every later state uses is loaded
 // without waiting for the state, the rest once it is known.
+template <bool NT>
 __device__ __forceinline__ void load_rec(const PathRecs& I, uint32_t ri, float4 dp, Rec& R, bool primary)
 {
     using F = PathRecs;
-    R.m0 = *reinterpret_cast<const int4*>(I.f(F::M0, ri));
+    const float4 m0 = rec_load<NT>(I.f(F::M0, ri));
+    R.m0 = make_int4(__float_as_int(m0.x), __float_as_int(m0.y), __float_as_int(m0.z), __float_as_int(m0.w));
     R.dir = mk(dp.x, dp.y, dp.z, 0.0f);
     R.job = __float_as_int(dp.w);
     R.hp = R.hn = R.rd = R.direct = R.indirect = R.ls = mk(0, 0, 0, 0);
     R.tp = mk(1, 1, 1, 1);
     R.a = R.b = R.c = 0;
     if (!primary) {
-        const float4 m1 = *I.f(F::M1, ri);
+        const float4 m1 = rec_load<NT>(I.f(F::M1, ri));
         R.sample = __float_as_uint(m1.x);
         R.a = m1.y; R.b = m1.z; R.c = m1.w;
-        R.hp = ld(*I.f(F::HP, ri));
-        R.hn = ld(*I.f(F::HN, ri));
-        R.rd = ld(*I.f(F::RD, ri));
+        R.hp = ld(rec_load<NT>(I.f(F::HP, ri)));
+        R.hn = ld(rec_load<NT>(I.f(F::HN, ri)));
+        R.rd = ld(rec_load<NT>(I.f(F::RD, ri)));
     }
     const int code = R.m0.y & ST_MASK;
     if (code == ST_PRIMARY) {
@@ -93,11 +102,11 @@ __device__ __forceinline__ void load_rec(const PathRecs& I, uint32_t ri, float4 
         R.m0.z = 0;
     } else {
         if (R.m0.z > 0) {
-            R.tp = ld(*I.f(F::TP, ri));
-            R.indirect = ld(*I.f(F::INDIRECT, ri));
+            R.tp = ld(rec_load<NT>(I.f(F::TP, ri)));
+            R.indirect = ld(rec_load<NT>(I.f(F::INDIRECT, ri)));
         }
-        if (R.m0.z > 0 || code == ST_BOUNCE) R.direct = ld(*I.f(F::DIRECT, ri));
-        if (code == ST_NEE_MIS) R.ls = ld(*I.f(F::LS, ri));
+        if (R.m0.z > 0 || code == ST_BOUNCE) R.direct = ld(rec_load<NT>(I.f(F::DIRECT, ri)));
+        if (code == ST_NEE_MIS) R.ls = ld(rec_load<NT>(I.f(F::LS, ri)));
     }
 }
 
@@ -105,18 +114,19 @@ __device__ __forceinline__ void load_rec(const PathRecs& I, uint32_t ri, float4 
 __device__ __forceinline__ void store_rec(const PathRecs& O, uint32_t ri, const Rec& R)
 {
     using F = PathRecs;
-    *reinterpret_cast<int4*>(O.f(F::M0, ri)) = R.m0;
-    *O.f(F::M1, ri) = make_float4(__uint_as_float(R.sample), R.a, R.b, R.c);
-    *O.f(F::HP, ri) = st4(R.hp);
-    *O.f(F::HN, ri) = st4(R.hn);
-    *O.f(F::RD, ri) = st4(R.rd);
+    nt_store(O.f(F::M0, ri), make_float4(__int_as_float(R.m0.x), __int_as_float(R.m0.y), __int_as_float(R.m0.z),
+                                         __int_as_float(R.m0.w)));
+    nt_store(O.f(F::M1, ri), make_float4(__uint_as_float(R.sample), R.a, R.b, R.c));
+    nt_store(O.f(F::HP, ri), st4(R.hp));
+    nt_store(O.f(F::HN, ri), st4(R.hn));
+    nt_store(O.f(F::RD, ri), st4(R.rd));
     const int code = R.m0.y & ST_MASK;
     if (R.m0.z > 0) {
-        *O.f(F::TP, ri) = st4(R.tp);
-        *O.f(F::INDIRECT, ri) = st4(R.indirect);
+        nt_store(O.f(F::TP, ri), st4(R.tp));
+        nt_store(O.f(F::INDIRECT, ri), st4(R.indirect));
     }
-    if (R.m0.z > 0 || code == ST_BOUNCE) *O.f(F::DIRECT, ri) = st4(R.direct);
-    if (code == ST_NEE_MIS) *O.f(F::LS, ri) = st4(R.ls);
+    if (R.m0.z > 0 || code == ST_BOUNCE) nt_store(O.f(F::DIRECT, ri), st4(R.direct));
+    if (code == ST_NEE_MIS) nt_store(O.f(F::LS, ri), st4(R.ls));
 }
 
 // The result of a path's ray in the results arrays, read when a step needs
@@ -125,7 +135,7 @@ struct QueueResult {
     const float4* hit_at;
     const int32_t* occ_at;
     uint32_t i;
-    __device__ __forceinline__ float4 hit() const { return hit_at[i]; }
+    __device__ __forceinline__ float4 hit() const { return nt_load(hit_at + i); }
     __device__ __forceinline__ int occ() const { return occ_at[i]; }
 };
 
