@@ -422,6 +422,13 @@ def rows_for(res, summary):
         # result (closest hit 16 B, any hit 4 B)
         alg_ext = (cst.nodes_ext * node_b + cst.tris_ext * 48) / max(cst.rays_ext, 1) + 32 + 16
         alg_sh = (cst.nodes_shadow * node_b + cst.tris_shadow * 48) / max(cst.rays_shadow, 1) + 32 + 4
+    if d["trace_launches_ext"] == 0:
+        # each batch ran as one launch of whole paths and a resolve (1% of the
+        # step): the row's time is the step's
+        return [kernel_row("k_paths_bdpt" if bdpt else "k_paths", "ray", d["rays_ext"] + d["rays_shadow"], res["steps"],
+                           res["dt"] * 1e3, summary, "paths_bytes_per_ray", None, "paths")]
+    # the rays include those that k_paths ran to their ends after the
+    # wavefront's last iteration (a few per cent)
     return [
         kernel_row("k_trace_rf closest hit", "ray", d["rays_ext"], d["trace_launches_ext"], d["ms_trace_ext"],
                    summary, "trace_ext_bytes_per_ray", alg_ext, "trace_ext"),
