@@ -1,4 +1,4 @@
-// pt.hip — generate, shade, resolve and tonemap kernels of the wavefront
+// pt.hip — generate, shade and resolve kernels of the wavefront
 // unidirectional path tracer (kernels/legacy/udpt.cl semantics).
 //
 // The reference runs one path per work-item from camera ray to the end
