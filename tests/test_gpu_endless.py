@@ -1,0 +1,57 @@
+"""Paths that reach the bounce limit of a launch (k_paths) before they end."""
+import numpy as np
+import pytest
+
+import yune_amd as Y
+from mirror_box import mirror_box
+
+pytestmark = pytest.mark.gpu
+ENDLESS = dict(max_bounces=1 << 30, rr_threshold=1 << 30)
+
+
+def bits(a):
+    return np.asarray(a).view(np.int32)
+
+
+def test_frames_that_fail_leave_their_images():
+    """A frame with a path that does not end is an error, and what the image
+    held stays: samples that were never written are not folded into it."""
+    torch = pytest.importorskip("torch")
+    box, cornell = mirror_box(), Y.gen_cornell()
+    p, ok = Y.params_reference(**ENDLESS), Y.params_reference(mis=1, max_bounces=4)
+    with Y.Context(max_paths=1 << 12) as c:
+        a, b = c.scene(box), c.scene(cornell)
+
+        def good():                     # also leaves its samples in the buffer
+            j = c.job(b, cornell.cam, 16, 16, ok, base_seed=3)
+            j.render(2)
+            img = j.read()
+            j.release()
+            return img
+
+        first = good()
+        prev = torch.arange(2 * 3 * 4, dtype=torch.float32, device="cuda").reshape(2, 3, 4) + 5
+        out = torch.full_like(prev, -7)
+        torch.cuda.synchronize()
+        with pytest.raises(Y.YuneError):
+            c.pathtracer(out, prev, box.cam, a, 3, 2, p, 1, 0, 99)
+        assert np.array_equal(bits(out.cpu()), bits(prev.cpu()))
+        job = c.job(a, box.cam, 3, 2, p, base_seed=4)
+        with pytest.raises(Y.YuneError):
+            job.render(3)
+        assert not job.read().any()
+        assert np.array_equal(bits(good()), bits(first))
+
+
+def test_rounds_that_fail_leave_their_images():
+    box, cornell = mirror_box(), Y.gen_cornell()
+    with Y.Context(max_paths=1 << 12, serve_mode=1) as c:
+        a, b = c.scene(box), c.scene(cornell)
+        warm = c.job(b, cornell.cam, 16, 16, Y.params_reference(mis=1), base_seed=3)
+        warm.render(2)                  # samples in the buffer
+        fine = c.submit(b, cornell.cam, 8, 8, Y.params_reference(mis=1), 2, base_seed=5)
+        bad = c.submit(a, box.cam, 3, 2, Y.params_reference(**ENDLESS), 2, base_seed=5)
+        fine_was, bad_was = bits(fine.read()), bits(bad.read())
+        with pytest.raises(Y.YuneError):
+            c.serve(1)
+        assert np.array_equal(bits(fine.read()), fine_was) and np.array_equal(bits(bad.read()), bad_was)

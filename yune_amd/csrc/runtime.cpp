@@ -688,10 +688,12 @@ int enqueue_paths_bdpt(yn_ctx* c, const LoopCfg& L, const IterArgs& A, const Gen
     return 0;
 }
 
-// Folds a batch's samples into an image; the batch's last one also hands the
-// counters to the host and clears them.
+// Folds samples into an image.  BATCH, LAST: those of a batch, unless it
+// failed; the batch's last one also hands the counters to the host and clears
+// them.  STREAM: those of whole pieces of the continuous loop.
+enum class Fold { STREAM, BATCH, LAST };
 void resolve(yn_ctx* c, const DevJob& d, int x0, int y0, int w, int h, int frames, bool reset_first, float4* accum,
-             const float4* prev, bool last)
+             const float4* prev, Fold kind)
 {
     ResolveArgs ra{};
     ra.W = d.W;
@@ -705,8 +707,8 @@ void resolve(yn_ctx* c, const DevJob& d, int x0, int y0, int w, int h, int frame
     ra.reset_first = reset_first ? 1 : 0;
     ra.accum = accum;
     ra.prev = prev ? prev : accum;
-    ra.ctr = last ? c->ctr : nullptr;
-    ra.host = c->h_ctr;
+    ra.ctr = kind == Fold::STREAM ? nullptr : c->ctr;
+    ra.host = kind == Fold::LAST ? c->h_ctr : nullptr;
     launch_resolve(ra, c->stream);
 }
 
@@ -715,7 +717,7 @@ int finish_batch(yn_ctx* c, int64_t total, JobRec& stat_job)
 {
     HIPCK(c, hipGetLastError());
     HIPCK(c, hipStreamSynchronize(c->stream));
-    c->ctr_clear = true;
+    c->ctr_clear = c->h_ctr->q[6][0] == 0 && c->h_ctr->q[7][0] == 0;
     if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
     if (c->h_ctr->q[6][0]) return fail(c, YN_ERR_HIP, "paths did not end");
     stat_job.st.rays_ext += c->h_ctr->rays_ext;
@@ -752,8 +754,8 @@ int upload_jobs(yn_ctx* c, const std::vector<Region>& regs)
 // Runs one batch of primary-ray regions; samples land in samples[slot][pixel]
 // of each region's job (the sample buffer is shared: job slots are laid out
 // by the caller so regions do not overlap).  The last launches may still run
-// when it returns: the caller folds the samples (resolve, the last one with
-// `last`) and then calls finish_batch with *paths.
+// when it returns: the caller folds the samples (resolve, the last time with
+// Fold::LAST) and then calls finish_batch with *paths.
 int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, const DevCapture& cap, int64_t* paths)
 {
     std::vector<GenSeg> segs;
@@ -960,7 +962,7 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
             int64_t paths = 0;
             int r = run_batch(c, regs, J, cp, &paths);
             if (r) return r;
-            resolve(c, J.dev, x0, y0, w, h, nslots, reset_first && f == 0, accum, f == 0 ? prev : nullptr, true);
+            resolve(c, J.dev, x0, y0, w, h, nslots, reset_first && f == 0, accum, f == 0 ? prev : nullptr, Fold::LAST);
             if (int e = finish_batch(c, paths, J)) return e;
         } else {
             // image larger than the path capacity: row bands, one frame at a time
@@ -979,7 +981,7 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
                 int64_t paths = 0;
                 int r = run_batch(c, regs, J, cp, &paths);
                 if (r) return r;
-                resolve(c, J.dev, x0, yb, w, hh, 1, reset_first && f == 0, accum, f == 0 ? prev : nullptr, true);
+                resolve(c, J.dev, x0, yb, w, hh, 1, reset_first && f == 0, accum, f == 0 ? prev : nullptr, Fold::LAST);
                 if (int e = finish_batch(c, paths, J)) return e;
             }
         }
@@ -1103,7 +1105,8 @@ int serve_round(yn_ctx* c, int* frames_out)
     if (int r = run_batch(c, regs, c->serve_rec, DevCapture{}, &paths)) return r;
     for (const Plan& pl : plan) {
         JobRec& J = c->jobs[pl.jid];
-        resolve(c, J.dev, 0, 0, J.W, J.H, pl.k, pl.reset, J.accum, nullptr, &pl == &plan.back());
+        resolve(c, J.dev, 0, 0, J.W, J.H, pl.k, pl.reset, J.accum, nullptr,
+                &pl == &plan.back() ? Fold::LAST : Fold::BATCH);
     }
     if (int r = finish_batch(c, paths, c->serve_rec)) return r;
     double now = ms_since(c);
@@ -1325,7 +1328,7 @@ int stream_fold(yn_ctx* c)
                 if ((int64_t)J.frame != P.f0) continue;      // an earlier piece of the job is not folded yet
                 DevJob d = make_devjob(J);
                 d.samples = c->samples + P.soff;
-                resolve(c, d, 0, 0, J.W, J.H, P.k, P.f0 == 0, J.accum, nullptr, false);
+                resolve(c, d, 0, 0, J.W, J.H, P.k, P.f0 == 0, J.accum, nullptr, Fold::STREAM);
                 J.frame += (uint64_t)P.k;
                 J.st.frames += (uint64_t)P.k;
                 J.st.samples += (uint64_t)P.items;
@@ -2247,8 +2250,15 @@ int yn_pathtracer(yn_ctx* c, float* out_img, const float* in_img, const yn_cam* 
     J = JobRec();
     J.scene = sid; J.cam = *cam; J.W = W; J.H = H; J.p = *params; J.p.gi = gi_check;
     std::vector<uint32_t> seeds(1, rand);
-    return render_rect(c, jid, (float4*)out_img, x0, y0, w, h, seeds, reset != 0, DevCapture{},
-                       reset ? nullptr : (const float4*)in_img);
+    const int r = render_rect(c, jid, (float4*)out_img, x0, y0, w, h, seeds, reset != 0, DevCapture{},
+                              reset ? nullptr : (const float4*)in_img);
+    if (r && !reset && in_img != out_img) {     // the tile's image is then the one before the frame
+        const size_t at = 4 * ((size_t)y0 * W + x0);
+        HIPCK(c, hipMemcpy2DAsync(out_img + at, (size_t)W * 16, in_img + at, (size_t)W * 16, (size_t)w * 16, (size_t)h,
+                                  hipMemcpyDeviceToDevice, c->stream));
+        HIPCK(c, hipStreamSynchronize(c->stream));
+    }
+    return r;
 }
 
 int yn_tonemap_op(yn_ctx* c, const float* in_img, float* out_img, int32_t W, int32_t H, int32_t op)

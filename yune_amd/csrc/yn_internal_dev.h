@@ -253,13 +253,13 @@ __device__ __forceinline__ GenSeg seg_of(const GenArgs& a, int item)
     return g;
 }
 
-// Clears every counter (one wave calls it).
+// Clears every counter but the error flags q[6] and q[7] (one wave calls it).
 __device__ __forceinline__ void clear_counters(DevCounters* c)
 {
     const int i = (int)__lane_id();
     unsigned long long* h = &c->rays_ext;
     if (i < 6) h[i] = 0;
-    if (i < 12) c->q[i][0] = 0;
+    if (i < 12 && i != 6 && i != 7) c->q[i][0] = 0;
     if (i < 2 * kMaxXcd) c->work[i / kMaxXcd][i % kMaxXcd][0] = 0;
 }
 
@@ -286,8 +286,8 @@ struct ResolveArgs {
     int32_t reset_first;        // first frame of the batch overwrites (kernel arg 9)
     float4* accum;              // the job's RGBA32F image, .w = count
     const float4* prev;         // the image before the first frame (kernel arg 1; accum itself for a job)
-    DevCounters* ctr;           // not null: the batch's counters go to `host` (pinned) and are cleared
-    DevCounters* host;
+    DevCounters* ctr;           // not null: the batch's counters; with an error flag up the image stays as it is
+    DevCounters* host;          // not null: the counters go there (pinned) and are cleared, but for the flags
 };
 
 // Capture of the first frame for hit-ID parity (null pointers: off).
