@@ -55,3 +55,50 @@ def test_rounds_that_fail_leave_their_images():
         with pytest.raises(Y.YuneError):
             c.serve(1)
         assert np.array_equal(bits(fine.read()), fine_was) and np.array_equal(bits(bad.read()), bad_was)
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+def test_an_endless_job_is_served_beside_others(graph):
+    """Continuous serving: a job whose paths do not end stays pending, and
+    the others are rendered as if it were not there: one with paths of several
+    launches, small ones, and, submitted later, one of more work than fits
+    (so that the wavefront goes on with the endless paths in it)."""
+    box, cornell = mirror_box(), Y.gen_cornell()
+    ok = Y.params_reference(mis=1)
+    specs = [(0, 3, 2, Y.params_reference(**ENDLESS), 2), (0, 5, 3, Y.params_reference(max_bounces=3000, rr_threshold=1 << 30), 2),
+             (1, 16, 12, ok, 3), (1, 64, 64, ok, 5), (0, 7, 1, Y.params_reference(max_bounces=511, rr_threshold=1 << 30), 1),
+             (1, 9, 9, ok, 1)]
+    got = []
+    with Y.Context(max_paths=1 << 12, serve_mode=0, graph=graph) as c:
+        sids = [c.scene(box), c.scene(cornell)]
+        cams = [box.cam, cornell.cam]
+        jobs = []
+
+        def submit(k):
+            scene, w, h, p, frames = specs[k]
+            jobs.append(c.submit(sids[scene], cams[scene], w, h, p, frames, 11 + k))
+
+        def serve():
+            for _ in range(4000):
+                if c.serve(1) == 1:
+                    return
+            raise AssertionError("the other jobs did not end")
+
+        for k in (0, 1, 2):
+            submit(k)
+        serve()
+        for k in (3, 4):
+            submit(k)
+        serve()
+        submit(5)
+        serve()
+        assert not jobs[0].status()["done"]
+        got = [bits(j.read()) for j in jobs]
+    with Y.Context(max_paths=1 << 14) as c:
+        sids = [c.scene(box), c.scene(cornell)]
+        for k, (scene, w, h, p, frames) in enumerate(specs):
+            if k:
+                alone = c.job(sids[scene], cams[scene], w, h, p, base_seed=11 + k)
+                alone.set_counting(True)        # in the wavefront
+                alone.render(frames)
+                assert np.array_equal(got[k], bits(alone.read())), k

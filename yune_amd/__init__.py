@@ -266,8 +266,8 @@ class Context:
 
     def serve(self, max_rounds: int = 1) -> int:
         """Run up to max_rounds scheduler steps (serve_mode 0: groups of four
-        bounce iterations of the continuous loop, or its last paths to their
-        ends; 1: rounds); returns the jobs still pending."""
+        bounce iterations of the continuous loop, or its last paths for up to
+        512 bounces; 1: rounds); returns the jobs still pending."""
         pend = C.c_int32()
         self._ck(lib().yn_serve(self._p, max_rounds, C.byref(pend)))
         return pend.value

@@ -54,8 +54,8 @@ __device__ __forceinline__ auto tables_of(const PathsArgs& a)
 
 }  // namespace
 
-// ONE: all paths of one job (LM 1).
-template <int LM, bool ONE>
+// ONE: all paths of one job (LM 1).  PARK: see PathsArgs::parked.
+template <int LM, bool ONE, bool PARK>
 __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArgs a)
 {
     constexpr int BL = kPathsBlock;
@@ -144,7 +144,16 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
             dp = o.d_p;
             any = o.kind == 2;
             live = o.kind != 0;
-            if (live && R.m0.z >= kMaxPathBounces) {
+            if constexpr (PARK) {   // once in every stretch: a bounce has one closest-hit ray
+                if (o.kind == 1 && (R.m0.z & (kParkBounces - 1)) == kParkBounces - 1) {
+                    const uint32_t at = atomicAdd(a.parked, 1u);
+                    s.ext_out.o_t[at] = ot;
+                    s.ext_out.d_p[at] = dp;
+                    store_rec(s.out, at, R);
+                    atomicAdd(a.left + (R.job - s.done_base), 1u);
+                    live = false;
+                }
+            } else if (live && R.m0.z >= kMaxPathBounces) {
                 *a.endless = 1;
                 live = false;
             }
@@ -154,10 +163,13 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
             if (idle) {
                 uint32_t b = 0;
                 // after an endless path no more are taken
-                if (lane == 0)
+                if constexpr (PARK) {
+                    if (lane == 0) b = n_waves * per + atomicAdd(a.next, (uint32_t)__popcll(idle));
+                } else if (lane == 0) {
                     b = __hip_atomic_load(a.endless, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                             ? total
                             : n_waves * per + atomicAdd(a.next, (uint32_t)__popcll(idle));
+                }
                 b = __shfl(b, 0);
                 if (b >= total) more = false;
                 const uint32_t i = b + (uint32_t)__popcll(idle & below);
@@ -172,10 +184,17 @@ __global__ __launch_bounds__(kPathsBlock, paths_waves(LM)) void k_paths(PathsArg
 void launch_paths(const PathsArgs& a, int grid, hipStream_t stream)
 {
     const int lm = a.s.lmats != nullptr && a.s.n_lmats <= kLdsMats ? a.s.lmode : 0;
-    if (lm == 1 && a.one) hipLaunchKernelGGL((k_paths<1, true>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
-    else if (lm == 1) hipLaunchKernelGGL((k_paths<1, false>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
-    else if (lm == 2) hipLaunchKernelGGL((k_paths<2, false>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
-    else hipLaunchKernelGGL((k_paths<0, false>), dim3(grid), dim3(kPathsBlock), 0, stream, a);
+    const dim3 g(grid), b(kPathsBlock);
+    if (a.parked) {
+        if (lm == 1) hipLaunchKernelGGL((k_paths<1, false, true>), g, b, 0, stream, a);
+        else if (lm == 2) hipLaunchKernelGGL((k_paths<2, false, true>), g, b, 0, stream, a);
+        else hipLaunchKernelGGL((k_paths<0, false, true>), g, b, 0, stream, a);
+    } else {
+        if (lm == 1 && a.one) hipLaunchKernelGGL((k_paths<1, true, false>), g, b, 0, stream, a);
+        else if (lm == 1) hipLaunchKernelGGL((k_paths<1, false, false>), g, b, 0, stream, a);
+        else if (lm == 2) hipLaunchKernelGGL((k_paths<2, false, false>), g, b, 0, stream, a);
+        else hipLaunchKernelGGL((k_paths<0, false, false>), g, b, 0, stream, a);
+    }
 }
 
 }  // namespace yune

@@ -115,6 +115,7 @@ struct StreamState {
     std::map<int64_t, int64_t> sfree; // free ranges of the samples buffer: offset -> length
     int64_t live = 0;                 // paths in flight at the last sync
     unsigned long long last[6] = {0, 0, 0, 0, 0, 0};   // device statistics at the last sync
+    int64_t steps = 0;                // groups of four iterations, or bounces of k_paths by fours
     std::vector<GenSeg> segs;         // the last refill's segments (kept until it ran)
 };
 
@@ -172,7 +173,7 @@ struct yn_ctx {
     int64_t batch_paths = 0;          // paths per wavefront batch (0: the whole capacity)
     void* na_scratch = nullptr;       // device address of yn_trace_noalloc's static array on this device
     StreamState strm;                 // continuous serving
-    uint32_t* done_ctr = nullptr;     // per piece: paths ended (device)
+    uint32_t* done_ctr = nullptr;     // per piece: paths ended (device); from kMaxPieces on: paths parked
     uint32_t* h_done = nullptr;       // pinned mirror
     float* h_rays = nullptr;          // pinned: rays and results of small yn_trace calls
     uint32_t* h_full = nullptr;       // pinned: stack overflow flag of caller rays
@@ -647,14 +648,19 @@ void one_job(const yn_ctx* c, const LoopCfg& L, A& a)
 }
 
 // Enqueues k_paths on the rays of the queues that A's shade reads: their
-// paths run to their ends in one launch.
-int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary)
+// paths run to their ends in one launch.  park: or to the closest-hit queue
+// that A's shade would fill (see PathsArgs::parked).
+int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary, bool park = false)
 {
     PathsArgs pa{};
     pa.s = A.sa;
     pa.s.ext_primary = primary ? 1 : 0;
     pa.next = &c->ctr->work[0][0][0];
     pa.endless = &c->ctr->q[6][0];
+    if (park) {
+        pa.parked = &c->ctr->q[4][0];
+        pa.left = c->done_ctr + kMaxPieces;
+    }
     one_job(c, L, pa);
     // the blocks that fit at once
     const int grid = c->n_cu * paths_waves(pa.s.lmode);
@@ -781,7 +787,7 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     const DevScene* scenes = c->d_scenes;
     auto q = [&](int k) { return &c->ctr->q[k][0]; };
     // counters (q(k) = q[k][0]): q[0],q[1] extension queue counts, q[2],q[3] shadow queue
-    // counts, q[6] endless-path flag (k_paths), q[7] stack overflow flag, q[8],q[9] path-list counts
+    // counts, q[4] parked paths (k_paths), q[6] endless-path flag (k_paths), q[7] stack overflow flag, q[8],q[9] path-list counts
     // (bidirectional mode), q[10] free slots (regeneration), q[11] where a
     // regeneration's rays start in their queue; work[0], work[1]
     // the chunk counters of the extend / shadow traces, per queue slice.
@@ -1343,15 +1349,49 @@ int stream_fold(yn_ctx* c)
     return 0;
 }
 
-// One group of four bounce iterations of the persistent wavefront (or the
-// last paths to their ends), with admission, planning and refill before it
-// and folding after it.  `plan`
+// After a launch of k_paths over all paths in flight (everything planned was
+// issued): the paths it parked are the wavefront now, and what has none of
+// them is whole.
+int stream_settle(yn_ctx* c)
+{
+    StreamState& S = c->strm;
+    const uint32_t parked = c->h_ctr->q[4][0];
+    S.live = parked;
+    if (parked == 0) {      // all are folded, and the next work starts a new wavefront
+        for (int i = 0; i < kMaxPieces; ++i)
+            if (S.pieces[i].live) S.pieces[i].done = true;
+        S.active = false;
+        return stream_fold(c);
+    }
+    hipStream_t s = c->stream;
+    const size_t half = sizeof(uint32_t) * kMaxPieces;
+    HIPCK(c, hipMemcpyAsync(c->h_done + kMaxPieces, c->done_ctr + kMaxPieces, half, hipMemcpyDeviceToHost, s));
+    HIPCK(c, hipStreamSynchronize(s));
+    for (int i = 0; i < kMaxPieces; ++i) {
+        const Piece& P = S.pieces[i];
+        c->h_done[i] = P.live ? (uint32_t)P.items - c->h_done[kMaxPieces + i] : 0u;
+        c->h_done[kMaxPieces + i] = 0;
+    }
+    HIPCK(c, hipMemcpyAsync(c->done_ctr, c->h_done, 2 * half, hipMemcpyHostToDevice, s));
+    ++S.it;
+    c->h_ctr->q[S.it & 1][0] = parked;
+    c->h_ctr->q[2 + (S.it & 1)][0] = 0;
+    c->h_ctr->q[4][0] = 0;
+    HIPCK(c, hipMemcpyAsync(&c->ctr->q, &c->h_ctr->q, sizeof c->ctr->q, hipMemcpyHostToDevice, s));
+    HIPCK(c, hipMemsetAsync(&c->ctr->work, 0, sizeof c->ctr->work, s));     // the launch's path counter
+    return stream_fold(c);
+}
+
+// One group of four bounce iterations of the persistent wavefront (or, for
+// the last paths, kParkBounces bounces and mostly their ends), with
+// admission, planning and refill before it and folding after it.  `plan`
 // false: no new pieces (the loop drains).  *ran: whether any path was in
 // flight.
 int stream_group(yn_ctx* c, bool plan, bool* ran)
 {
     StreamState& S = c->strm;
     *ran = false;
+    ++S.steps;
     const auto h0 = std::chrono::steady_clock::now();
     if (!S.active)
         if (int r = stream_start(c)) return r;
@@ -1384,16 +1424,19 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
     // rays.  2 / 4 / 6 / 12 small jobs 1.69 / 3.38 / 6.03 / 11.2 ms -> 0.75 /
     // 1.02 / 2.91 / 8.6 ms; 12 jobs of 17.8M paths 38.8 / 38.1 / 37.6 / 37.6
     // / 38.4 / 41.9 ms with this limit at 0 / 2 / 4 / 8 / 12 / 17M.  What is
-    // submitted meanwhile waits for it, at most as long as 8M paths take.
+    // submitted meanwhile waits for it, at most as long as 8M paths take for
+    // kParkBounces bounces.
     const bool last = S.issue.empty() && S.live <= kPathsTail && paths_fit(L, false);
+    const int it0 = S.it;
     if (last) {
-        if (int r = enqueue_paths(c, L, iters[S.it & 1], false)) return r;
-    } else if (c->cfg.graph) {     // a group starts at queue parity 0 (four iterations per group)
+        S.steps += kParkBounces / 4 - 1;
+        if (int r = enqueue_paths(c, L, iters[S.it & 1], false, true)) return r;
+    } else if (c->cfg.graph && !(S.it & 1)) {     // a graph's group starts at queue parity 0
         if (int r = ensure_group_graph(c, L, iters, 4)) return r;
         HIPCK(c, hipGraphLaunch(c->gexec, c->stream));
         S.it += 4;
-    } else {
-        for (int g = 0; g < 4; ++g, ++S.it)
+    } else {        // three iterations after parked paths, so that the next group starts there
+        for (int g = S.it & 1; g < 4; ++g, ++S.it)
             if (int r = enqueue_iter(c, L, iters[S.it & 1], DevCapture{}, &spans)) return r;
     }
     hipStream_t s = c->stream;
@@ -1403,7 +1446,6 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
     HIPCK(c, hipStreamSynchronize(s));
     *ran = true;
     if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
-    if (c->h_ctr->q[6][0]) return fail(c, YN_ERR_HIP, "paths did not end");
     yn_stats& st = c->serve_rec.st;
     add_spans(spans, st);
     const unsigned long long now[6] = {c->h_ctr->rays_ext, c->h_ctr->rays_shadow, c->h_ctr->nodes_ext,
@@ -1415,16 +1457,10 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
     st.nodes_shadow += now[4] - S.last[4];
     st.tris_shadow += now[5] - S.last[5];
     for (int k = 0; k < 6; ++k) S.last[k] = now[k];
-    if (last) {     // every piece is whole: all are folded, and the next work starts a new wavefront
-        for (int i = 0; i < kMaxPieces; ++i)
-            if (S.pieces[i].live) S.pieces[i].done = true;
-        S.live = 0;
-        S.active = false;
-        return stream_fold(c);
-    }
-    st.iterations += 4;
-    st.trace_launches_ext += 4;
-    st.trace_launches_shadow += 4;
+    if (last) return stream_settle(c);
+    st.iterations += (uint64_t)(S.it - it0);
+    st.trace_launches_ext += (uint64_t)(S.it - it0);
+    st.trace_launches_shadow += (uint64_t)(S.it - it0);
     // every path in flight has one ray in the queues the next iteration reads
     S.live = (int64_t)c->h_ctr->q[S.it & 1][0] + c->h_ctr->q[2 + (S.it & 1)][0];
     return stream_fold(c);
@@ -1435,8 +1471,8 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
 // wavefront buffers.
 int stream_drain(yn_ctx* c)
 {
-    for (int guard = 0; c->strm.active; ++guard) {
-        if (guard > 1000000) return fail(c, YN_ERR_HIP, "continuous loop did not drain");
+    for (const int64_t s0 = c->strm.steps; c->strm.active;) {
+        if (c->strm.steps - s0 > 1000000) return fail(c, YN_ERR_HIP, "continuous loop did not drain");
         // items not yet issued stay with their pieces; finish them too
         bool ran = false;
         if (int r = stream_group(c, false, &ran)) return r;
@@ -1681,15 +1717,18 @@ int yn_create(const yn_config* cfg, yn_ctx** out)
     c->scenes.resize(kMaxScenes);
     c->jobs.resize(kMaxJobs);
     if ((r = dalloc(c, &c->d_scenes, kMaxScenes)) || (r = dalloc(c, &c->d_jobs, kMaxJobs + kMaxPieces)) ||
-        (r = dalloc(c, &c->ctr, 1)) || (r = dalloc(c, &c->done_ctr, kMaxPieces))) {
+        (r = dalloc(c, &c->ctr, 1)) || (r = dalloc(c, &c->done_ctr, 2 * kMaxPieces))) {
         g_err = c->err; return bail(r);
     }
     c->allocs.push_back(c->d_scenes);
     c->allocs.push_back(c->d_jobs);
     c->allocs.push_back(c->ctr);
     c->allocs.push_back(c->done_ctr);
+    if (hipMemset(c->done_ctr, 0, sizeof(uint32_t) * 2 * kMaxPieces) != hipSuccess) {
+        g_err = "hipMemset failed"; return bail(YN_ERR_HIP);
+    }
     if (hipHostMalloc((void**)&c->h_ctr, sizeof(DevCounters), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_done, sizeof(uint32_t) * kMaxPieces, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_done, sizeof(uint32_t) * 2 * kMaxPieces, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&c->h_rays, (size_t)kRaysHost * 44, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&c->h_full, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         g_err = "hipHostMalloc failed"; return bail(YN_ERR_HIP);
