@@ -292,8 +292,7 @@ int  yn_trace(yn_ctx* ctx, int32_t scene_id, const float* rays, int32_t n,
  * device array per GPU (35,663,104 bytes, held until the process ends),
  * whose address the context takes at creation.  Every call on a GPU shares
  * that array, so calls that overlap on one GPU (two contexts, two threads)
- * race.  A
- * traversal deeper than the array's stack (the LDS part plus 32 entries)
+ * race.  A traversal deeper than 32 entries beyond cfg.lds_stack (16 if 0)
  * fails with YN_ERR_INVALID.  Synchronous on the context's stream, like
  * yn_trace, and bit-identical to it. ---- */
 #define YN_TRACE_NOALLOC_MAX_RAYS 262144

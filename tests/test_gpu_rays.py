@@ -101,3 +101,26 @@ def test_traversal_beyond_the_fixed_stack_is_refused():
         assert call(a) == -2
         assert call(b) == 0
         assert same([o.cpu().numpy() for o in out], c.trace(b, rays))
+
+
+@pytest.mark.parametrize("lds,fits,deep", [(32, 60, 80), (16, 44, 60), (12, 40, 60), (8, 36, 60), (0, 44, 60)])
+def test_fixed_stack_for_every_lds_size(lds, fits, deep):
+    """yn_trace_noalloc takes traversals of 32 entries beyond the configured
+    LDS part, whatever of it the kernel keeps in LDS."""
+    torch = pytest.importorskip("torch")
+    from test_gpu_pt import comb_scene
+    rays = np.zeros((64, 8), np.float32)
+    rays[:, 0] = np.linspace(-0.01, 0.01, 64)
+    rays[:, 3] = np.inf
+    rays[:, 6] = -1.0
+    d = torch.from_numpy(rays).cuda()
+    out = [torch.zeros(64, dtype=t, device="cuda") for t in (torch.int32, torch.int32, torch.float32)]
+    torch.cuda.synchronize()
+    with Y.Context(bvh_width=2, max_paths=1 << 12, hoist_frac=-1, leaf_max=10, bvh_build=2, lds_stack=lds) as c:
+        for n, rc in ((fits, 0), (deep, -2)):
+            s = comb_scene(n)
+            sid = c.scene(s, s.nodes)
+            p = [C.c_void_p(o.data_ptr()) for o in out]
+            assert lib().yn_trace_noalloc(c._p, sid, C.c_void_p(d.data_ptr()), 64, *p) == rc, n
+            if rc == 0:
+                assert same([o.cpu().numpy() for o in out], c.trace(sid, rays))

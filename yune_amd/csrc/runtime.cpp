@@ -2404,7 +2404,7 @@ int yn_trace_noalloc(yn_ctx* c, int32_t sid, const float* rays, int32_t n, int32
     HIPCK(c, hipStreamSynchronize(s));
     if (*a.full)
         return fail(c, YN_ERR_INVALID, "traversal deeper than the no-allocation stack (" +
-                                           std::to_string(rays_lds_stack(lds) + kTraceNoAllocOvfDepth) +
+                                           std::to_string(trace_lds_stack(lds) + kTraceNoAllocOvfDepth) +
                                            " entries)");
     return 0;
 }

@@ -70,10 +70,11 @@ int trace_noalloc_enqueue(void* base, const RaysArgs& rays, int width, int lds, 
     a.ovf_ref = reinterpret_cast<uint32_t*>(b);
     a.ovf_t = reinterpret_cast<uint16_t*>(b + kOffOvfT);
     a.work = reinterpret_cast<uint32_t*>(b + kOffWork);
-    // as many entries per thread as the scene needs, kTraceNoAllocOvfDepth at
-    // most (a deeper traversal stops there and raises the overflow flag), and
-    // as many threads as then have room
-    a.ovf_depth = std::min(std::max(max_depth - rays_lds_stack(lds), 0), kTraceNoAllocOvfDepth);
+    // as many entries per thread as the scene needs, kTraceNoAllocOvfDepth
+    // beyond the configured LDS part at most (a deeper traversal stops there
+    // and raises the overflow flag), and as many threads as then have room
+    const int entries = std::min(max_depth, trace_lds_stack(lds) + kTraceNoAllocOvfDepth);
+    a.ovf_depth = std::max(entries - rays_lds_stack(lds), 0);
     const size_t threads = kOvfEntries / (size_t)std::max(a.ovf_depth, 1);
     const int grid = (int)std::min<size_t>((size_t)max_grid, threads / kRaysBlock);
     if ((int64_t)a.n > (int64_t)(grid / a.n_slices) * a.n_slices * kRaysBlock)

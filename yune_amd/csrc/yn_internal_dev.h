@@ -402,7 +402,7 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred)
 #endif
 
 // yn_trace_noalloc (trace_noalloc.hip): rays per call at most, and traversal
-// stack entries per ray beyond the LDS part at most.
+// stack entries per ray beyond the configured LDS part at most.
 constexpr int kTraceNoAllocMaxRays = YN_TRACE_NOALLOC_MAX_RAYS;
 constexpr int kTraceNoAllocOvfDepth = 32;
 int trace_noalloc_init(int device, void** ptr);
