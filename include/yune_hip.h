@@ -47,9 +47,11 @@ typedef struct yn_config {
     int32_t max_paths;        /* paths in flight per batch (0: default, 64M)        */
     size_t  mem_budget;       /* bytes for job buffers; 0: 64 GiB                   */
     int32_t bvh_width;        /* GPU node width 2 or 4 (0: 4)                       */
-    int32_t trace_block;      /* trace kernel block size 64/128/256 (0: 256)        */
+    int32_t trace_block;      /* trace kernel block size 64/128/256 (0: 256); a
+                                 caller's rays are always traced in blocks of 256  */
     int32_t trace_chunk;      /* rays per wave per queue fetch (0: 64)              */
-    int32_t trace_grid;       /* trace blocks per launch (0: the blocks that fit)  */
+    int32_t trace_grid;       /* trace blocks per launch (0: the blocks that fit);
+                                 yn_trace: blocks of 256 with as many threads      */
     float   hoist_frac;       /* triangles whose box area exceeds this fraction of the
                                  root box's are tested by every ray instead of living
                                  in the tree (0: 0.01; < 0: off)                    */

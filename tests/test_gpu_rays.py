@@ -124,3 +124,29 @@ def test_fixed_stack_for_every_lds_size(lds, fits, deep):
             assert lib().yn_trace_noalloc(c._p, sid, C.c_void_p(d.data_ptr()), 64, *p) == rc, n
             if rc == 0:
                 assert same([o.cpu().numpy() for o in out], c.trace(sid, rays))
+
+
+@pytest.mark.parametrize("opts", [dict(trace_grid=1), dict(trace_grid=7, trace_block=64, trace_xcd=16),
+                                  dict(trace_grid=20000)])
+def test_configured_grid(room, opts):
+    """Caller's rays keep to trace_grid blocks of trace_block threads: fewer
+    of them take longer, for the same results."""
+    import time
+
+    def timed(c, sid):
+        c.trace(sid, rays)
+        best = 1e9
+        for _ in range(3):
+            t0 = time.perf_counter()
+            r = c.trace(sid, rays)
+            best = min(best, time.perf_counter() - t0)
+        return r, best
+
+    rays = mixed_rays(60_001, 6)
+    with Y.Context(max_paths=1 << 16) as c:
+        want, t = timed(c, c.scene(room))
+    with Y.Context(max_paths=1 << 16, **opts) as c:
+        got, tc = timed(c, c.scene(room))
+    assert same(got, want)
+    if opts["trace_grid"] < 20:
+        assert tc > 4 * t               # at most 1,792 of 393,216 lanes

@@ -1599,8 +1599,9 @@ int build_scene(yn_ctx* c, int sid, int width)
     return 0;
 }
 
-// Caller's rays (k_rays): launches of the blocks that fit at once, so that a
-// call of few rays spreads them over every wave of the chip.
+// Caller's rays (k_rays, blocks of kRaysBlock): launches of the blocks that
+// fit at once, so that a call of few rays spreads them over every wave of the
+// chip.
 constexpr int kRaysHost = 8192;
 
 int rays_grid(const yn_ctx* c, int lds) { return c->n_cu * trace_resident_waves(rays_lds_stack(lds)); }
@@ -2335,7 +2336,9 @@ int yn_trace(yn_ctx* c, int32_t sid, const float* rays, int32_t n, int32_t* tri,
     hipStream_t s = c->stream;
     const SceneRec& S = c->scenes[sid];
     const int lds = lds_for(c, S.info.node_bytes);
-    const int grid = rays_grid(c, lds);
+    // a configured grid: as many threads as its blocks have
+    const int64_t threads = (int64_t)c->cfg.trace_grid * c->cfg.trace_block;
+    const int grid = c->cfg.trace_grid > 0 ? (int)((threads + kRaysBlock - 1) / kRaysBlock) : rays_grid(c, lds);
     RaysArgs a = rays_args(c, sid, n);
     // Up to kRaysHost rays the kernel reads and writes pinned host memory: a
     // copy command each way costs more than the few hundred kB over the bus.
