@@ -289,9 +289,9 @@ int  yn_trace(yn_ctx* ctx, int32_t scene_id, const float* rays, int32_t n,
  * allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  rays, tri, light and t are
  * DEVICE pointers in yn_trace's layouts; n <= YN_TRACE_NOALLOC_MAX_RAYS,
- * larger n is refused with YN_ERR_INVALID.  The call allocates nothing:
- * its traversal-stack overflow area and work counters live in one static
- * device array per GPU (35,663,104 bytes, held until the process ends),
+ * larger n is refused with YN_ERR_INVALID.  Results may be written over the
+ * rays.  The call allocates nothing: its traversal-stack overflow area, work
+ * counters and, then, a copy of the rays live in one static device array per GPU (35,663,104 bytes, held until the process ends),
  * whose address the context takes at creation.  Every call on a GPU shares
  * that array, so calls that overlap on one GPU (two contexts, two threads)
  * race.  A traversal deeper than 32 entries beyond cfg.lds_stack (16 if 0)

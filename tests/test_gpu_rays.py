@@ -150,3 +150,33 @@ def test_configured_grid(room, opts):
     assert same(got, want)
     if opts["trace_grid"] < 20:
         assert tc > 4 * t               # at most 1,792 of 393,216 lanes
+
+
+@pytest.mark.parametrize("shift", [0, 5, -5])
+@pytest.mark.parametrize("deep", [False, True])
+def test_results_over_the_device_rays(room, deep, shift):
+    """Results may be written where the rays lie: every ray is read first.
+    A deep tree's stacks leave room for fewer lanes than there are rays."""
+    torch = pytest.importorskip("torch")
+    from test_gpu_pt import comb_scene
+    n = 262_143
+    rays = mixed_rays(n, 12)
+    opts = dict(bvh_width=2, hoist_frac=-1, leaf_max=10, bvh_build=2, lds_stack=32) if deep else {}
+    s = comb_scene(80) if deep else room
+    if deep:                            # short ways through the comb, one triangle each
+        rng = np.random.default_rng(3)
+        i = rng.integers(0, 80, n)
+        rays[:, 0], rays[:, 1], rays[:, 2] = 0.0, -0.03, -1.0 - 0.1 * i + 0.05
+        rays[:, 3], rays[:, 7] = rng.uniform(0.01, 5.0, n), 0.0
+        rays[:, 4], rays[:, 5], rays[:, 6] = rng.uniform(-0.6, 0.6, n), 0.0, -1.0
+    with Y.Context(max_paths=1 << 18, **opts) as c:
+        sid = c.scene(s, s.nodes) if deep else c.scene(s)
+        want = c.trace(sid, rays)
+        assert not deep or 0.2 < (want[0] >= 0).mean() < 1.0
+        d = torch.zeros(n * 8 + 16, device="cuda")
+        d[8:8 + n * 8] = torch.from_numpy(rays.reshape(-1)).cuda()
+        torch.cuda.synchronize()
+        at = [d.data_ptr() + 4 * (8 + shift + k * n) for k in range(3)]
+        assert lib().yn_trace_noalloc(c._p, sid, C.c_void_p(d.data_ptr() + 32), n, *(C.c_void_p(a) for a in at)) == 0
+        got = [d[8 + shift + k * n:8 + shift + (k + 1) * n].cpu().numpy() for k in range(3)]
+        assert same(got, want)

@@ -3,8 +3,9 @@
 // (code under HIP graph capture, tight serving loops).
 //
 // What the call needs beyond the caller's inputs and outputs (the traversal
-// stack's overflow area and the work counters) lives in `scratch`, one static
-// device array per GPU.  Its device address is taken once per device with
+// stack's overflow area, the work counters and, where results are to be
+// written over the rays, the rays) lives in `scratch`, one static device array
+// per GPU.  Its device address is taken once per device with
 // hipGetSymbolAddress at context creation; host code only ever uses that
 // address, never the array's name (a host-side stand-in).  Every call on one
 // GPU shares the array: calls that overlap on one GPU race.
@@ -20,10 +21,17 @@ using namespace yune;
 constexpr size_t kScratchBytes = 35663104;
 // traversal stack overflow entries, 6 B each (a reference and a distance)
 constexpr size_t kWorkBytes = sizeof(uint32_t) * kMaxXcd * kWorkStride;
-constexpr size_t kOvfEntries = (kScratchBytes - kWorkBytes) / 6 / 256 * 256;
-constexpr size_t kOffOvfT = kOvfEntries * 4;
 constexpr size_t kOffWork = kScratchBytes - kWorkBytes;
-static_assert(kOffOvfT + kOvfEntries * 2 <= kOffWork && kOffWork % 256 == 0, "the scratch array's parts");
+static_assert(kOffWork % 256 == 0, "the scratch array's parts");
+
+// Overflow entries in `bytes` of the array.
+constexpr size_t ovf_entries(size_t bytes) { return bytes / 6 / 256 * 256; }
+
+// Whether two arrays share memory.
+bool overlap(const void* a, size_t na, const void* b, size_t nb)
+{
+    return (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
 
 }  // namespace
 
@@ -67,15 +75,27 @@ int trace_noalloc_enqueue(void* base, const RaysArgs& rays, int width, int lds, 
     if (rays.n == 0) return 0;
     uint8_t* b = static_cast<uint8_t*>(base);
     RaysArgs a = rays;
-    a.ovf_ref = reinterpret_cast<uint32_t*>(b);
-    a.ovf_t = reinterpret_cast<uint16_t*>(b + kOffOvfT);
+    // Results over the rays: the kernel writes a ray's while others are still
+    // to be read, so it reads a copy (8 MB at most).
+    const size_t n = (size_t)a.n;
+    size_t used = 0;
+    if (overlap(a.tri, 4 * n, a.rays, 32 * n) || overlap(a.light, 4 * n, a.rays, 32 * n) ||
+        overlap(a.t, 4 * n, a.rays, 32 * n)) {
+        used = (32 * n + 255) / 256 * 256;
+        if (hipMemcpyAsync(b, a.rays, 32 * n, hipMemcpyDeviceToDevice, s) != hipSuccess) return -1;
+        a.rays = reinterpret_cast<const float*>(b);
+        a.aligned = 1;
+    }
+    const size_t ovf = ovf_entries(kOffWork - used);
+    a.ovf_ref = reinterpret_cast<uint32_t*>(b + used);
+    a.ovf_t = reinterpret_cast<uint16_t*>(b + used + 4 * ovf);
     a.work = reinterpret_cast<uint32_t*>(b + kOffWork);
     // as many entries per thread as the scene needs, kTraceNoAllocOvfDepth
     // beyond the configured LDS part at most (a deeper traversal stops there
     // and raises the overflow flag), and as many threads as then have room
     const int entries = std::min(max_depth, trace_lds_stack(lds) + kTraceNoAllocOvfDepth);
     a.ovf_depth = std::max(entries - rays_lds_stack(lds), 0);
-    const size_t threads = kOvfEntries / (size_t)std::max(a.ovf_depth, 1);
+    const size_t threads = ovf / (size_t)std::max(a.ovf_depth, 1);
     const int grid = (int)std::min<size_t>((size_t)max_grid, threads / kRaysBlock);
     if ((int64_t)a.n > (int64_t)(grid / a.n_slices) * a.n_slices * kRaysBlock)
         hipLaunchKernelGGL(k_na_clear, dim3(1), dim3(64), 0, s, a.work);
