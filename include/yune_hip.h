@@ -254,8 +254,9 @@ double yn_clock_ms(yn_ctx* ctx);                     /* ms since yn_create */
  * the fastest BVH width (the scenes' GPU layout is rebuilt), trace block
  * size, rays per queue fetch, LDS stack depth, shade occupancy, paths
  * per batch, batch_factor, trace_overlap, graph, trace_xcd and trace_refill in
- * the context's configuration.  Not while
- * served jobs are pending.  yn_config_get reads the configuration in effect. ---- */
+ * the context's configuration; what governs the wavefront alone is timed in it,
+ * also when the view's own batches are small enough for whole-path launches.
+ * Not while served jobs are pending.  yn_config_get reads the configuration in effect. ---- */
 typedef struct yn_tune_result {
     int32_t bvh_width, trace_block, trace_chunk, lds_stack, shade_waves, n_tried;
     int64_t batch_paths;      /* paths in flight per batch                              */
@@ -291,10 +292,10 @@ int  yn_trace(yn_ctx* ctx, int32_t scene_id, const float* rays, int32_t n,
  * DEVICE pointers in yn_trace's layouts; n <= YN_TRACE_NOALLOC_MAX_RAYS,
  * larger n is refused with YN_ERR_INVALID.  Results may be written over the
  * rays.  The call allocates nothing: its traversal-stack overflow area, work
- * counters and, then, a copy of the rays live in one static device array per GPU (35,663,104 bytes, held until the process ends),
- * whose address the context takes at creation.  Every call on a GPU shares
- * that array, so calls that overlap on one GPU (two contexts, two threads)
- * race.  A traversal deeper than 32 entries beyond cfg.lds_stack (16 if 0)
+ * counters and, then, a copy of the rays live in one static device array per
+ * GPU (35,663,104 bytes, held until the process ends), whose address the
+ * context takes at creation.  Every call on a GPU shares that array, so calls
+ * that overlap on one GPU (two contexts, two threads) race.  A traversal deeper than 32 entries beyond cfg.lds_stack (16 if 0)
  * fails with YN_ERR_INVALID.  Synchronous on the context's stream, like
  * yn_trace, and bit-identical to it. ---- */
 #define YN_TRACE_NOALLOC_MAX_RAYS 262144

@@ -391,3 +391,15 @@ def test_batched_mix_matches_alone_and_oracle():
         err = float((np.abs(a - b).sum(-1) / np.maximum(np.abs(b).sum(-1), 1e-2)).mean())
         print(f"  job {k} (scene {sc}, {len(x.tris)} triangles): tile bit-identical {same:.4f}, mean rel err {err:.2e}")
         assert same >= 0.99 and err <= 0.01, (k, same, err)
+
+
+def test_autotune_measures_what_its_knobs_change():
+    """A view that runs in one launch of whole paths reads few of the knobs:
+    the others are measured where they count, so a poor setting (two shade
+    waves cost the wavefront a fifth and more) is left."""
+    s = Y.gen_cornell()
+    p = Y.params_reference(mis=1, max_bounces=8, rr_threshold=2)
+    with Y.Context(max_paths=1 << 20, shade_waves=2) as c:
+        r = c.autotune(c.scene(s), s.cam, 512, 512, p, frames=4)
+        assert r["shade_waves"] == 4 and c.config()["shade_waves"] == 4
+        assert r["bvh_width"] == 4

@@ -171,6 +171,7 @@ struct yn_ctx {
     int64_t submit_seq = 0;
     JobRec serve_rec;                 // statistics of scheduler rounds
     int64_t batch_paths = 0;          // paths per wavefront batch (0: the whole capacity)
+    bool wave_only = false;           // no whole-path launches (yn_autotune)
     void* na_scratch = nullptr;       // device address of yn_trace_noalloc's static array on this device
     StreamState strm;                 // continuous serving
     uint32_t* done_ctr = nullptr;     // per piece: paths ended (device); from kMaxPieces on: paths parked
@@ -627,7 +628,10 @@ bool bdpt_paths_win(int64_t paths, int vertices, size_t node_bytes)
 }
 
 // What whole-path launches need: width-4 trees, nothing counted or captured.
-bool paths_fit(const LoopCfg& L, bool capture) { return !L.count && L.width == 4 && !capture; }
+bool paths_fit(const yn_ctx* c, const LoopCfg& L, bool capture)
+{
+    return !c->wave_only && !L.count && L.width == 4 && !capture;
+}
 
 // The launch's one job and scene as kernel arguments, when it has one and the
 // scene's materials fit LDS.
@@ -810,7 +814,7 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     make_iter(c, L, 0, iters[0]);
     make_iter(c, L, 1, iters[1]);
     const bool any_cap = cap.prim_tri || cap.prim_light || cap.prim_t || cap.shadow_o || cap.shadow_d || cap.shadow_occ;
-    const bool paths_ok = paths_fit(L, any_cap);
+    const bool paths_ok = paths_fit(c, L, any_cap);
     bool direct = paths_ok && !regen && total <= kPathsDirect;
     if (bdpt) {
         int vertices = 0;
@@ -1426,7 +1430,7 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
     // / 38.4 / 41.9 ms with this limit at 0 / 2 / 4 / 8 / 12 / 17M.  What is
     // submitted meanwhile waits for it, at most as long as 8M paths take for
     // kParkBounces bounces.
-    const bool last = S.issue.empty() && S.live <= kPathsTail && paths_fit(L, false);
+    const bool last = S.issue.empty() && S.live <= kPathsTail && paths_fit(c, L, false);
     const int it0 = S.it;
     if (last) {
         S.steps += kParkBounces / 4 - 1;
@@ -2122,7 +2126,11 @@ int yn_config_get(yn_ctx* c, yn_config* out, int64_t* batch_paths)
 
 // Coordinate descent over the launch and layout knobs on short timed
 // renders of the caller's view: each knob in turn takes each of its values
-// with the others held, and keeps a value that is more than 1% faster.
+// with the others held, and keeps a value that is more than 1% faster.  The
+// tree's width and the batch size are timed as renders run (they also decide
+// what runs in whole-path launches), the others with the wavefront alone: a
+// view of few paths would otherwise run in one launch that reads none of
+// them, and the noise of its timings would choose.
 int yn_autotune(yn_ctx* c, int32_t sid, const yn_cam* cam, int32_t W, int32_t H, const yn_render_params* p,
                 int32_t frames, yn_tune_result* out)
 {
@@ -2137,10 +2145,11 @@ int yn_autotune(yn_ctx* c, int32_t sid, const yn_cam* cam, int32_t W, int32_t H,
         if (int r = stream_drain(c)) return r;
     int tried = 0;
     int err = 0;
-    auto measure = [&]() -> double {
+    auto measure = [&](bool wave) -> double {
         int32_t jid = -1;
         if ((err = yn_job_create(c, sid, cam, W, H, p, 0x9e3779b9u, &jid))) return -1.0;
         double rate = -1.0;
+        c->wave_only = wave;
         if (!(err = yn_job_render(c, jid, 1))) {
             yn_stats a = c->jobs[jid].st;
             auto t0 = std::chrono::steady_clock::now();
@@ -2150,6 +2159,7 @@ int yn_autotune(yn_ctx* c, int32_t sid, const yn_cam* cam, int32_t W, int32_t H,
                 rate = (double)((b.rays_ext - a.rays_ext) + (b.rays_shadow - a.rays_shadow)) / std::max(dt, 1e-9);
             }
         }
+        c->wave_only = false;
         yn_job_release(c, jid);
         ++tried;
         return rate;
@@ -2206,21 +2216,28 @@ int yn_autotune(yn_ctx* c, int32_t sid, const yn_cam* cam, int32_t W, int32_t H,
         default: c->cfg.trace_refill = (int)v; return 0;
         }
     };
-    double best = measure();
-    if (best < 0) return err ? err : fail(c, YN_ERR_HIP, "autotune: first render failed");
+    double best[2];             // as renders run, and in the wavefront alone
+    for (int w = 0; w < 2; ++w)
+        if ((best[w] = measure(w == 1)) < 0) return err ? err : fail(c, YN_ERR_HIP, "autotune: first render failed");
     for (int pass = 0; pass < 2; ++pass) {
         bool changed = false;
         for (const Knob& k : knobs) {
-            int64_t keep = get(k.kind);
+            const int w = k.kind == 0 || k.kind == 5 || k.kind == 6 ? 0 : 1;
+            const int64_t was = get(k.kind);
+            int64_t keep = was;
             for (int64_t v : k.vals) {
                 if (v == keep || v <= 0) continue;
                 if (int r = set(k.kind, v)) return r;
-                double m = measure();
+                double m = measure(w == 1);
                 if (m < 0) return err;
-                if (m > best * 1.01) { best = m; keep = v; changed = true; }
+                if (m > best[w] * 1.01) { best[w] = m; keep = v; }
             }
             if (get(k.kind) != keep)
                 if (int r = set(k.kind, keep)) return r;
+            if (keep != was) {
+                changed = true;
+                if ((best[1 - w] = measure(w == 0)) < 0) return err;
+            }
         }
         if (!changed) break;
     }
@@ -2235,7 +2252,7 @@ int yn_autotune(yn_ctx* c, int32_t sid, const yn_cam* cam, int32_t W, int32_t H,
     out->graph = c->cfg.graph;
     out->trace_xcd = c->cfg.trace_xcd;
     out->trace_refill = c->cfg.trace_refill;
-    out->mrays_per_s = best / 1e6;
+    out->mrays_per_s = best[0] / 1e6;
     out->n_tried = tried;
     return 0;
 }
