@@ -202,14 +202,20 @@ int  yn_job_set_tonemap(yn_ctx* ctx, int32_t job_id, int32_t op);
 int  yn_job_save(yn_ctx* ctx, int32_t job_id, const char* path);
 int  yn_job_release(yn_ctx* ctx, int32_t job_id);
 
+/* Batches small enough, and the last paths of larger ones, run in launches
+ * that trace and shade whole paths: their rays are counted, but they are no
+ * iterations and no trace launches, and their time is ms_other.  A rate per
+ * kernel needs a counting job, which runs in the wavefront alone. */
 typedef struct yn_stats {
     uint64_t frames, samples;
     uint64_t rays_ext, rays_shadow;       /* BVH queries (closest / any hit)      */
     uint64_t nodes_ext, tris_ext;         /* counting mode only: interior nodes    */
     uint64_t nodes_shadow, tris_shadow;   /* visited and triangles tested          */
-    uint64_t trace_launches_ext, trace_launches_shadow, iterations;
+    uint64_t trace_launches_ext, trace_launches_shadow, iterations;   /* the wavefront's */
     double   ms_total;                    /* wall time of yn_job_render calls      */
-    double   ms_trace_ext, ms_trace_shadow, ms_shade, ms_other;   /* HIP events */
+    double   ms_trace_ext, ms_trace_shadow, ms_shade;   /* the wavefront's launches, HIP events */
+    double   ms_other;                    /* whole-path launches: host time from the launch to
+                                             the end of the batch, its fold included */
     /* continuous serving (yn_serve_stats): groups of bounce iterations run,
      * the sum of the paths in flight at each group's start, refills, groups
      * whose planning stopped for want of samples-buffer room or piece

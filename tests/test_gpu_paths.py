@@ -133,3 +133,17 @@ def test_continuous_jobs_end_in_one_launch(size, frames):
             alone.render(frames)
             assert np.array_equal(j.read().view(np.int32), alone.read().view(np.int32)), k
             alone.release()
+
+
+@pytest.mark.parametrize("mode", [0, 1], ids=["pt", "bdpt"])
+def test_whole_path_launches_report_their_time(mode):
+    s = Y.gen_cornell()
+    with Y.Context(max_paths=1 << 18) as ctx:
+        j = ctx.job(ctx.scene(s), s.cam, 320, 200, Y.params_reference(mode, mis=1, bdpt_bounces=3), base_seed=2)
+        j.render(2)
+        st = j.stats()
+        assert st.iterations == 0 and st.ms_trace_ext == 0
+        assert 0 < st.ms_other <= st.ms_total
+        one = st.ms_other
+        j.render(2)
+        assert j.stats().ms_other > one

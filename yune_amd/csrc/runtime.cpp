@@ -172,6 +172,8 @@ struct yn_ctx {
     JobRec serve_rec;                 // statistics of scheduler rounds
     int64_t batch_paths = 0;          // paths per wavefront batch (0: the whole capacity)
     bool wave_only = false;           // no whole-path launches (yn_autotune)
+    std::chrono::steady_clock::time_point t_paths;   // when the batch's whole-path launch was made
+    bool paths_launched = false;      // since the last paths_time
     void* na_scratch = nullptr;       // device address of yn_trace_noalloc's static array on this device
     StreamState strm;                 // continuous serving
     uint32_t* done_ctr = nullptr;     // per piece: paths ended (device); from kMaxPieces on: paths parked
@@ -627,6 +629,15 @@ bool bdpt_paths_win(int64_t paths, int vertices, size_t node_bytes)
     return paths <= kPathsDirectBdptLong || vertices <= 8 || node_bytes <= ((size_t)32 << 10);
 }
 
+// Host time of a batch's whole-path launch, to be called once it is done:
+// device events around it would cost a small batch more than they tell.
+void paths_time(yn_ctx* c, yn_stats& st)
+{
+    if (!c->paths_launched) return;
+    c->paths_launched = false;
+    st.ms_other += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - c->t_paths).count();
+}
+
 // What whole-path launches need: width-4 trees, nothing counted or captured.
 bool paths_fit(const yn_ctx* c, const LoopCfg& L, bool capture)
 {
@@ -673,6 +684,8 @@ int enqueue_paths(yn_ctx* c, const LoopCfg& L, const IterArgs& A, bool primary, 
     pa.ovf_ref = c->ovf_ref;
     pa.ovf_t = c->ovf_t;
     pa.ovf_depth = c->ovf_depth;
+    c->t_paths = std::chrono::steady_clock::now();
+    c->paths_launched = true;
     launch_paths(pa, grid, c->stream);
     HIPCK(c, hipGetLastError());
     return 0;
@@ -693,6 +706,8 @@ int enqueue_paths_bdpt(yn_ctx* c, const LoopCfg& L, const IterArgs& A, const Gen
     pa.ovf_ref = c->ovf_ref;
     pa.ovf_t = c->ovf_t;
     pa.ovf_depth = c->ovf_depth;
+    c->t_paths = std::chrono::steady_clock::now();
+    c->paths_launched = true;
     launch_paths_bdpt(pa, grid, c->stream);
     HIPCK(c, hipGetLastError());
     return 0;
@@ -727,6 +742,7 @@ int finish_batch(yn_ctx* c, int64_t total, JobRec& stat_job)
 {
     HIPCK(c, hipGetLastError());
     HIPCK(c, hipStreamSynchronize(c->stream));
+    paths_time(c, stat_job.st);
     c->ctr_clear = c->h_ctr->q[6][0] == 0 && c->h_ctr->q[7][0] == 0;
     if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
     if (c->h_ctr->q[6][0]) return fail(c, YN_ERR_HIP, "paths did not end");
@@ -788,6 +804,7 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     hipStream_t s = c->stream;
     const bool clear = c->ctr_clear;
     c->ctr_clear = false;       // until finish_batch
+    c->paths_launched = false;
     const DevScene* scenes = c->d_scenes;
     auto q = [&](int k) { return &c->ctr->q[k][0]; };
     // counters (q(k) = q[k][0]): q[0],q[1] extension queue counts, q[2],q[3] shadow queue
@@ -1452,6 +1469,7 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
     if (c->h_ctr->q[7][0]) return fail(c, YN_ERR_INVALID, "traversal stack overflow");
     yn_stats& st = c->serve_rec.st;
     add_spans(spans, st);
+    paths_time(c, st);
     const unsigned long long now[6] = {c->h_ctr->rays_ext, c->h_ctr->rays_shadow, c->h_ctr->nodes_ext,
                                        c->h_ctr->tris_ext, c->h_ctr->nodes_shadow, c->h_ctr->tris_shadow};
     st.rays_ext += now[0] - S.last[0];
