@@ -102,3 +102,22 @@ def test_an_endless_job_is_served_beside_others(graph):
                 alone.set_counting(True)        # in the wavefront
                 alone.render(frames)
                 assert np.array_equal(got[k], bits(alone.read())), k
+
+
+def test_a_large_round_that_fails_leaves_its_images():
+    """More paths than one launch takes: the wavefront's last paths, several
+    scenes' among them, do not end."""
+    box, cornell = mirror_box(), Y.gen_cornell()
+    with Y.Context(max_paths=1 << 23, serve_mode=1) as c:
+        a, b = c.scene(box), c.scene(cornell)
+        fine = c.submit(b, cornell.cam, 1024, 1024, Y.params_reference(mis=1), 5, base_seed=5)
+        bad = c.submit(a, box.cam, 3, 2, Y.params_reference(**ENDLESS), 1, base_seed=5)
+        fine_was, bad_was = bits(fine.read()), bits(bad.read())
+        with pytest.raises(Y.YuneError):
+            c.serve(1)
+        assert c.serve_stats().iterations > 0
+        assert np.array_equal(bits(fine.read()), fine_was) and np.array_equal(bits(bad.read()), bad_was)
+        bad.release()
+        while c.serve(1):
+            pass
+        assert fine.read()[..., 3].min() == 5
