@@ -180,3 +180,38 @@ def test_results_over_the_device_rays(room, deep, shift):
         assert lib().yn_trace_noalloc(c._p, sid, C.c_void_p(d.data_ptr() + 32), n, *(C.c_void_p(a) for a in at)) == 0
         got = [d[8 + shift + k * n:8 + shift + (k + 1) * n].cpu().numpy() for k in range(3)]
         assert same(got, want)
+
+
+def test_reciprocal_rounds_as_division():
+    """x_rcp against IEEE division over every exponent and both signs.  A ray
+    straight at the plane of one right triangle of unit legs has the
+    determinant s (its direction's length along the plane's normal) and the
+    distance 1 / s exactly: both are reported bit for bit, and so is a hit that
+    1 / s = inf, or 0, rules out."""
+    s = Y.gen_cornell()
+    s.tris = np.zeros(1, dtype=Y.TRI_DTYPE)
+    s.tris["v1"], s.tris["v2"], s.tris["v3"] = (0, 0, 0, 1), (1, 0, 0, 1), (0, 1, 0, 1)
+    for k in ("vn1", "vn2", "vn3"):
+        s.tris[k] = (0, 0, 1, 0)
+    s.mats = s.mats[:1]
+    s.light = Y.light_quad((50, 50, 50), (0, -1, 0), (1, 1, 1), (0.1, 0, 0), (0, 0, 0.1))
+    rng = np.random.default_rng(7)
+    m = np.concatenate([rng.integers(0, 1 << 23, 2000), np.arange(24), (1 << 23) - 1 - np.arange(24),
+                        (1 << 22) + np.arange(-8, 8)]).astype(np.uint32)
+    x = ((np.arange(1, 255, dtype=np.uint32)[:, None] << 23) | m).reshape(-1).view(np.float32)
+    rays = np.zeros((2 * len(x), 8), np.float32)
+    rays[:, :2] = 0.25
+    rays[:, 3] = np.inf
+    rays[:len(x), 2], rays[:len(x), 6] = 1.0, -x        # det = x
+    rays[len(x):, 2], rays[len(x):, 6] = -1.0, x        # det = -x
+    with np.errstate(all="ignore"):
+        inv = np.float32(1) / x
+        u = (x * np.float32(0.25)) * inv                # both coordinates
+        want = np.where((u >= 0) & (u + u <= 1) & (inv > 0) & (inv < np.inf), inv, np.float32(np.inf))
+    with Y.Context(max_paths=1 << 21) as c:
+        tri, light, t = c.trace(c.scene(s, brute=True), rays)
+    assert (light == -1).all()
+    for part in (slice(0, len(x)), slice(len(x), None)):
+        assert np.array_equal(t[part].view(np.int32), want.view(np.int32))
+        assert np.array_equal(tri[part] == 0, np.isfinite(want))
+    assert np.isfinite(want).mean() > 0.99
