@@ -147,3 +147,16 @@ def test_whole_path_launches_report_their_time(mode):
         one = st.ms_other
         j.render(2)
         assert j.stats().ms_other > one
+
+
+@pytest.mark.parametrize("room,vertices,w,h,whole", [
+    ((7, 6, 3), 8, 1200, 1000, True), ((7, 24, 4), 5, 640, 400, True), ((7, 24, 4), 5, 1200, 1000, False),
+    ((7, 24, 4), 3, 1200, 1000, True), ((7, 24, 4), 3, 1500, 1500, False), ((7, 24, 4), 12, 1200, 1000, False)])
+def test_large_bidirectional_batches_of_large_trees_run_in_the_wavefront(room, vertices, w, h, whole):
+    """One launch of whole paths takes 1.2 times as long and more there."""
+    s = Y.gen_icosphere_room(*room)
+    params = Y.params_reference(1, mis=1, bdpt_bounces=vertices)
+    with Y.Context(max_paths=1 << 22) as ctx:
+        j = ctx.job(ctx.scene(s), s.cam, w, h, params, base_seed=9)
+        j.render(1)
+        assert (j.stats().iterations == 0) == whole

@@ -2,12 +2,12 @@
 launches that ordinary scenes do not reach.
 
 Batches of more than 4M paths run in the wavefront until 8M rays are left;
-bidirectional ones of more than 1M paths, long subpaths and a tree above 32 KB
-to the end.  The settings of its launches must not change an image, which is
+bidirectional ones of more than 1M paths and a tree above 4 MB to the end.  The settings of its launches must not change an image, which is
 compared with the counting wavefront's (other template instances) and, on a
 tile, with the oracle's.
 """
 import dataclasses
+import functools
 
 import numpy as np
 import pytest
@@ -18,8 +18,8 @@ from test_gpu_pt import comb_scene, identical, mre, ocam, oscene
 
 pytestmark = pytest.mark.gpu
 
-PT = dict(mode=0, W=1024, H=1024, F=9, kw=dict(mis=1, max_bounces=8, rr_threshold=2), max_paths=1 << 24)
-BD = dict(mode=1, W=1040, H=1024, F=1, kw=dict(mis=1, bdpt_bounces=9), max_paths=1 << 21)
+PT = dict(mode=0, W=1024, H=1024, F=9, kw=dict(mis=1, max_bounces=8, rr_threshold=2), max_paths=1 << 24, room=(9, 2))
+BD = dict(mode=1, W=1040, H=1024, F=1, kw=dict(mis=1, bdpt_bounces=5), max_paths=1 << 21, room=(24, 4))
 SETTINGS = [dict(), dict(trace_overlap=1, lds_stack=8), dict(graph=1), dict(graph=1, trace_overlap=1), dict(trace_xcd=1),
             dict(trace_xcd=3, trace_refill=1), dict(trace_refill=-1), dict(trace_refill=64, lds_stack=12),
             dict(shade_waves=2), dict(shade_waves=3, lds_stack=32)]
@@ -29,8 +29,9 @@ def bits(img):
     return img.view(np.int32)
 
 
-def scene():
-    return Y.gen_icosphere_room(3, 9, 2)
+@functools.lru_cache(maxsize=None)
+def scene(spheres=9, subdiv=2, seed=3):
+    return Y.gen_icosphere_room(seed, spheres, subdiv)
 
 
 def render(c, sid, s, k, seed=23, calls=1, counting=False):
@@ -48,12 +49,12 @@ def render(c, sid, s, k, seed=23, calls=1, counting=False):
 @pytest.fixture(scope="module")
 def counted():
     """The images of the counting wavefront, of one call and of two."""
-    s = scene()
     out = {}
     for name, k in (("pt", PT), ("bdpt", BD)):
+        s = scene(*k["room"])
         with Y.Context(max_paths=k["max_paths"]) as c:
             sid = c.scene(s)
-            assert c.scene_info(sid).node_bytes > 32 << 10
+            assert name == "pt" or c.scene_info(sid).node_bytes > 4 << 20
             out[name] = {n: render(c, sid, s, k, calls=n, counting=True) for n in (1, 2)}
     return out
 
@@ -61,7 +62,7 @@ def counted():
 @pytest.mark.parametrize("name,k", [("pt", PT), ("bdpt", BD)])
 @pytest.mark.parametrize("opts", SETTINGS, ids=lambda o: "-".join(f"{a}{b}" for a, b in o.items()) or "default")
 def test_settings_keep_large_images(name, k, opts, counted):
-    s = scene()
+    s = scene(*k["room"])
     with Y.Context(max_paths=k["max_paths"], **opts) as c:
         got = render(c, c.scene(s), s, k)
     assert got[1] == counted[name][1][1]
@@ -72,7 +73,7 @@ def test_settings_keep_large_images(name, k, opts, counted):
 def test_graph_follows_its_arguments(name, k, counted):
     """Two scenes and sizes in turn (captured again each time) and two calls
     of one job (replayed), with ray queries and small batches between them."""
-    s, other = scene(), Y.gen_icosphere_room(5, 4, 3)
+    s, other = scene(*k["room"]), scene(*((22, 4, 5) if k["mode"] else (4, 3, 5)))
     ko = dict(k, W=k["W"] + 24)
     rays = np.zeros((9000, 8), np.float32) + np.float32((0, 0, 4, 1e9, 0, 0, -1, 0))
     with Y.Context(max_paths=k["max_paths"]) as c:
@@ -92,7 +93,7 @@ def test_graph_follows_its_arguments(name, k, counted):
 
 @pytest.mark.parametrize("name,k", [("pt", PT), ("bdpt", BD)])
 def test_large_images_match_the_oracle_on_a_tile(name, k, counted):
-    s = scene()
+    s = scene(*k["room"])
     x0, y0, n = 500, 300, 40
     oimg, _, _, _ = oscene(s, s.bvh()).render(ocam(s.cam), k["W"], k["H"], O.params(k["mode"], **k["kw"]),
                                               O.mt19937(23, k["F"]), rect=(x0, y0, x0 + n, y0 + n), threads=8)

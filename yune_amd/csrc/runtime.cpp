@@ -615,18 +615,35 @@ constexpr int64_t kPathsDirect = (int64_t)1 << 22;
 constexpr int64_t kPathsTail = (int64_t)1 << 23;
 
 // Bidirectional batches run in k_paths_bdpt from the start or in the
-// wavefront to the end.  Wavefront against k_paths_bdpt:
-//                                1M paths          4.2M paths        8.4M paths
-//   Cornell box, 5 vertices      5.55 / 3.10 ms    14.0 / 11.0 ms    25.7 / 21.6 ms
-//   Cornell box, 20 vertices     12.7 / 6.66 ms    35.7 / 24.9 ms    64.8 / 48.5 ms
-//   15k triangles, 5 vertices    8.77 / 7.25 ms    28.7 / 27.4 ms    55.1 / 53.7 ms
-//   15k triangles, 20 vertices   37.6 / 34.1 ms    122 / 126 ms      231 / 246 ms
-// Long subpaths over trees larger than an L1 cache go to the wavefront above
-// 1M paths: their lanes wait for each other's walks.
-constexpr int64_t kPathsDirectBdptLong = (int64_t)1 << 20;
-bool bdpt_paths_win(int64_t paths, int vertices, size_t node_bytes)
+// wavefront to the end.  Time of the wavefront over that of k_paths_bdpt
+// (rooms of icospheres, NEE + MIS):
+//   nodes           vertices   0.9M    1.8M    2.7M    3.7M    5.5M    8.2M paths
+//   194 KB             5       1.68    1.38    1.26    1.20            1.10
+//   324 KB             3               1.52    1.38    1.30    1.22    1.16
+//                      8               1.26    1.17    1.14    1.09    1.06
+//   519 KB             3               1.36    1.24    1.18    1.11    1.06
+//                      8               1.14    1.06    1.03    0.99    0.95
+//   779 KB             3       1.57    1.25    1.13    1.07            0.98
+//                      8       1.22    1.06    0.98    0.94            0.87
+//   1.0 MB             3               1.19    1.08    1.03    0.98    0.95
+//                      8               1.00    0.94    0.90    0.87    0.84
+//   3.0 MB             3       1.46    1.16    1.06    1.00            0.91
+//                      8       1.16    0.99    0.92    0.88            0.82
+//   12 MB              3       1.23    1.01    0.91    0.87            0.80
+//                      8       1.02    0.86    0.79    0.77            0.72
+//   48 MB              3       1.19    0.96    0.87    0.84            0.76
+//                      8       0.98    0.83    0.75    0.72            0.68
+// and at 12 or 20 vertices as at 5 to 8 (48 MB, 0.9M and 2.7M: 1.03 and 0.78,
+// 1.10 and 0.80).  The Cornell box: 1.27 at least.  The lanes of a wave wait
+// for each other's walks, the longer the deeper the tree; the wavefront's
+// launches cost the same for every tree.
+int64_t bdpt_paths_limit(int vertices, size_t node_bytes)
 {
-    return paths <= kPathsDirectBdptLong || vertices <= 8 || node_bytes <= ((size_t)32 << 10);
+    if (node_bytes <= ((size_t)512 << 10)) return INT64_MAX;
+    const int64_t most = node_bytes <= ((size_t)3 << 19) ? (int64_t)3 << 20
+                         : node_bytes <= ((size_t)4 << 20) ? (int64_t)2 << 20
+                                                           : (int64_t)1 << 20;
+    return vertices <= 3 ? 2 * most : most;
 }
 
 // Host time of a batch's whole-path launch, to be called once it is done:
@@ -836,7 +853,7 @@ int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, cons
     if (bdpt) {
         int vertices = 0;
         for (const Region& r : regs) vertices = std::max(vertices, (int)c->jobs[r.job].p.bdpt_bounces);
-        direct = paths_ok && bdpt_paths_win(total, vertices, L.node_bytes);
+        direct = paths_ok && total <= bdpt_paths_limit(vertices, L.node_bytes);
     }
 
     GenArgs ga{};
