@@ -325,7 +325,7 @@ def context_kwargs(args, wl, trace_overlap=None):
                 trace_refill=args.trace_refill or wl.get("trace_refill", 0), bvh_build=args.bvh_build)
 
 
-STAT_KEYS = ("rays_ext", "rays_shadow", "samples", "ms_trace_ext", "ms_trace_shadow", "ms_shade",
+STAT_KEYS = ("rays_ext", "rays_shadow", "samples", "ms_trace_ext", "ms_trace_shadow", "ms_shade", "ms_other",
              "trace_launches_ext", "trace_launches_shadow", "iterations")
 
 
@@ -428,7 +428,7 @@ def rows_for(res, summary):
         return [kernel_row("k_paths_bdpt" if bdpt else "k_paths", "ray", d["rays_ext"] + d["rays_shadow"], res["steps"],
                            res["dt"] * 1e3, summary, "paths_bytes_per_ray", None, "paths")]
     # the rays include those that k_paths ran to their ends after the
-    # wavefront's last iteration (a few per cent)
+    # wavefront's last iteration (ms_whole_paths says how long that took)
     return [
         kernel_row("k_trace_rf closest hit", "ray", d["rays_ext"], d["trace_launches_ext"], d["ms_trace_ext"],
                    summary, "trace_ext_bytes_per_ray", alg_ext, "trace_ext"),
@@ -450,7 +450,7 @@ def config_summary(res):
         "rays": int(rays), "rays_per_sample": round(rays / max(d["samples"], 1), 3),
         "samples_per_s": round(d["samples"] / res["dt"], 1),
         "ms_trace_ext": round(d["ms_trace_ext"], 2), "ms_trace_shadow": round(d["ms_trace_shadow"], 2),
-        "ms_shade": round(d["ms_shade"], 2), "launch": res["launch"],
+        "ms_shade": round(d["ms_shade"], 2), "ms_whole_paths": round(d["ms_other"], 2), "launch": res["launch"],
     }
 
 

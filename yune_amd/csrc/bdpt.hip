@@ -648,11 +648,13 @@ constexpr int kBdptRefill = 56;
 // too, their results bits of a mask) and runs the steps between, until the
 // path ends; then it takes another work item.  The path's vertices and
 // pending-ray fields stay in memory, in the slot of the lane (not of the
-// path), so that they stay in cache; its scalars and colour in registers.
+// path), so that they take no more of it than there are lanes (214 MB for
+// 262,144 of 5 vertices: beyond the L2s, 433 bytes of HBM traffic a ray with
+// the spilled registers'); its scalars and colour in registers.
 //
 // Bound by vector issue with few lanes at work (84% busy, 16% of the lanes,
 // before the stages below).  The wavefront is bound by launches and the
-// longest ray of each: 640x360 of the Cornell box, 5 vertices, 2,018 -> 1,105
+// longest ray of each: 640x360 of the Cornell box, 5 vertices, 2,000 -> 831
 // us.  Lanes of a wave go through the stages of a path together and wait for
 // each other there: 4.2M paths of the Cornell box 15.7 -> 13.5 ms, of a
 // 15k-triangle room 45.9 -> 33.8.  128 registers with 88 spilled, at 4 waves

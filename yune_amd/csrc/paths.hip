@@ -15,8 +15,8 @@
 // of the lanes at work, since a wave's lanes wait for its longest walk and
 // run each other's shade steps; when a wave holds few paths, the chain of one
 // path's fetches.  97x61 pixels of the Cornell box without a bounce limit:
-// 2,070 -> 360 us; 1280x720 of a 245k-triangle room (NEE + MIS, depth 8):
-// 7,400 -> 2,120 us.  Variants measured at 4.2M paths of that room: 3 waves
+// 2,100 -> 285 us; 1280x720 of a 245k-triangle room (NEE + MIS, depth 8):
+// 7,590 -> 3,290 us.  Variants measured at 4.2M paths of that room: 3 waves
 // per SIMD (no spills) 7.9 ms, 4 waves (8 registers spilled) 6.8, 5 waves
 // (102) 6.5 but 7% slower at 262,144 paths; lanes that finish their walk
 // shaded while the others walk on (30 spilled at 3 waves) 8.0; all closest-

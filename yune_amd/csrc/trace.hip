@@ -302,11 +302,11 @@ __global__ __launch_bounds__(BLOCK, trace_waves<LST>()) void k_trace_rf(TraceArg
 // with no more rays than the grid has lanes each wave takes an equal share
 // of them and no counter is touched.
 // What bounds it: at a million rays the vector memory pipe, as k_trace_rf
-// (285 us for 1,000,003 rays over 123k triangles); at a few hundred the chain
-// of one ray's dependent fetches (48 us).  yn_trace of 1,000,003 host rays
-// 13.7 -> 2.24 ms (the rest is the bus: 32 MB in, 12 MB out), of 150,001
-// shadow rays 1.29 -> 0.43 ms, of 200 rays 104 -> 70 us; yn_trace_noalloc of
-// 200,003 rays 191 -> 111 us.
+// (260 us for 1,000,003 rays over 123k triangles); at a few hundred the chain
+// of one ray's dependent fetches (45 us).  yn_trace of 1,000,003 host rays
+// 13.3 -> 2.15 ms (the rest is the bus: 32 MB in, 12 MB out), of 150,001
+// shadow rays 1.27 -> 0.41 ms, of 200 rays 95 -> 50 us; yn_trace_noalloc of
+// 200,003 rays 189 -> 105 us.
 template <int W, int LST>
 __global__ __launch_bounds__(kRaysBlock, trace_waves<LST>()) void k_rays(RaysArgs a)
 {

@@ -46,8 +46,8 @@ struct DevJob {
 };
 
 // A queue of rays: rays[i] = {o.xyz, tmax}, {d.xyz, w}.  w: the path index
-// (bidirectional paths, caller rays), or the job-table entry of the path
-// whose state travels with the ray (unidirectional paths).
+// (bidirectional paths), or the job-table entry of the path whose state
+// travels with the ray (unidirectional paths).
 struct RayQueue {
     float4* o_t;
     float4* d_p;

@@ -7,8 +7,7 @@
 // keeps every intermediate normal takes the hardware's approximation and one
 // of Newton's steps in FMAs (Markstein, IBM J. R&D 34, 1990), any other the
 // division; a wave without such a lane skips it.  Compared with the division
-// for all 2^32 arguments on gfx950: equal for exponent fields 1..252 of
-// either sign, the range tested below.
+// for all 2^32 arguments on gfx950: equal.
 #pragma once
 
 #include <math.h>

@@ -12,8 +12,8 @@ namespace yune {
 // Streamed memory: the wavefront's records, rays and results are written by
 // one launch and read once, by the next, gigabytes later.  Marked so, they
 // leave the caches to the tree and the triangles: 32 frames of 1920x1080 of a
-// 1M-triangle room 163.9 -> 160.5 ms, twelve served jobs 34.8 -> 34.3 ms, 64
-// frames of 512x512 of the Cornell box 12.41 -> 12.28 ms (the records alone:
+// 1M-triangle room 159.7 -> 155.9 ms, twelve served jobs 34.8 -> 34.3 ms, 64
+// frames of 512x512 of the Cornell box 12.03 -> 11.94 ms (the records alone:
 // 0.3%, 0.7% and 0.8%).  k_paths reads the few records it is handed plainly
 // (1280x720 of a 245k-triangle room 0.5% slower with them streamed).
 typedef float nt_v4f __attribute__((ext_vector_type(4)));
@@ -126,7 +126,7 @@ struct ShadeArgs {
     int32_t lscene;             //   lmode 1: scene lscene's, 2: those of scene slots [0, n_lights)
     int32_t n_lights;
     int32_t ext_primary;        // 1: every extension-queue entry is a camera ray (a batch's
-                                //    first iteration), whose record holds only m0, m1, rd
+                                //    first iteration), whose record holds only M0
 };
 
 // Where a shade step finds a path's job and scene: the device tables, or, in
@@ -383,21 +383,6 @@ __device__ __forceinline__ void block_reserve(BlockReserveLds<NQ, BLOCK>& sm, in
         for (int v = 0; v < w; ++v) b += sm.tot[par][v][q];
         first[q] = b + x[q] - n[q];
     }
-}
-
-// Wave-aggregated append: one atomic per wave, lanes get consecutive slots
-// in lane order.  Every active lane of the wave must call it.
-__device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred)
-{
-    unsigned long long mask = __ballot(pred);
-    if (mask == 0) return 0;
-    const int lane = (int)__lane_id();
-    uint32_t prefix = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-    int leader = __ffsll((long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    return base + prefix;
 }
 #endif
 

@@ -368,10 +368,10 @@ __device__ bool traverse(const DevScene& S, RayState& r, Stack<LST, BLOCK>& st, 
 // loads of one address by every lane.  Those were a tenth of a walk's loads
 // through the vector memory pipe, which bounds the walks of large trees, and
 // a chain of a dozen trips to memory before each of them: 32 frames of
-// 1920x1080 of a 1M-triangle room 72.9 -> 68.8 ms, 1280x720 of a 245k-triangle
-// room 1,955 -> 1,868 us, 16.8M paths of the Cornell box (4 hoisted) 12.9 ->
-// 12.5 ms, 8 bidirectional frames of 1280x720 of it 13.35 -> 12.49 ms, twelve
-// served jobs of three scenes 35.3 -> 33.5 ms.
+// 1920x1080 of a 1M-triangle room 171.0 -> 159.1 ms, 1280x720 of a
+// 245k-triangle room 3,448 -> 3,235 us, 16.8M paths of the Cornell box (4
+// hoisted) 12.5 -> 12.1 ms, 8 bidirectional frames of 1280x720 of it 12.5 ->
+// 11.6 ms, twelve served jobs of three scenes 35.3 -> 33.5 ms.
 // Returns whether the walk ends here.
 template <int ANY, bool COUNT>
 __device__ __forceinline__ bool hoisted(yn_cv4f* hb, yn_cv4f* ht, int n, RayState& r, bool& got, Counts& c)
@@ -474,8 +474,8 @@ __device__ __forceinline__ bool descend(const V& LX, const V& HX, const V& LY, c
 // The first step of a walk over a tree of width 4 in a wave of one scene: the
 // root through the scalar unit (every new ray of the wave is there), seven
 // vector loads and one of their trips fewer.  8 bidirectional frames of
-// 1280x720 of the Cornell box 12.52 -> 12.24 ms, a 160x90 frame 300 -> 293 us,
-// 1280x720 of a 245k-triangle room 1,868 -> 1,852 us.
+// 1280x720 of the Cornell box 11.63 -> 11.35 ms, a 160x90 frame 440 -> 431 us;
+// rooms of 245k and 1M triangles within 0.4%.
 template <bool COUNT, bool EXACT, typename ST>
 __device__ __forceinline__ bool trav_root(const float4* __restrict__ nodes, uint32_t& node, RayState& r, ST& st,
                                           Counts& c)
