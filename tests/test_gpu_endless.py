@@ -1,4 +1,6 @@
 """Paths that reach the bounce limit of a launch (k_paths) before they end."""
+import time
+
 import numpy as np
 import pytest
 
@@ -121,3 +123,33 @@ def test_a_large_round_that_fails_leaves_its_images():
         while c.serve(1):
             pass
         assert fine.read()[..., 3].min() == 5
+
+
+def test_a_released_endless_job_is_dropped():
+    """Once the job is released, other calls need not wait for its paths."""
+    box, cornell = mirror_box(), Y.gen_cornell()
+    rays = np.zeros((100, 8), np.float32) + np.float32((0, 0, -3, 1e9, 0.1, 0.2, -1, 0))
+    p = Y.params_reference(mis=1)
+
+    def use(c, b):
+        j = c.job(b, cornell.cam, 16, 16, p, base_seed=3)
+        j.render(2)
+        return [bits(a) for a in (*c.trace(b, rays), j.read())]
+
+    with Y.Context(max_paths=1 << 12) as c:
+        want = use(c, c.scene(cornell))
+    with Y.Context(max_paths=1 << 12, serve_mode=0) as c:
+        a, b = c.scene(box), c.scene(cornell)
+        for _ in range(2):
+            endless = c.submit(a, box.cam, 3, 2, Y.params_reference(**ENDLESS), 2)
+            fine = c.submit(b, cornell.cam, 16, 16, p, 2, base_seed=3)
+            while c.serve(1) > 1:
+                pass
+            c.serve(2)
+            endless.release()
+            t0 = time.perf_counter()
+            got = use(c, b)
+            assert time.perf_counter() - t0 < 2
+            assert all(np.array_equal(x, y) for x, y in zip(got, want))
+            assert np.array_equal(bits(fine.read()), want[-1])
+        c.release_scene(a)

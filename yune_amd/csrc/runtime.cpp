@@ -1507,10 +1507,20 @@ int stream_group(yn_ctx* c, bool plan, bool* ran)
 
 // Runs the continuous loop without new pieces until every issued path has
 // ended and every piece is folded: other entry points use the same
-// wavefront buffers.
+// wavefront buffers.  Released jobs' paths alone are dropped, as their samples
+// are: they need not end.
 int stream_drain(yn_ctx* c)
 {
     for (const int64_t s0 = c->strm.steps; c->strm.active;) {
+        bool wanted = false;
+        for (const Piece& P : c->strm.pieces) wanted |= P.live && !P.orphan;
+        if (!wanted) {
+            for (Piece& P : c->strm.pieces) P = Piece();
+            c->strm.issue.clear();
+            c->strm.live = 0;
+            c->strm.active = false;
+            return 0;
+        }
         if (c->strm.steps - s0 > 1000000) return fail(c, YN_ERR_HIP, "continuous loop did not drain");
         // items not yet issued stay with their pieces; finish them too
         bool ran = false;
