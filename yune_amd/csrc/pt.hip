@@ -169,8 +169,10 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a)
 {
     int q = blockIdx.x * blockDim.x + threadIdx.x;
     // paths that were given up, or not taken, have no sample to fold (the
-    // flags stay up, since every block of the batch's folds reads them)
-    const bool failed = a.ctr && (a.ctr->q[6][0] | a.ctr->q[7][0]) != 0;
+    // flags stay up, since every block of the batch's folds reads them; they
+    // are asked for here and looked at only before the store, behind the
+    // samples' loads)
+    const uint32_t failed = a.ctr->q[6][0] | a.ctr->q[7][0];
     if (a.host && blockIdx.x == 0 && threadIdx.x < 64) {    // the batch's last launch: its counters
         const int i = (int)threadIdx.x;
         unsigned long long *from = &a.ctr->rays_ext, *to = &a.host->rays_ext;
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a)
         if (i < 12) a.host->q[i][0] = a.ctr->q[i][0];
         clear_counters(a.ctr);
     }
-    if (failed || q >= a.w * a.h) return;
+    if (q >= a.w * a.h) return;
     int x = a.x0 + q % a.w, y = a.y0 + q / a.w;
     size_t pix = (size_t)y * a.W + x;
     size_t npix = (size_t)a.W * a.H;
@@ -195,7 +197,7 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a)
         }
         acc = c;
     }
-    a.accum[pix] = st4(acc);
+    if (failed == 0) a.accum[pix] = st4(acc);
 }
 
 // The kernels' sin / cos / pow evaluated on the device (diagnostics).

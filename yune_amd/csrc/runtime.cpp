@@ -730,12 +730,10 @@ int enqueue_paths_bdpt(yn_ctx* c, const LoopCfg& L, const IterArgs& A, const Gen
     return 0;
 }
 
-// Folds samples into an image.  BATCH, LAST: those of a batch, unless it
-// failed; the batch's last one also hands the counters to the host and clears
-// them.  STREAM: those of whole pieces of the continuous loop.
-enum class Fold { STREAM, BATCH, LAST };
+// Folds samples into an image, unless their paths failed.  last: a batch's last
+// one also hands the counters to the host and clears them.
 void resolve(yn_ctx* c, const DevJob& d, int x0, int y0, int w, int h, int frames, bool reset_first, float4* accum,
-             const float4* prev, Fold kind)
+             const float4* prev, bool last)
 {
     ResolveArgs ra{};
     ra.W = d.W;
@@ -749,8 +747,8 @@ void resolve(yn_ctx* c, const DevJob& d, int x0, int y0, int w, int h, int frame
     ra.reset_first = reset_first ? 1 : 0;
     ra.accum = accum;
     ra.prev = prev ? prev : accum;
-    ra.ctr = kind == Fold::STREAM ? nullptr : c->ctr;
-    ra.host = kind == Fold::LAST ? c->h_ctr : nullptr;
+    ra.ctr = c->ctr;
+    ra.host = last ? c->h_ctr : nullptr;
     launch_resolve(ra, c->stream);
 }
 
@@ -798,7 +796,7 @@ int upload_jobs(yn_ctx* c, const std::vector<Region>& regs)
 // of each region's job (the sample buffer is shared: job slots are laid out
 // by the caller so regions do not overlap).  The last launches may still run
 // when it returns: the caller folds the samples (resolve, the last time with
-// Fold::LAST) and then calls finish_batch with *paths.
+// `last`) and then calls finish_batch with *paths.
 int run_batch(yn_ctx* c, const std::vector<Region>& regs, JobRec& stat_job, const DevCapture& cap, int64_t* paths)
 {
     std::vector<GenSeg> segs;
@@ -1006,7 +1004,7 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
             int64_t paths = 0;
             int r = run_batch(c, regs, J, cp, &paths);
             if (r) return r;
-            resolve(c, J.dev, x0, y0, w, h, nslots, reset_first && f == 0, accum, f == 0 ? prev : nullptr, Fold::LAST);
+            resolve(c, J.dev, x0, y0, w, h, nslots, reset_first && f == 0, accum, f == 0 ? prev : nullptr, true);
             if (int e = finish_batch(c, paths, J)) return e;
         } else {
             // image larger than the path capacity: row bands, one frame at a time
@@ -1025,7 +1023,7 @@ int render_rect(yn_ctx* c, int jid, float4* accum, int x0, int y0, int w, int h,
                 int64_t paths = 0;
                 int r = run_batch(c, regs, J, cp, &paths);
                 if (r) return r;
-                resolve(c, J.dev, x0, yb, w, hh, 1, reset_first && f == 0, accum, f == 0 ? prev : nullptr, Fold::LAST);
+                resolve(c, J.dev, x0, yb, w, hh, 1, reset_first && f == 0, accum, f == 0 ? prev : nullptr, true);
                 if (int e = finish_batch(c, paths, J)) return e;
             }
         }
@@ -1149,8 +1147,7 @@ int serve_round(yn_ctx* c, int* frames_out)
     if (int r = run_batch(c, regs, c->serve_rec, DevCapture{}, &paths)) return r;
     for (const Plan& pl : plan) {
         JobRec& J = c->jobs[pl.jid];
-        resolve(c, J.dev, 0, 0, J.W, J.H, pl.k, pl.reset, J.accum, nullptr,
-                &pl == &plan.back() ? Fold::LAST : Fold::BATCH);
+        resolve(c, J.dev, 0, 0, J.W, J.H, pl.k, pl.reset, J.accum, nullptr, &pl == &plan.back());
     }
     if (int r = finish_batch(c, paths, c->serve_rec)) return r;
     double now = ms_since(c);
@@ -1372,7 +1369,7 @@ int stream_fold(yn_ctx* c)
                 if ((int64_t)J.frame != P.f0) continue;      // an earlier piece of the job is not folded yet
                 DevJob d = make_devjob(J);
                 d.samples = c->samples + P.soff;
-                resolve(c, d, 0, 0, J.W, J.H, P.k, P.f0 == 0, J.accum, nullptr, Fold::STREAM);
+                resolve(c, d, 0, 0, J.W, J.H, P.k, P.f0 == 0, J.accum, nullptr, false);
                 J.frame += (uint64_t)P.k;
                 J.st.frames += (uint64_t)P.k;
                 J.st.samples += (uint64_t)P.items;

@@ -294,7 +294,7 @@ struct ResolveArgs {
     int32_t reset_first;        // first frame of the batch overwrites (kernel arg 9)
     float4* accum;              // the job's RGBA32F image, .w = count
     const float4* prev;         // the image before the first frame (kernel arg 1; accum itself for a job)
-    DevCounters* ctr;           // not null: the batch's counters; with an error flag up the image stays as it is
+    DevCounters* ctr;           // with an error flag up there the image stays as it is
     DevCounters* host;          // not null: the counters go there (pinned) and are cleared, but for the flags
 };
 
